@@ -1,0 +1,785 @@
+"""What a user of this framework has it do, as cases that can be timed.
+
+Three kinds, each through the package's public entry points:
+
+* ``segment``: a stretch of a simulation between two outputs. The state in the
+  caller's device buffers (THOR's layout) goes in through
+  ``thor_dyn_set_state``, ``Dyn.run`` takes ``steps`` large steps (ProfX with
+  the forcing, then the dynamics) and ``thor_dyn_get_state`` hands the new
+  state back: the main loop of a run, an ensemble member, a restart.
+* ``step``: ``Dyn.step``, the dynamics step on the caller's own arrays with the
+  caller's forcing (a THOR build that keeps its own ProfX).
+* ``train``: one epoch of the radiative-heating network on sampled columns.
+
+Sizes are those of the Held-Suarez and hot-Jupiter runs of the bench and the
+tests (icosahedral levels 4 to 7, 12 to 63 layers), odd layer counts among
+them, in both precision forms. ``exact`` computes the same results in plain
+torch in 64 bits from the grid's operators.
+"""
+from __future__ import annotations
+
+import ctypes as C
+import functools
+import math
+import os
+
+import numpy as np
+import torch
+
+from thor_amd import capi
+from thor_amd import surrogate as sg
+
+DEVICE = "cuda"
+CACHE = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), ".thor_cache")
+STATE = ("Mh", "Wh", "W", "Rho", "pressure")
+EARTH = dict(A=6.371e6, Omega=7.292e-5, Gravit=9.8, P_Ref=1e5, Rd=287.0, Cp=1005.0, Tmean=300.0, top=36000.0,
+             Diffc=0.0048, DivDampc=0.0048)
+HOT = dict(A=1e8, Omega=2.06e-5, Gravit=9.42, P_Ref=1e7, Rd=3779.0, Cp=13226.0, Tmean=1600.0, top=sg.HJ_TOP,
+           Diffc=0.02, DivDampc=0.03)
+FORCING = {"none": capi.FORCING_NONE, "held_suarez": capi.FORCING_HELD_SUAREZ, "newtonian": capi.FORCING_NEWTONIAN,
+           "double_gray": capi.FORCING_DOUBLE_GRAY, "surrogate": capi.FORCING_RT_SURROGATE}
+# Day-night relaxation of the hot-Jupiter runs: 1600 K +- 600 K, time scales 1e4 to 1e7 s.
+NEWTONIAN = dict(T_mean=1600.0, dT=600.0, lon_sub=0.0, p_top=1e2, p_bottom=1e7, p_contrast=1e6, tau_top=1e4,
+                 tau_bottom=1e7)
+JUDGE = 10  # the surrogate's exact judge runs every tenth step
+HIDDEN = 256
+
+
+def _dynamics(kind, planet, glevel, nv, precision, forcing, steps, ns, dt, deep=1, nonhydro=1, ghv=0, order=4,
+              sponge=0):
+    return dict(kind=kind, planet=planet, glevel=glevel, nv=nv, precision=precision, forcing=forcing, steps=steps,
+                ns=ns, dt=dt, deep=deep, nonhydro=nonhydro, ghv=ghv, order=order, sponge=sponge)
+
+
+def listed():
+    D = _dynamics
+    return [
+        # the smallest call: one dynamics step on a caller's arrays, an odd number of layers, launch-bound
+        dict(D("step", "earth", 4, 23, "fp64", "given", 1, 6, 1000.0), name="step_g4_l23_fp64"),
+        # the 100-step drift check's workload (Held-Suarez, 2 562 columns)
+        dict(D("segment", "earth", 4, 32, "fp64", "held_suarez", 2, 6, 1000.0), name="hs_g4_l32_fp64"),
+        # a low-resolution spin-up in the mixed form, two steps between outputs
+        dict(D("segment", "earth", 4, 20, "mixed", "held_suarez", 2, 6, 1000.0), name="hs_g4_l20_mixed"),
+        # hot-Jupiter Newtonian relaxation, both forms
+        dict(D("segment", "hot", 5, 40, "fp64", "newtonian", 2, 6, 300.0), name="newtonian_g5_l40_fp64"),
+        dict(D("segment", "hot", 5, 40, "mixed", "newtonian", 2, 6, 300.0), name="newtonian_g5_l40_mixed"),
+        # the drop-in step in the mixed form: shallow, hydrostatic, an odd number of layers
+        dict(D("step", "earth", 5, 33, "mixed", "given", 1, 6, 600.0, deep=0, nonhydro=0), name="step_g5_l33_mixed"),
+        # spin-up that trains the surrogate: exact radiation and the sponge
+        dict(D("segment", "hot", 5, 40, "mixed", "double_gray", 2, 6, 300.0, sponge=1),
+             name="double_gray_g5_l40_mixed"),
+        # the learned radiation in the step, its judge once in ten steps
+        dict(D("segment", "hot", 5, 40, "mixed", "surrogate", JUDGE, 6, 300.0, sponge=1),
+             name="surrogate_g5_l40_mixed"),
+        # the headline workload in both forms
+        dict(D("segment", "earth", 6, 48, "fp64", "held_suarez", 2, 8, 300.0), name="hs_g6_l48_fp64"),
+        dict(D("segment", "earth", 6, 48, "mixed", "held_suarez", 2, 8, 300.0), name="hs_g6_l48_mixed"),
+        # the largest: 163 842 columns with the learned radiation
+        dict(D("segment", "hot", 7, 48, "mixed", "surrogate", JUDGE, 6, 120.0, sponge=1),
+             name="surrogate_g7_l48_mixed"),
+        # one epoch of the surrogate's training on sampled columns
+        dict(kind="train", nv=40, rows=16384, batch=512, name="train_l40_b512"),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    if rng.random() < 0.12:
+        return dict(kind="train", nv=_log_int(rng, 16, 63), rows=_log_int(rng, 3000, 40000),
+                    batch=rng.choice([128, 200, 256, 512, 1000]))
+    glevel = rng.choice([4, 4, 5, 5, 6])
+    nv = _log_int(rng, 14, 63)
+    precision = rng.choice(["fp64", "mixed"])
+    ns = rng.choice([4, 6, 8, 10])
+    deep, nonhydro = (1, 1) if rng.random() < 0.8 else (0, 0)
+    order = 4 if rng.random() < 0.85 else 6
+    ghv = int(rng.random() < 0.15)
+    if rng.random() < 0.5:
+        kind = "step" if rng.random() < 0.4 else "segment"
+        return _dynamics(kind, "earth", glevel, nv, precision, "given" if kind == "step" else "held_suarez",
+                         1 if kind == "step" else rng.randint(1, 4), ns, {4: 900.0, 5: 500.0, 6: 250.0}[glevel],
+                         deep, nonhydro, ghv, order)
+    forcing = rng.choice(["newtonian", "double_gray", "surrogate"])
+    return _dynamics("segment", "hot", glevel, nv, precision, forcing, JUDGE if forcing == "surrogate"
+                     else rng.randint(1, 4), ns, {4: 400.0, 5: 300.0, 6: 200.0}[glevel], deep, 1 if deep else 0, 0,
+                     order, int(rng.random() < 0.5))
+
+
+# ------------------------------------------------------------- preparation
+
+@functools.lru_cache(maxsize=4)
+def _grid(glevel, nv, radius, top):
+    os.makedirs(CACHE, exist_ok=True)
+    return capi.Grid(glevel, nv, radius, top, spring=True, beta=1.15, cache_dir=CACHE)
+
+
+def _planet(case):
+    return EARTH if case["planet"] == "earth" else HOT
+
+
+def _case_grid(case):
+    q = _planet(case)
+    return _grid(case["glevel"], case["nv"], q["A"], q["top"])
+
+
+def _t(a):
+    return torch.as_tensor(np.array(a), device=DEVICE)
+
+
+@functools.lru_cache(maxsize=2)
+def _core(key):
+    """The dynamical core of a configuration, as a program keeps it for its whole run."""
+    case = dict(key)
+    q = _planet(case)
+    g = _case_grid(case)
+    p = capi.default_params(glevel=case["glevel"], timestep=case["dt"], n_substeps=case["ns"],
+                            precision=capi.PRECISION_MIXED if case["precision"] == "mixed" else capi.PRECISION_FP64,
+                            DeepModel=case["deep"], NonHydro=case["nonhydro"], GravHeightVar=case["ghv"],
+                            HyDiffOrder=case["order"], **{k: v for k, v in q.items() if k != "top"})
+    d = capi.Dyn(g, p)
+    if case["forcing"] == "newtonian":
+        d.set_newtonian(capi.NewtonianParams(**NEWTONIAN))
+    if case["forcing"] in ("double_gray", "surrogate"):
+        d.set_rt(sg.double_gray())
+    if case["forcing"] == "surrogate":
+        net = capi.MLP(2 * case["nv"] + 1, HIDDEN, case["nv"], seed=5)
+        net.set_params(_network(case["nv"]))
+        d.set_rt_surrogate(net, _norm(case), judge_every=JUDGE)
+    if case["sponge"]:
+        d.set_sponge(sg.hot_jupiter_sponge())
+    return d
+
+
+def _key(case):
+    return tuple(sorted((k, v) for k, v in case.items() if k not in ("name", "kind", "steps")))
+
+
+def _network(nv, seed=5):
+    """Parameters of a heating network (thor_mlp.h's flat layout) as random as a new one's."""
+    r = np.random.RandomState(seed + nv)
+    sizes, out = ((2 * nv + 1, HIDDEN), (HIDDEN, HIDDEN), (HIDDEN, nv)), []
+    for i, (a, b) in enumerate(sizes):
+        lim = math.sqrt(6.0 / a) * (1.0 if i < 2 else 0.6)
+        out += [r.uniform(-lim, lim, a * b), r.uniform(-0.05, 0.05, b)]
+    return np.concatenate(out).astype(np.float32)
+
+
+def _rest_column(case):
+    """Altitudes and the isothermal rest column's pressure at the layer centres."""
+    q = _planet(case)
+    dz = q["top"] / case["nv"]
+    alt = (np.arange(case["nv"]) + 0.5) * dz
+    return alt, q["P_Ref"] * np.exp(-q["Gravit"] * alt / (q["Rd"] * q["Tmean"]))
+
+
+def _norm(case):
+    """Input and output scales of the network for the columns of _state: means
+    and spreads of T, ln p and cos z, and heating of the order of 1e-4 K/s. A few
+    columns in a thousand leave the envelope and take the exact radiation."""
+    q, nv = _planet(case), case["nv"]
+    _, p = _rest_column(case)
+    heat = 1e-4 * p / (q["Rd"] * q["Tmean"]) * (q["Cp"] - q["Rd"])
+    f = lambda *a: np.concatenate(a).astype(np.float32)  # noqa: E731
+    return {"in_mean": f(np.full(nv, q["Tmean"]), np.log(p), [0.25]), "in_std": f(np.full(nv, 20.0), np.full(nv, 0.02),
+                                                                                  [0.32]),
+            "in_lo": f(np.full(nv, -4.5), np.full(nv, -8.0), [-2.0]),
+            "in_hi": f(np.full(nv, 4.5), np.full(nv, 8.0), [3.0]),
+            "out_mean": f(np.zeros(nv)), "out_std": f(heat)}
+
+
+def _state(case, seed):
+    """A hydrostatic state with zonal jets, large-scale waves and grid-scale
+    noise, in THOR's layout on the GPU."""
+    q, g, nv = _planet(case), _case_grid(case), case["nv"]
+    gen = torch.Generator(device=DEVICE).manual_seed(seed)
+    rnd = lambda *s: torch.rand(*s, generator=gen, device=DEVICE, dtype=torch.float64) * 2 - 1  # noqa: E731
+    P = g.P
+    lon, lat = _t(g.lonlat).reshape(P, 2).T
+    alt, alth = _t(g.Altitude), _t(g.Altitudeh)
+    hot = case["planet"] == "hot"
+    U, amp, noise = (200.0, 20.0, 0.1) if hot else (20.0, 2.0, 1e-3)
+    zeta = (alt / q["top"])[None]
+    z = torch.stack([torch.cos(lat) ** 2 * torch.cos(m * lon + math.pi * float(rnd(1))) for m in (1, 2, 3)], 1)
+    shape = torch.stack([torch.sin((k + 1) * math.pi * alt / q["top"]) for k in range(3)], 0)
+    T = q["Tmean"] + amp * z @ rnd(3, 3) @ shape + noise * rnd(P, nv)
+    Rd, G = q["Rd"], q["Gravit"]
+    p = [torch.full((P,), q["P_Ref"], dtype=torch.float64, device=DEVICE) * torch.exp(-G * alt[0] / (Rd * T[:, 0]))]
+    for k in range(nv - 1):  # discrete hydrostatic balance between layer centres
+        d = alt[k + 1] - alt[k]
+        a, b = (alt[k + 1] - alth[k + 1]) / d, (alth[k + 1] - alt[k]) / d
+        p.append(p[-1] * (1 - G * d * a / (Rd * T[:, k])) / (1 + G * d * b / (Rd * T[:, k + 1])))
+    p = torch.stack(p, 1)
+    rho = p / (Rd * T)
+    u = U * torch.cos(lat)[:, None] * (0.5 + zeta) * (1 + 0.2 * rnd(1)) + 0.2 * U * z @ rnd(3, 3) @ shape
+    u = u + 0.1 * rnd(P, nv)
+    v = 0.2 * U * torch.cos(lat)[:, None] * (z @ rnd(3, 3) @ shape) + 0.1 * rnd(P, nv)
+    e_lon = torch.stack([-torch.sin(lon), torch.cos(lon), torch.zeros_like(lon)], 1)
+    e_lat = torch.stack([-torch.sin(lat) * torch.cos(lon), -torch.sin(lat) * torch.sin(lon), torch.cos(lat)], 1)
+    Mh = rho[..., None] * (u[..., None] * e_lon[:, None] + v[..., None] * e_lat[:, None])
+    Wh = torch.zeros(P, nv + 1, dtype=torch.float64, device=DEVICE)
+    Wh[:, 1:-1] = (0.5 * (rho[:, 1:] + rho[:, :-1])) * 0.01 * (1 + rnd(P, nv - 1)) * torch.sin(
+        math.pi * alth[1:-1] / q["top"])
+    st = {"Mh": Mh, "Wh": Wh, "W": _center(Wh, alt, alth), "Rho": rho, "pressure": p}
+    return {k: st[k].contiguous() for k in STATE}
+
+
+def _given_forcing(case, st):
+    """Heating and drag as a caller's own physics leaves them: 1 K per day of
+    heating with the day side, a five-day drag."""
+    q, g = _planet(case), _case_grid(case)
+    lon, lat = _t(g.lonlat).reshape(g.P, 2).T
+    heat = st["Rho"] * (q["Cp"] - q["Rd"]) / 86400.0 * (torch.cos(lat) * torch.cos(lon))[:, None]
+    return {"Qheat": heat.contiguous(), "dMh": (-st["Mh"] / (5 * 86400.0)).contiguous(),
+            "dWh": torch.zeros_like(st["Wh"])}
+
+
+def _columns(case, seed):
+    """Normalised training columns: smooth temperature profiles and the heating
+    that a fixed smooth function of them gives, plus noise."""
+    r = np.random.RandomState(seed % (2 ** 31))
+    n, nv = case["rows"], case["nv"]
+    s = np.linspace(0, 1, nv)
+    basis = np.stack([np.cos(k * np.pi * s) for k in range(6)])
+    a = r.standard_normal((n, 6)) / (1 + np.arange(6))
+    mu = np.maximum(r.uniform(-1, 1, n), 0)
+    lnp = 0.1 * r.standard_normal((n, 2)) @ basis[:2] + 0.02 * r.standard_normal((n, nv))
+    X = np.concatenate([a @ basis, lnp, mu[:, None]], 1).astype(np.float32)
+    Y = np.tanh(np.roll(a, 1, 1) @ basis) * (0.3 + mu[:, None]) + 0.05 * r.standard_normal((n, nv))
+    return X, Y.astype(np.float32)
+
+
+LR = 1e-3  # the learning rate of the surrogate's first epochs
+
+
+def prepare(case, seed):
+    if case["kind"] == "train":
+        X, Y = _columns(case, seed)
+        net = capi.MLP(2 * case["nv"] + 1, HIDDEN, case["nv"], seed=1)
+        net.set_params(_network(case["nv"], seed % 1000))
+        net.set_data(X, Y)
+        return {"case": case, "net": net, "seed": seed}
+    st = _state(case, seed)
+    s = {"case": case, "core": _core(_key(case)), "start": st, "new": {k: torch.empty_like(v) for k, v in st.items()}}
+    if case["kind"] == "step":
+        s["forcing"] = _given_forcing(case, st)
+        s["forcing_at"] = {k: v.data_ptr() for k, v in s["forcing"].items()}
+        s["new_at"] = {k: v.data_ptr() for k, v in s["new"].items()}
+    torch.cuda.synchronize()  # the core's stream does not wait for torch's
+    return s
+
+
+def _on_device(st):
+    cast = lambda t: C.cast(C.c_void_p(t.data_ptr()), C.POINTER(C.c_double))  # noqa: E731
+    return capi.State(1, *(cast(st[k]) for k in STATE))
+
+
+def run(state):
+    case = state["case"]
+    if case["kind"] == "train":
+        net = state["net"]
+        loss = net.train_epoch(case["batch"], LR, state["seed"])
+        return {"loss": loss, "params": net.params()}
+    core = state["core"]
+    if case["kind"] == "step":
+        for k in STATE:  # the step overwrites the caller's arrays
+            state["new"][k].copy_(state["start"][k])
+        core.step(state["new_at"], state["forcing_at"], stream=torch.cuda.current_stream().cuda_stream)
+        return state["new"]
+    core._chk(core.L.thor_dyn_set_state(core._h, C.byref(_on_device(state["start"]))))
+    core.run(case["steps"], FORCING[case["forcing"]])
+    core._chk(core.L.thor_dyn_get_state(core._h, C.byref(_on_device(state["new"]))))
+    return state["new"]
+
+
+def work(case):
+    if case["kind"] == "train":
+        nin, nh, nout, n = 2 * case["nv"] + 1, HIDDEN, case["nv"], case["rows"]
+        macs = nin * nh + nh * nh + nh * nout
+        return {"bytes": 4.0 * (n * (nin + nout) + 2 * macs), "flops": 2.0 * n * (3 * macs - nin * nh)}
+    P = 10 * 4 ** case["glevel"] + 2
+    N, substeps = P * case["nv"], 1 + case["ns"] // 2 + case["ns"]
+    # state in and out (and the forcing arrays), the grid's operators once
+    values = N * (14 + (5 if case["kind"] == "step" else 0)) + P * 120
+    # operations per cell: three stages of the slow part, the substeps, the forcing
+    flops = N * case["steps"] * (3 * 950 + substeps * 520 + 60)
+    if case["forcing"] == "surrogate":
+        flops += 2.0 * P * case["steps"] * ((2 * case["nv"] + 1) * HIDDEN + HIDDEN ** 2 + HIDDEN * case["nv"])
+    return {"bytes": 8.0 * values, "flops": float(flops)}
+
+
+def tolerance(case):
+    """About four times the largest distance from exact() seen over the ranges
+    (Wh and W, small differences of large terms, are the farthest off)."""
+    if case["kind"] == "train":  # Adam turns a gradient near zero into a whole step
+        return {"rel": 4e-3, "max": 0.5}
+    if case["forcing"] == "surrogate":  # a BF16 network's heating: 3e-3
+        return {"rel": 1.2e-2}
+    if case["precision"] == "mixed":  # 32-bit momentum and tendencies: 1.3e-4
+        return {"rel": 5e-4}
+    return {"rel": 1e-10}  # 64-bit sums in another order: 1.3e-11
+
+
+# ----------------------------------------------------------------- 64 bits
+
+def _center(Wh, alt, alth):
+    """Interface values at the layer centres."""
+    t = (alt - alth[1:]) / (alth[:-1] - alth[1:])
+    b = (alt - alth[:-1]) / (alth[1:] - alth[:-1])
+    return Wh[:, :-1] * t + Wh[:, 1:] * b
+
+
+class _Exact:
+    """The dynamical core and its forcings in plain torch, 64 bits."""
+
+    def __init__(self, case):
+        self.case, q, g = case, _planet(case), _case_grid(case)
+        self.q, self.nv, self.P = q, case["nv"], g.P
+        P = g.P
+        self.deep, self.nonhydro, self.ghv = case["deep"], case["nonhydro"], case["ghv"]
+        f = lambda n, *s: _t(getattr(g, n)).reshape(P, *s)  # noqa: E731
+        self.div, self.grad, self.fr = f("div", 7, 3), f("grad", 7, 3), f("func_r", 3)
+        self.alt, self.alth = _t(g.Altitude), _t(g.Altitudeh)
+        self.lon, self.lat = f("lonlat", 2).T
+        local = f("point_local", 6).long()
+        five = torch.zeros(P, dtype=torch.bool, device=DEVICE)
+        five[[int(i) for i in g.pent_ind if 0 <= i < P] + [P - 2, P - 1]] = True
+        self.pole = torch.zeros(P, dtype=torch.bool, device=DEVICE)
+        self.pole[-2:] = True
+        local[five, 5] = local[five, 4]
+        self.ring = torch.cat([torch.arange(P, device=DEVICE)[:, None], local], 1)
+        self._operators(f("areas", 6, 3), f("areasTr", 6), f("nvecti", 6, 3), f("nvecte", 6, 3), f("nvecoa", 6, 3),
+                        five)
+        A = q["A"]
+        one = torch.ones_like(self.alt)
+        self.rs = A / (self.alt + A) if self.deep else one
+        if self.deep:
+            self.r2m, self.r2h = (self.alt + A) ** 2, (self.alth + A) ** 2
+            self.dr = ((self.alth[1:] + A) ** 3 - (self.alth[:-1] + A) ** 3) / 3
+        else:
+            self.r2m, self.r2h = one, torch.ones_like(self.alth)
+            self.dr = self.alth[1:] - self.alth[:-1]
+        self.dz = self.alth[1:] - self.alth[:-1]
+        dbar = math.sqrt(2 * math.pi / 5) * A / 2 ** case["glevel"]
+        self.kdh = q["Diffc"] * dbar ** case["order"] / case["dt"]
+        self.kdz = q["DivDampc"] * dbar ** 4 / case["dt"]
+        self.gz = q["Gravit"] * (A / (A + self.alt)) ** 2 if self.ghv else q["Gravit"] * one
+        d = self.alt[1:] - self.alt[:-1]
+        self.up, self.lo = (self.alth[1:-1] - self.alt[:-1]) / d, (self.alt[1:] - self.alth[1:-1]) / d
+
+    def _operators(self, ar, aT, ti, te, oa, five):
+        """Laplacian and grad-div of the triangles around each point as
+        coefficients on the point and its ring."""
+        P = self.P
+        nf = torch.where(five, 5, 6)
+        E = torch.eye(7, dtype=torch.float64, device=DEVICE)
+        G, D, U = [], [], []
+        self_ = E[0].expand(P, 7)
+        nxts = [torch.where(torch.tensor(t + 1, device=DEVICE) >= nf, 0, t + 1) for t in range(6)]
+        rows = torch.arange(P, device=DEVICE)
+        for t in range(6):
+            nx = nxts[t]
+            a, b = E[1 + t].expand(P, 7), E[1 + nx]
+            at = torch.where(t < nf, aT[:, t], 1.0)[:, None]  # five triangles: the sixth is left out below
+            w2 = torch.where(self.pole, ar[:, t, 1], ar[:, t, 2])
+            star = (ar[:, t, :1] * self_ + ar[:, t, 1:2] * a + ar[:, t, 2:3] * b) / at
+            l1, l2, l3 = 0.5 * (a + self_) - star, 0.5 * (a + b) - star, 0.5 * (self_ + b) - star
+            tn = ti[rows, nx]
+            vec = lambda s, n: s[:, :, None] * n[:, None, :]  # noqa: E731
+            G.append((-vec(l1, ti[:, t]) + vec(l2, te[:, t]) + vec(l3, tn)) / at[..., None])
+            D.append((-vec(self_ + a, ti[:, t]) + vec(a + b, te[:, t]) + vec(self_ + b, tn)) * (0.5 / at[..., None]))
+            U.append((ar[:, t, :1] * self_ + ar[:, t, 1:2] * a + w2[:, None] * b) / at)
+        G, D, U = torch.stack(G, 1), torch.stack(D, 1), torch.stack(U, 1)
+        lap = torch.zeros(P, 7, dtype=torch.float64, device=DEVICE)
+        dd = torch.zeros(P, 3, 7, 3, dtype=torch.float64, device=DEVICE)
+        dw = torch.zeros(P, 3, 7, dtype=torch.float64, device=DEVICE)
+        for j in range(6):
+            on = (j < nf)[:, None]
+            nx = nxts[j]
+            n = torch.where(on, oa[:, j], 0.0) * 0.5
+            lap += ((G[:, j] + G[rows, nx]) * n[:, None, :]).sum(-1)
+            dd += n[:, :, None, None] * (D[:, j] + D[rows, nx])[:, None]
+            dw += n[:, :, None] * (U[:, j] + U[rows, nx])[:, None]
+        self.lap_w, self.dd_w, self.dw_w = lap, dd, dw
+
+    def _flux(self, M, *scalars):
+        """rscale times the divergence of M, and of M times each scalar."""
+        out = [torch.zeros_like(M[..., 0]) for _ in range(1 + len(scalars))]
+        for s in range(7):
+            i = self.ring[:, s]
+            d = (M[i] * self.div[:, s][:, None]).sum(-1)
+            out[0] += d
+            for k, f in enumerate(scalars):
+                out[1 + k] += d * f[i]
+        return [o * self.rs for o in out]
+
+    def _gradient(self, a):
+        out = torch.zeros(*a.shape, 3, dtype=torch.float64, device=DEVICE)
+        for s in range(7):
+            out += a[self.ring[:, s]][..., None] * self.grad[:, s][:, None]
+        return out * self.rs[:, None]
+
+    def _laplacian(self, a):
+        """of fields [P, nv, n]; the differences to the centre value"""
+        out = torch.zeros_like(a)
+        for s in range(1, 7):
+            out += self.lap_w[:, s, None, None] * (a[self.ring[:, s]] - a)
+        return out * (self.rs ** 2)[:, None]
+
+    def _tangent(self, v):
+        return v - (v * self.fr[:, None]).sum(-1, keepdim=True) * self.fr[:, None]
+
+    def _divdamp(self, M, Wh):
+        dw = (Wh[:, :-1] - Wh[:, 1:]) * (-1.0 / self.dz) * self.rs
+        one = torch.zeros_like(M)
+        for s in range(7):
+            i = self.ring[:, s]
+            Mi = M[i] * (self.rs ** 2)[:, None]
+            for c in range(3):
+                one[..., c] += (Mi * self.dd_w[:, c, s][:, None]).sum(-1) + self.dw_w[:, c, s, None] * dw[i]
+        two = torch.zeros_like(M)
+        for s in range(7):
+            Mi = one[self.ring[:, s]] * (self.rs ** 2)[:, None]
+            for c in range(3):
+                two[..., c] += (Mi * self.dd_w[:, c, s][:, None]).sum(-1)
+        return -self._tangent(two) * self.kdz
+
+    def _between(self, a):
+        """Layer values at the interior interfaces."""
+        return a[:, :-1] * self.lo + a[:, 1:] * self.up
+
+    def _advection(self, Mh, Wh, W, rho):
+        q, fr = self.q, self.fr[:, None]
+        v = Mh / rho[..., None] + (W / rho)[..., None] * fr
+        adv = torch.stack(self._flux(Mh, v[..., 0], v[..., 1], v[..., 2])[1:], -1)
+        vh = v[:, :-1] * self.lo[:, None] + v[:, 1:] * self.up[:, None]
+        fl = torch.zeros(self.P, self.nv + 1, 3, dtype=torch.float64, device=DEVICE)
+        fl[:, 1:-1] = vh * (Wh[:, 1:-1] * self.r2h[1:-1])[..., None]
+        adv = adv + (fl[:, 1:] - fl[:, :-1]) / (self.dz * self.r2m)[:, None]
+        x, y, z = v.unbind(-1)
+        o = q["Omega"] * 2 * rho
+        if self.deep:
+            cor = torch.stack([-o * y, o * x, torch.zeros_like(x)], -1)
+        else:
+            f0, f1, f2 = (self.fr[:, k, None] for k in range(3))
+            cor = torch.stack([o * (z * f2 * f1 - y * f2 ** 2), -o * (z * f2 * f0 - x * f2 ** 2),
+                               o * (y * f2 * f0 - x * f2 * f1)], -1)
+        return adv + cor
+
+    def _thermo(self, s):
+        q, alt, alth, nv = self.q, self.alt, self.alth, self.nv
+        p, rho = s["pressure"], s["Rho"]
+        T = p / (rho * q["Rd"])
+        h = (q["Cp"] - q["Rd"]) * T + p / rho
+        pt = q["P_Ref"] / (q["Rd"] * rho) * (p / q["P_Ref"]) ** ((q["Cp"] - q["Rd"]) / q["Cp"])
+        z = torch.zeros_like(p[:, :1])
+        hh = torch.cat([h[:, :1], self._between(h), h[:, -1:]], 1)
+        e0 = (alth[0] - alt[1]) / (alt[1] - alt[0])
+        e1 = (2 * alth[-1] - alt[-1] - alt[-2]) / (alt[-1] - alt[-2])
+        pth = torch.cat([pt[:, 1:2] + (pt[:, 1:2] - pt[:, :1]) * e0, self._between(pt),
+                         pt[:, -2:-1] + (pt[:, -1:] - pt[:, -2:-1]) * e1], 1)
+        dp = (p[:, 1:] - p[:, :-1]) / (alt[1:] - alt[:-1])
+        rh = self._between(rho)
+        mid = -s["Wh"][:, 1:-1] / rh * dp
+        gi = torch.cat([z, mid, z], 1)
+        gtil = _center(gi, alt, alth)
+        below = p[:, 1:2] - rho[:, :1] * self.gz[0] * (-alt[0] - alt[1])
+        rb = rho[:, 1:2] + (rho[:, 1:2] - rho[:, :1]) * (-alt[0] - alt[1]) / (alt[1] - alt[0])
+        g0 = -(p[:, :1] - below) / (2 * alt[0]) / (0.5 * (rho[:, :1] + rb))
+        above = p[:, -2:-1] - rho[:, -1:] * self.gz[-1] * (2 * alth[-1] - alt[-1] - alt[-2])
+        ra = rho[:, -2:-1] + (rho[:, -1:] - rho[:, -2:-1]) * e1
+        g1 = -(above - p[:, -1:]) / (2 * (alth[-1] - alt[-1])) / (0.5 * (rho[:, -1:] + ra))
+        return T, h, pt, hh, pth, gtil, torch.cat([g0, -dp / rh, g1], 1)
+
+    def _slow(self, s, adv, T, h, hh, gtil, forcing):
+        q, fr = self.q, self.fr[:, None]
+        Mh, Wh, W, rho, p = (s[k] for k in STATE)
+        RoC = q["Rd"] / (q["Cp"] - q["Rd"])
+        a = torch.cat([rho[..., None], Mh / rho[..., None], (W / rho)[..., None], (q["Rd"] * T)[..., None]], -1)
+        for _ in range(self.case["order"] // 2 - 1):
+            a = self._laplacian(a)
+        a = torch.cat([a[..., :1], a[..., 1:] * rho[..., None]], -1)
+        a = self._laplacian(a) * (-self.kdh * (-1) ** (self.case["order"] // 2))
+        drho, dmh, dw, dpr = a[..., 0], self._tangent(a[..., 1:4]), a[..., 4], a[..., 5]
+        gp = self._gradient(p)
+        gpt = self._tangent(gp)
+        fr_, fh = self._flux(Mh, h)
+        slow_m = -gpt - self._tangent(adv) + self._divdamp(Mh, Wh) + dmh + forcing["dMh"]
+        advr = (adv * fr).sum(-1) if self.nonhydro else (Mh ** 2).sum(-1) / (rho * (self.alt + q["A"]))
+        grav = rho * self.gz + (advr if self.deep else 0.0)
+        swr = self._between(grav) + (p[:, 1:] - p[:, :-1]) / (self.alt[1:] - self.alt[:-1])
+        if self.nonhydro:
+            swr = swr - self._between(dw)
+        slow_w = torch.zeros_like(Wh)
+        slow_w[:, 1:-1] = -(swr - forcing["dWh"][:, 1:-1])
+        up = Wh * self.r2h
+        up = torch.cat([torch.zeros_like(up[:, :1]), up[:, 1:]], 1)
+        flat = (up[:, 1:] - up[:, :-1]) / (self.dz * self.r2m)
+        dwdz = torch.where(self.pole[:, None], flat, (up[:, 1:] - up[:, :-1]) / self.dr)
+        slow_r = -(fr_ + dwdz) + drho
+        uh = up * hh
+        vgp = (gpt * Mh).sum(-1) / rho
+        slow_p = RoC * (-fh - gtil - (uh[:, 1:] - uh[:, :-1]) / (self.dz * self.r2m) + vgp + forcing["Qheat"]) + dpr
+        return slow_m, slow_w, slow_r, slow_p, dpr
+
+    def _matrix(self, hh, gh, dt):
+        """Tridiagonal coefficients at the interior interfaces."""
+        q, alt, alth = self.q, self.alt, self.alth
+        CvoR = (q["Cp"] - q["Rd"]) / q["Rd"]
+        dzp, dzm, dzh = 1 / (alth[2:] - alth[1:-1]), 1 / (alth[1:-1] - alth[:-2]), 1 / (alt[1:] - alt[:-1])
+        CRdd = CvoR / dt ** 2
+        gl, gu = self.gz[:-1] * CvoR, self.gz[1:] * CvoR
+        GC = (gl * (alt[1:] - alth[1:-1]) + gu * (alth[1:-1] - alt[:-1])) * dzh
+        H = hh * self.r2h
+        o2 = 1 / self.r2h[1:-1]
+        o3 = 2 / (alth[1:-1] + q["A"]) ** 3 if self.deep else torch.zeros_like(o2)
+        il = (alt[1:] - alth[1:-1]) * dzp * dzh
+        im = -(alt[:-1] - alth[1:-1]) * dzm * dzh
+        c = -dzp * dzh * o2 * H[:, 2:] - im * (gh[:, 2:] + GC - o3 * H[:, 2:])
+        b = (dzp + dzm) * dzh * o2 * H[:, 1:-1] + (il - im) * (gh[:, 1:-1] + GC - o3 * H[:, 1:-1])
+        if self.nonhydro:
+            b = b + CRdd
+        a = -dzm * dzh * o2 * H[:, :-2] + il * (gh[:, :-2] + GC - o3 * H[:, :-2])
+        return a, b, c, CRdd
+
+    def _solve(self, a, b, c, d):
+        n = b.shape[1]
+        cs, ds = [c[:, 0] / b[:, 0]], [d[:, 0] / b[:, 0]]
+        for k in range(1, n):
+            t = 1 / (b[:, k] - cs[-1] * a[:, k])
+            cs.append(c[:, k] * t)
+            ds.append((d[:, k] - ds[-1] * a[:, k]) * t)
+        x = [ds[-1]]
+        for k in range(n - 2, -1, -1):
+            x.append(ds[k] - cs[k] * x[-1])
+        return torch.stack(x[::-1], 1)
+
+    def thor(self, y, forcing):
+        q, case = self.q, self.case
+        Rd, Cp = q["Rd"], q["Cp"]
+        Cv, RoC, P0 = Cp - Rd, Rd / (Cp - Rd), q["P_Ref"]
+        s = dict(y)
+        for rk in range(3):
+            n = (1, case["ns"] // 2, case["ns"])[rk]
+            dt = case["dt"] / 3 if rk == 0 else case["dt"] / case["ns"]
+            adv = self._advection(s["Mh"], s["Wh"], s["W"], s["Rho"])
+            T, h, pt, hh, pth, gtil, gh = self._thermo(s)
+            sm, sw, sr, sp, dpr = self._slow(s, adv, T, h, hh, gtil, forcing)
+            M = self._tangent(y["Mh"] - s["Mh"])
+            R, p = y["Rho"] - s["Rho"], y["pressure"] - s["pressure"]
+            w = y["Wh"] - s["Wh"]
+            w = torch.cat([torch.zeros_like(w[:, :1]), w[:, 1:-1], torch.zeros_like(w[:, :1])], 1)
+            a, b, c, CRdd = self._matrix(hh, gh, dt)
+            for _ in range(n):
+                M = M + self._tangent((-self._gradient(p) + sm + self._divdamp(M, w)) * dt)
+                fr_, fh = self._flux(M, h)
+                Sp, Sd = sp - RoC * fh, sr - fr_
+                dzi = 1 / (self.alt[1:] - self.alt[:-1])
+                rhs = (dt ** 2 * (Sp[:, 1:] - Sp[:, :-1]) * dzi + dt ** 2 * self.gz[1:] * self._between(Sd)
+                       + self.gz[1:] * dt * self._between(R) + dt * (p[:, 1:] - p[:, :-1]) * dzi - dt * sw[:, 1:-1])
+                if self.nonhydro:
+                    rhs = rhs - w[:, 1:-1]
+                w = torch.cat([torch.zeros_like(w[:, :1]), self._solve(a, b, c, -rhs * CRdd),
+                               torch.zeros_like(w[:, :1])], 1)
+                fpt = self._flux(M + s["Mh"], pt)[1]
+                up = w * self.r2h
+                flat = (up[:, 1:] - up[:, :-1]) / (self.dz * self.r2m)
+                dwdz = torch.where(self.pole[:, None], flat, (up[:, 1:] - up[:, :-1]) / self.dr)
+                u2 = (w + s["Wh"]) * pth * self.r2h
+                u2 = torch.cat([torch.zeros_like(u2[:, :1]), u2[:, 1:]], 1)
+                aux = -(fpt + (u2[:, 1:] - u2[:, :-1]) / (self.dz * self.r2m)) * dt
+                r = s["Rho"] + R
+                R = R + (sr - fr_ - dwdz) * dt
+                ptc = P0 / (Rd * r) * ((p + s["pressure"]) / P0) ** (Cv / Cp)
+                new = P0 * (Rd * (aux + ptc * r) / P0) ** (Cp / Cv)
+                p = new - s["pressure"] + dpr * dt + RoC * forcing["Qheat"] * dt
+            Wh = s["Wh"] + w
+            Wh = torch.cat([torch.zeros_like(w[:, :1]), Wh[:, 1:-1], torch.zeros_like(w[:, :1])], 1)
+            s = {"Mh": self._tangent(M + s["Mh"]), "Wh": Wh, "W": _center(Wh, self.alt, self.alth),
+                 "Rho": s["Rho"] + R, "pressure": s["pressure"] + p}
+        return s
+
+    # ------------------------------------------------------------ forcings
+    def _sponge(self, s):
+        q, sp, dt = self.q, sg.hot_jupiter_sponge(), self.case["dt"]
+        n = sp.nlat_bins
+        lon = torch.where(self.lon < 0, self.lon + 2 * math.pi, self.lon)
+        e1 = torch.stack([-torch.sin(lon), torch.cos(lon), torch.zeros_like(lon)], 1)
+        e2 = torch.stack([-torch.sin(self.lat) * torch.cos(lon), -torch.sin(self.lat) * torch.sin(lon),
+                          torch.cos(self.lat)], 1)
+        rho = s["Rho"]
+        u, v = (s["Mh"] * e1[:, None]).sum(-1) / rho, (s["Mh"] * e2[:, None]).sum(-1) / rho
+        w = s["W"] / rho
+        des = math.pi / n
+        edges = [-math.pi / 2]
+        for _ in range(n):
+            edges.append(edges[-1] + des)
+        band = torch.bucketize(self.lat.contiguous(), torch.tensor(edges[1:], dtype=torch.float64, device=DEVICE),
+                               right=True).clamp(max=n - 1)
+        count = torch.bincount(band, minlength=n).double()
+        center = -math.pi / 2 + 0.5 * des + des * torch.arange(n, device=DEVICE)
+        at = ((self.lat - center[0]) / des).clamp(0, n - 1)
+        i = at.floor().long().clamp(max=n - 2)
+        frac = (at - i)[:, None]
+        rate = torch.sin(0.5 * math.pi * (self.alt / q["top"] - sp.ns) / (1 - sp.ns)) ** 2
+        rate = torch.where(self.alt / q["top"] >= sp.ns, rate, 0.0)
+
+        def relax(a, R):
+            mean = torch.zeros(n, self.nv, dtype=torch.float64, device=DEVICE).index_add_(0, band, a) / count[:, None]
+            mean = mean[i] * (1 - frac) + mean[i + 1] * frac
+            return (a / dt + R * rate * mean) / (1 / dt + R * rate)
+        u, v, w = relax(u, sp.Ruv), relax(v, sp.Ruv), relax(w, sp.Rw)
+        W = w * rho
+        Wh = s["Wh"].clone()
+        Wh[:, 1:-1] = self._between(W)
+        M = (u[..., None] * e1[:, None] + v[..., None] * e2[:, None]) * rho[..., None]
+        return dict(s, Mh=M, W=W, Wh=Wh)
+
+    def _radiation(self, s, T):
+        """Double-gray heating. The optical depths of these columns stay far
+        above the thin-layer series' threshold."""
+        q, r, nv, alt, alth = self.q, sg.double_gray(), self.nv, self.alt, self.alth
+        p, rho = s["pressure"], s["Rho"]
+        Th = torch.cat([T[:, :1], self._between(T), T[:, -1:]], 1)
+        top = (p[:, -2] + (p[:, -1] - p[:, -2]) / (alt[-1] - alt[-2]) * (2 * alth[-1] - alt[-1] - alt[-2])).clamp(min=0)
+        ptop = 0.5 * (p[:, -1] + top)
+        mu = (torch.cos(self.lat) * torch.cos(self.lon - r.lon_sub)).clamp(min=0)
+        day = mu > 0
+        mu = torch.where(day, mu, 1.0)
+        tsw = r.n_sw * r.kappa_sw * (p / r.ps0) ** (r.n_sw - 1) * rho * self.dz
+        tlw = r.kappa_lw * (1 + r.n_lw * (1 - r.f_lw) / r.f_lw * (p / r.ps0) ** (r.n_lw - 1)) * rho * self.dz
+        sw = [r.incflx * mu * (1 - r.albedo) * torch.exp(-r.kappa_sw / q["Gravit"] * ptop / mu) * day]
+        for k in range(nv - 1, -1, -1):
+            sw.append(sw[-1] * torch.exp(-tsw[:, k] / mu))
+        net = -torch.stack(sw[::-1], 1)
+        bc, D = 5.677036e-8, r.diff_ang
+        B, Bh = bc * T ** 4, bc * Th ** 4
+
+        def source(b, l, t, tau):
+            x = tau / 2 / D
+            e = torch.exp(-x)
+            return (b - l + (l - (b - l) / x) * (1 - e)) + (l - t + (t - (l - t) / x) * (1 - e)) * e
+        dn, up = [torch.zeros_like(ptop)], []
+        for k in range(nv - 1, -1, -1):
+            dn.append(source(Bh[:, k], B[:, k], Bh[:, k + 1], tlw[:, k]) + dn[-1] * torch.exp(-tlw[:, k] / D))
+        dn = torch.stack(dn[::-1], 1)
+        up = [bc * r.Tint ** 4 + dn[:, 0]]
+        for k in range(nv):
+            up.append(source(Bh[:, k + 1], B[:, k], Bh[:, k], tlw[:, k]) + up[-1] * torch.exp(-tlw[:, k] / D))
+        net = net + torch.stack(up, 1) - dn
+        Q = (net[:, :-1] - net[:, 1:]) / self.dz
+        low = p + q["Rd"] / (q["Cp"] - q["Rd"]) * Q * self.case["dt"] < 0
+        return torch.where(low, -p / self.case["dt"], Q)
+
+    def _learned(self, s, T, exact):
+        q, nv, n = self.q, self.nv, _norm(self.case)
+        f = {k: _t(v).double() for k, v in n.items()}
+        mu = (torch.cos(self.lat) * torch.cos(self.lon)).clamp(min=0)
+        x = (torch.cat([T, torch.log(s["pressure"]), mu[:, None]], 1) - f["in_mean"]) / f["in_std"]
+        out = ((x < f["in_lo"]) | (x > f["in_hi"])).any(1)
+        w, k = _t(_network(nv)).double(), 0
+        for i, (a, b) in enumerate(((2 * nv + 1, HIDDEN), (HIDDEN, HIDDEN), (HIDDEN, nv))):
+            x = x @ w[k:k + a * b].reshape(a, b) + w[k + a * b:k + a * b + b]
+            k += a * b + b
+            if i < 2:
+                x = torch.nn.functional.gelu(x, approximate="tanh")
+        Q = x * f["out_std"] + f["out_mean"]
+        low = s["pressure"] + q["Rd"] / (q["Cp"] - q["Rd"]) * Q * self.case["dt"] < 0
+        Q = torch.where(low, -s["pressure"] / self.case["dt"], Q)
+        return torch.where(out[:, None], exact, Q)
+
+    def profx(self, s, step):
+        """The state after the forcing, and the tendencies it leaves."""
+        case, q, dt = self.case, self.q, self.case["dt"]
+        z = torch.zeros_like
+        none = {"Qheat": z(s["W"]), "dMh": z(s["Mh"]), "dWh": z(s["Wh"])}
+        s = dict(s, W=_center(s["Wh"], self.alt, self.alth))
+        if case["sponge"]:
+            s = self._sponge(s)
+        p, rho, Rd = s["pressure"], s["Rho"], q["Rd"]
+        T = p / (Rd * rho)
+        lon, lat = self.lon[:, None], self.lat[:, None]
+        if case["forcing"] == "held_suarez":
+            ps = 0.5 * (p[:, :1] + p[:, 1:2] - rho[:, :1] * q["Gravit"] * (-self.alt[0] - self.alt[1]))
+            s0, day = p / 1e5, 86400.0
+            x = ((p / ps - 0.7) / 0.3).clamp(min=0)
+            Teq = ((315 - 60 * torch.sin(lat) ** 2 - 10 * torch.log(s0) * torch.cos(lat) ** 2)
+                   * s0 ** (Rd / q["Cp"])).clamp(min=200)
+            kt = 1 / (40 * day) + (1 / (4 * day) - 1 / (40 * day)) * x * torch.cos(lat) ** 4
+            T = T - kt * dt * (T - Teq)
+            s = dict(s, Mh=s["Mh"] / (1 + x / day * dt)[..., None])
+        elif case["forcing"] == "newtonian":
+            n, lp = NEWTONIAN, torch.log(p)
+            lt, lb, lc = (math.log(n[k]) for k in ("p_top", "p_bottom", "p_contrast"))
+            Teq = n["T_mean"] + n["dT"] * ((lb - lp) / (lb - lc)).clamp(0, 1) * torch.cos(lon) * torch.cos(lat)
+            f = ((lp - lt) / (lb - lt)).clamp(0, 1)
+            tau = torch.exp(math.log(n["tau_top"]) + f * math.log(n["tau_bottom"] / n["tau_top"]))
+            T = (T + dt * Teq / tau) / (1 + dt / tau)
+        else:
+            Q = self._radiation(s, T)
+            if case["forcing"] == "surrogate" and step % JUDGE:
+                Q = self._learned(s, T, Q)
+            none["Qheat"] = Q
+        return dict(s, pressure=T * Rd * rho), none
+
+
+def _shuffled(n, seed):
+    """The order in which an epoch visits the rows: a Fisher-Yates shuffle on
+    the 64-bit Mersenne Twister (Matsumoto and Nishimura 1998)."""
+    full = (1 << 64) - 1
+    mt = [seed & full]
+    for i in range(1, 312):
+        mt.append((6364136223846793005 * (mt[-1] ^ (mt[-1] >> 62)) + i) & full)
+    at, out = 312, list(range(n))
+    for i in range(n - 1, 0, -1):
+        if at == 312:
+            for k in range(312):
+                x = (mt[k] & 0xFFFFFFFF80000000) | (mt[(k + 1) % 312] & 0x7FFFFFFF)
+                mt[k] = mt[(k + 156) % 312] ^ (x >> 1) ^ (0xB5026F5AA96619E9 if x & 1 else 0)
+            at = 0
+        x = mt[at]
+        at += 1
+        x ^= (x >> 29) & 0x5555555555555555
+        x ^= (x << 17) & 0x71D67FFFEDA60000
+        x ^= (x << 37) & 0xFFF7EEE000000000
+        x ^= x >> 43
+        j = x % (i + 1)
+        out[i], out[j] = out[j], out[i]
+    return out
+
+
+def _train_exact(case, seed):
+    X, Y = (_t(a).double() for a in _columns(case, seed))
+    nin, nv = 2 * case["nv"] + 1, case["nv"]
+    w = _t(_network(nv, seed % 1000)).double().requires_grad_(True)
+    m, v, total = torch.zeros_like(w), torch.zeros_like(w), 0.0
+    order = torch.tensor(_shuffled(case["rows"], seed), device=DEVICE)
+    for step, rows in enumerate(order.split(case["batch"]), 1):
+        x, k = X[rows], 0
+        for i, (a, b) in enumerate(((nin, HIDDEN), (HIDDEN, HIDDEN), (HIDDEN, nv))):
+            x = x @ w[k:k + a * b].reshape(a, b) + w[k + a * b:k + a * b + b]
+            k += a * b + b
+            if i < 2:
+                x = torch.nn.functional.gelu(x, approximate="tanh")
+        sq = ((x - Y[rows]) ** 2).sum()
+        total += float(sq.detach())
+        (grad,) = torch.autograd.grad(sq / (len(rows) * nv), w)
+        with torch.no_grad():
+            m = 0.9 * m + 0.1 * grad
+            v = 0.999 * v + 0.001 * grad ** 2
+            w -= LR * (m / (1 - 0.9 ** step)) / (torch.sqrt(v / (1 - 0.999 ** step)) + 1e-8)
+    return {"loss": total / case["rows"] / nv, "params": w.detach().cpu().numpy()}
+
+
+def exact(case, seed):
+    if case["kind"] == "train":
+        return _train_exact(case, seed)
+    core, s = _Exact(case), _state(case, seed)
+    if case["kind"] == "step":
+        return core.thor(s, _given_forcing(case, s))
+    for k in range(case["steps"]):
+        s, f = core.profx(s, k)
+        s = core.thor(s, f)
+    return s
