@@ -177,16 +177,16 @@ def _rest_column(case):
 
 def _norm(case):
     """Input and output scales of the network for the columns of _state: means
-    and spreads of T, ln p and cos z, and heating of the order of 1e-4 K/s. A few
-    columns in a thousand leave the envelope and take the exact radiation."""
+    and spreads of T, ln p and cos z, and heating of the order of 1e-4 K/s. From
+    none to a few columns in a hundred leave the envelope and take the exact radiation."""
     q, nv = _planet(case), case["nv"]
     _, p = _rest_column(case)
     heat = 1e-4 * p / (q["Rd"] * q["Tmean"]) * (q["Cp"] - q["Rd"])
     f = lambda *a: np.concatenate(a).astype(np.float32)  # noqa: E731
-    return {"in_mean": f(np.full(nv, q["Tmean"]), np.log(p), [0.25]), "in_std": f(np.full(nv, 20.0), np.full(nv, 0.02),
+    return {"in_mean": f(np.full(nv, q["Tmean"]), np.log(p), [0.25]), "in_std": f(np.full(nv, 20.0), np.full(nv, 0.05),
                                                                                   [0.32]),
-            "in_lo": f(np.full(nv, -4.5), np.full(nv, -8.0), [-2.0]),
-            "in_hi": f(np.full(nv, 4.5), np.full(nv, 8.0), [3.0]),
+            "in_lo": f(np.full(nv, -3.0), np.full(nv, -4.5), [-2.0]),
+            "in_hi": f(np.full(nv, 3.0), np.full(nv, 4.5), [3.0]),
             "out_mean": f(np.zeros(nv)), "out_std": f(heat)}
 
 
