@@ -31,7 +31,7 @@ namespace thor {
             return fail(THOR_ERR_HIP, std::string(#expr ": ") + hipGetErrorString(_e));             \
     } while (0)
 
-constexpr int kLC = 8;  // levels per thread in the stencil kernels
+constexpr int kLC = 8;  // levels per thread of the stage update
 
 struct KernelStat {
     long launches = 0;
@@ -96,10 +96,10 @@ struct Dyn {
     std::vector<std::string> stat_order;
     double diff_sign = 1.0;
     bool mixed = false;  // THOR_PRECISION_MIXED
-    int lc = 16;         // levels per block of the mixed-precision momentum and divergence stencils
-    int lc_prep = 16;    // levels per block of the mixed-precision prepare stencil
-    int lc_slow = 16;    // levels per block of the chunked slow modes
-    int tcb = 64;        // columns per block of the substep Thomas kernel (16, 32 or 64)
+    int lc = 0;          // levels per block of the level-chunked stencils (0 at create: chunk_levels)
+    int lc_slow = 0;     // levels per block of the chunked slow modes
+    int tcb = 0;         // columns per block of the substep Thomas kernel (16, 32 or 64; 0 at create: by size)
+    bool small = false;  // the grid's columns alone do not fill the chip (see thor_dyn_create)
     bool slow_lc = false;  // mixed path: level-chunked slow modes (k_divm1_lc + k_slow_lc)
     bool slow_v2 = true;   // mixed path: k_slow_lc2 (two blocks per CU) in place of k_slow_lc
     // Stage kernels that do not depend on the hyperdiffusion chain can run on
@@ -255,6 +255,25 @@ static double sponge_shrink(const Dyn &d, long step) {
     return rv;
 }
 
+// Levels per block of the level-chunked stencils. A chunk is a serial chain of
+// levels (each waits for its tile's loads) after a prologue worth about four of
+// them (weights, the first two tiles), and an XCD holds `slots` blocks at a
+// time, so a launch takes about rounds x (levels + 4), rounds = its blocks per
+// XCD over the slots. The chunk with the least of that: one level at 2 562
+// columns x 20 levels (1 115 -> 587 us per mixed step against 16 levels), 4 at
+// 10 242 x 40 (1 352 -> 1 020 us), 16 at 40 962 x 48 (12: +7 %, 24: +17 %). At
+// four rounds and more the tail no longer matters and 16 levels are kept.
+static int chunk_levels(int nv, int tiles_per_xcd, int slots) {
+    int best = std::min(nv, 16);
+    auto rounds = [&](int lc) { return (tiles_per_xcd * ((nv + lc - 1) / lc) + slots - 1) / slots; };
+    if (rounds(best) >= 4) return best;
+    for (int n = 1; n <= nv; n++) {
+        const int lc = (nv + n - 1) / n;
+        if (lc <= 32 && rounds(lc) * (lc + 4) < rounds(best) * (best + 4)) best = lc;
+    }
+    return best;
+}
+
 static Fields stage_fields(Dyn &d, int rk) {
     Fields f = d.f;
     f.Mh = d.Mh;
@@ -303,13 +322,12 @@ template <bool MX> static int thor_step_t(Dyn &d) {
     auto W = [&](double n64, double n32) { return MX ? 8.0 * N * n64 + 4.0 * N * n32 : 8.0 * N * (n64 + n32); };
     const int ns_total = d.prm.n_substeps;
     const int hydiff = d.prm.HyDiff, divdamp = d.prm.DivDampP;
-    const dim3 blk(kTile), grid_s((d.P + kTile - 1) / kTile, (d.nv + kLC - 1) / kLC);
+    const dim3 blk(kTile);
     const dim3 grid_t2(8 * d.g.tiles_per_xcd * d.nv);  // LDS-tiled stencils: one tile x one level per block
     // mixed-precision substep stencils: one tile x lc levels per block
     const dim3 grid_lc(8 * d.g.tiles_per_xcd * ((d.nv + d.lc - 1) / d.lc));
-    const dim3 grid_lp(8 * d.g.tiles_per_xcd * ((d.nv + d.lc_prep - 1) / d.lc_prep));
     const dim3 grid_ls(8 * d.g.tiles_per_xcd * ((d.nv + d.lc_slow - 1) / d.lc_slow));
-    const int lc = d.lc, lcp = d.lc_prep, lcs = d.lc_slow;
+    const int lc = d.lc, lcs = d.lc_slow;
     // FP64 multi-level stencils: one tile x NL levels per block
     const bool ml = !MX && d.fp64_ml;
     auto grid_ml = [&](int nl) { return dim3(8 * d.g.tiles_per_xcd * ((d.nv + nl - 1) / nl)); };
@@ -544,9 +562,9 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             // split form reads h and pt as FP32 copies and writes no Sd (the
             // mixed vertical solve forms it from hflx_r and SlowRho)
             launch(d, "prepare", MX && d.prep_split ? W(4, 5) : W(7, 3), [&] {
-                if (MX && d.prep_split) k_prepare_lc<true><<<grid_lp, blk, 0, st>>>(g, f, lcp);
-                else if (MX) k_prepare_lc<false><<<grid_lp, blk, 0, st>>>(g, f, lcp);
-                else if (ml && d.prep64) k_prepare_lc64<<<grid_lp, blk, 0, st>>>(g, f, lcp);
+                if (MX && d.prep_split) k_prepare_lc<true><<<grid_lc, blk, 0, st>>>(g, f, lc);
+                else if (MX) k_prepare_lc<false><<<grid_lc, blk, 0, st>>>(g, f, lc);
+                else if (ml && d.prep64) k_prepare_lc64<<<grid_lc, blk, 0, st>>>(g, f, lc);
                 else if (ml) k_prepare_ml<2><<<grid_ml(2), blk, 0, st>>>(g, f);
                 else k_prepare<MX><<<grid_t2, blk, 0, st>>>(g, f);
             });
@@ -595,7 +613,11 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             // next substep's divergence-damping pass 0
             if (next) divm0();
         }
-        launch(d, "update_rk2", W(16, 3), [&] { k_update_rk2<kLC, MX><<<grid_s, blk, 0, st>>>(g, f); });
+        launch(d, "update_rk2", W(16, 3), [&] {
+            const unsigned nc = (unsigned)((d.P + kTile - 1) / kTile);
+            if (d.small) k_update_rk2<1, MX><<<dim3(nc, d.nv), blk, 0, st>>>(g, f);
+            else k_update_rk2<kLC, MX><<<dim3(nc, (d.nv + kLC - 1) / kLC), blk, 0, st>>>(g, f);
+        });
         rk_arrays(1);
     }
     std::swap(d.Mh, d.Mhk);
@@ -639,6 +661,7 @@ static int profx(Dyn &d, int forcing) {
     Fields f = stage_fields(d, 0);
     const Geo g = d.g;
     const dim3 blk(kTile), grid_c((d.P + 63) / 64);  // 64 columns x 4 level rows per block
+    const dim3 grid_c16((d.P + 15) / 16);            // 16 columns x 16 level rows
     const double B = 8.0 * d.P * d.nv;
     const double dt = d.prm.timestep;
     if (d.sponge_on && d.spg.mode == 0) {
@@ -669,13 +692,15 @@ static int profx(Dyn &d, int forcing) {
         launch(d, "boundary_layer", 8 * B, [&] { k_bl_rayleigh<<<grid_c, blk, 0, d.stream>>>(g, f, d.bl, dt); });
     if (forcing == THOR_FORCING_HELD_SUAREZ) {
         launch(d, "profx_held_suarez", 24 * B, [&] {
-            k_profx_relax<THOR_FORCING_HELD_SUAREZ><<<grid_c, blk, 0, d.stream>>>(g, f, dt, 1, d.nr, d.bl);
+            if (d.small) k_profx_relax<THOR_FORCING_HELD_SUAREZ, 16><<<grid_c16, blk, 0, d.stream>>>(g, f, dt, 1, d.nr, d.bl);
+            else k_profx_relax<THOR_FORCING_HELD_SUAREZ, 64><<<grid_c, blk, 0, d.stream>>>(g, f, dt, 1, d.nr, d.bl);
         });
     } else if (forcing == THOR_FORCING_NEWTONIAN) {
         if (!d.nr_set) return fail(THOR_ERR_BAD_ARG, "profx: Newtonian forcing parameters not set");
         // W, T, relaxation and pressure per cell: Wh 2, p, rho, Mh untouched -> 4 in, W, p, Qheat out
         launch(d, "profx_newtonian", 7 * B, [&] {
-            k_profx_relax<THOR_FORCING_NEWTONIAN><<<grid_c, blk, 0, d.stream>>>(g, f, dt, 1, d.nr, d.bl);
+            if (d.small) k_profx_relax<THOR_FORCING_NEWTONIAN, 16><<<grid_c16, blk, 0, d.stream>>>(g, f, dt, 1, d.nr, d.bl);
+            else k_profx_relax<THOR_FORCING_NEWTONIAN, 64><<<grid_c, blk, 0, d.stream>>>(g, f, dt, 1, d.nr, d.bl);
         });
     } else if (forcing == THOR_FORCING_DOUBLE_GRAY) {
         if (!d.rt_set) return fail(THOR_ERR_BAD_ARG, "profx: RT parameters not set");
@@ -929,7 +954,7 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
     // Levels per block of the mixed-precision substep stencils (tuning knob).
     if (const char *e = std::getenv("THOR_STENCIL_LEVELS")) {
         const int v = std::atoi(e);
-        if (v >= 1 && v <= kLcMax) d.lc = d.lc_prep = d.lc_slow = v;
+        if (v >= 1 && v <= kLcMax) d.lc = d.lc_slow = v;
     }
     if (const char *e = std::getenv("THOR_SLOW_LEVELS")) {
         const int v = std::atoi(e);
@@ -1026,6 +1051,16 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
     g.nv = nv;
     g.nr = gd->nr;
     g.tiles_per_xcd = (gd->nr + 1 + 7) / 8;
+    // Two blocks per CU, one for the FP64 slow modes (their register budget).
+    const int slots = std::max(1, d.ncu / 8);
+    if (!d.lc) d.lc = chunk_levels(nv, g.tiles_per_xcd, 2 * slots);
+    if (!d.lc_slow) d.lc_slow = chunk_levels(nv, g.tiles_per_xcd, d.mixed ? 2 * slots : slots);
+    // Column kernels of 64-column blocks leave CUs without two blocks each: 16
+    // columns per block then (FP64 vertical solve 47.8 -> 27.9 us at 10 242 x 40,
+    // 40.4 -> 19.9 at 2 562 x 32; at 40 962 x 48, 640 blocks of 64, it is 97
+    // against 114), one level per thread in the stage update.
+    d.small = (P + 63) / 64 < 2 * d.ncu;
+    if (!d.tcb) d.tcb = d.small ? 16 : 64;
     g.A = prm->A;
     g.Omega = prm->Omega;
     g.Gravit = prm->Gravit;

@@ -4025,10 +4025,12 @@ __global__ __launch_bounds__(256) void k_bl_rayleigh(Geo g, Fields f, BLPar bl, 
     for (int lev = row; lev < g.nv; lev += NROW) bl_drag(g, f, bl, p, lev, LV(f.p, lev), ps, time_step);
 }
 
-template <int F>
+// (With few columns: 16 columns x 16 level rows, so each thread's serial walk
+// over the levels is a quarter as long and the chip holds four times the blocks.)
+template <int F, int CB>
 __global__ __launch_bounds__(256) void k_profx_relax(Geo g, Fields f, double time_step, int zero_q, NRPar nr,
                                                      BLPar bl) {
-    constexpr int CB = 64, NROW = 4;
+    constexpr int NROW = 256 / CB;
     const int c = threadIdx.x % CB, row = threadIdx.x / CB;
     const int p = blockIdx.x * CB + c;
     const bool valid = p < g.P;
