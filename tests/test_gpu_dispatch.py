@@ -46,3 +46,30 @@ def test_shapes_by_size_equal_the_fixed_ones(built, glevel, nv, precision):
     for k in STATE:
         assert np.isfinite(a[k]).all(), k
         assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("nv,extra", [
+    (3, {}), (20, {}), (33, dict(DeepModel=0, NonHydro=0)), (23, dict(HyDiffOrder=8)), (21, dict(thermo_equation=1)),
+    (20, dict(DivDampP=0)), (20, dict(HyDiff=0)),
+    (23, dict(DiffSponge=1, order_diff_sponge=2)), (20, dict(HyDiffOrder=6, DiffSponge=1, order_diff_sponge=4)),
+])
+def test_fp64_operator_weights_equal_the_triangle_walk(built, nv, extra):
+    """FP64 operators as weights per point against the reference's walk over
+    the triangles (THOR_FP64_MULTILEVEL), one step with every option that
+    reaches them. An operator is a sum of at most 84 products: in another order
+    it moves by at most 84 x 2^-53 = 9e-15 of its largest term, and ten substeps
+    add that up; 1e-12 of the field's scale (rho c_s for the momenta), as for
+    the production build against the oracle."""
+    capi = built
+    print(f"case: FP64 g4 L{nv} {extra}: operator weights vs triangle walk, 1 step", flush=True)
+    g = grid(capi, 4, nv)
+    p = earth_params(capi, 4, dt=600.0, ns=6, **extra)
+    st = capi.ic_rest(g, p, seed=2140 + nv, temperature_noise=1e-3, wind_noise=1.0)
+    a = _run(capi, g, p, st, {}, steps=1)
+    b = _run(capi, g, p, st, {"THOR_FP64_MULTILEVEL": "1"}, steps=1)
+    cs = np.sqrt(p.Cp / (p.Cp - p.Rd) * p.Rd * p.Tmean)
+    for k in STATE:
+        scale = np.abs(b["Rho"]).max() * cs if k in ("Mh", "Wh", "W") else np.abs(b[k]).max()
+        err = np.abs(a[k] - b[k]).max() / scale
+        print(f"  {k}: {err:.2e}")
+        assert err < 1e-12, k

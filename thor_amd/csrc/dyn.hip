@@ -5,6 +5,7 @@
 #include "../../include/thor_mlp.h"
 #include "common.h"
 #include "dyn_kernels.h"
+#include "dyn_kernels_lw.h"
 #include "dyn_kernels_ml.h"
 #include "mlp_internal.h"
 #include "tracer_kernels.h"
@@ -114,6 +115,7 @@ struct Dyn {
     hipEvent_t ev_s[4] = {};
     float *dmbuf = nullptr;  // mixed form: DivM of the slow modes, [3][nv][S], when overlapped
     bool slow_lc64 = false;  // FP64 path: k_divm1_ml + k_slow_lc2<false> in place of k_slow<false>
+    bool lw = false;       // FP64 path: horizontal operators as FP64 weights over level chunks (*_lw kernels)
     bool fp64_ml = true;   // FP64 path: horizontal stencils over several levels per block (*_ml kernels)
     int ml_nl = 4;         // FP64 path: levels per block of the divergence-damping pass 0 and momentum (2 or 4)
     bool diff2_split64 = true;  // FP64 path: the last hyperdiffusion pass and the stage divergence-damping pass 0
@@ -330,6 +332,8 @@ template <bool MX> static int thor_step_t(Dyn &d) {
     const int lc = d.lc, lcs = d.lc_slow;
     // FP64 multi-level stencils: one tile x NL levels per block
     const bool ml = !MX && d.fp64_ml;
+    // FP64 weights over level chunks, in place of the triangle walk
+    const bool lw = !MX && d.lw;
     auto grid_ml = [&](int nl) { return dim3(8 * d.g.tiles_per_xcd * ((d.nv + nl - 1) / nl)); };
     // column_prep: (256 columns, level 0..nv) per block, XCD-major
     const dim3 grid_c(8 * (((d.P + kTile - 1) / kTile + 7) / 8) * (d.nv + 1));
@@ -426,6 +430,7 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             });
         launch(d, "adv_diff1", W(8 + (hydiff ? 7 : 0), 3 + (hydiff ? 6 : 0)), [&] {
             if (MX) k_adv_diff1_lc<<<grid_lc, blk, 0, st>>>(g, f, hydiff, lc);
+            else if (lw) k_adv_diff1_lw<<<grid_lc, blk, 0, st>>>(g, f, hydiff, lc);
             else if (ml) k_adv_diff1_ml<2><<<grid_ml(2), blk, 0, st>>>(g, f, hydiff);
             else k_adv_diff1<MX><<<grid_t2, blk, 0, st>>>(g, f, hydiff);
         });
@@ -440,8 +445,14 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             for (int ih = 0; ih < d.prm.HyDiffOrder / 2 - 2; ih++) {
                 auto *src = FS<MX>::diff(fd);
                 auto *dst = ih % 2 ? FS<MX>::diff(f) : FS<MX>::diffx(f);
-                launch(d, "diff_mid", W(0, 12),
-                       [&] { k_diff_mid<MX><<<grid_t2, blk, 0, st>>>(g, src, dst, (float)d.mid_scale); });
+                launch(d, "diff_mid", W(0, 12), [&] {
+                    if constexpr (!MX)
+                        if (lw) {
+                            k_diff_lw<false><<<grid_lc, blk, 0, st>>>(g, f, src, dst, 1.0, lc);
+                            return;
+                        }
+                    k_diff_mid<MX><<<grid_t2, blk, 0, st>>>(g, src, dst, (float)d.mid_scale);
+                });
                 FS<MX>::set_diff(fd, dst);
             }
             // pass s writes diff (s even) or the second array (s odd); the
@@ -456,6 +467,12 @@ template <bool MX> static int thor_step_t(Dyn &d) {
                 launch(d, "diff2", W(1, 12 + 12), [&] { k_diff2_lc<<<grid_lc, blk, 0, st>>>(g, fd, last_sign, lc); });
             if (divdamp && !ovl_divm)
                 launch(d, "divm0_stage", W(4, 3), [&] { k_divm0_lc<true><<<grid_lc, blk, 0, st>>>(g, f, lc); });
+        } else if (lw) {
+            if (hydiff)
+                launch(d, "diff2", W(1, 12 + 12),
+                       [&] { k_diff_lw<true><<<grid_lc, blk, 0, st>>>(g, fd, fd.diff, nullptr, last_sign, lc); });
+            if (divdamp)
+                launch(d, "divm0_stage", W(4, 3), [&] { k_divm0_lw<true><<<grid_lc, blk, 0, st>>>(g, f, lc); });
         } else if (ml && d.diff2_split64) {
             // FP64: the last hyperdiffusion pass, then divergence-damping pass 0
             // on the stage values, each kernel with its own register budget
@@ -529,7 +546,10 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             // FP64: DivM over several levels per block into the idle
             // hyperdiffusion scratch, then the slow modes over level chunks
             if (divdamp)
-                launch(d, "divm1", W(0, 6), [&] { k_divm1_ml<4><<<grid_ml(4), blk, 0, st>>>(g, f, f.diff); });
+                launch(d, "divm1", W(0, 6), [&] {
+                    if (lw) k_divm1_lw<<<grid_lc, blk, 0, st>>>(g, f, f.diff, lc);
+                    else k_divm1_ml<4><<<grid_ml(4), blk, 0, st>>>(g, f, f.diff);
+                });
             // booked as the reference's slow modes with DivM pass 1 (as the per-level kernel)
             launch(d, "slow_modes", W(19 + (rk ? 16 : 0), (divdamp ? 6 : 0) + 21 + (rk ? 3 : 0)),
                    [&] { k_slow_lc2<false><<<grid_ls, blk, 0, st>>>(g, f, f.diff, divdamp, rk, lcs); });
@@ -541,6 +561,7 @@ template <bool MX> static int thor_step_t(Dyn &d) {
         auto divm0 = [&] {
             launch(d, "divm0", W(1, 6), [&] {
                 if (MX) k_divm0_lc<false><<<grid_lc, blk, 0, st>>>(g, f, lc);
+                else if (lw) k_divm0_lw<false><<<grid_lc, blk, 0, st>>>(g, f, lc);
                 else if (ml && d.ml_nl == 2) k_divm0_ml<2><<<grid_ml(2), blk, 0, st>>>(g, f);
                 else if (ml) k_divm0_ml<4><<<grid_ml(4), blk, 0, st>>>(g, f);
                 else k_divm0<MX><<<grid_t2, blk, 0, st>>>(g, f);
@@ -553,6 +574,7 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             const int next = divdamp && ns < ns_it - 1;
             launch(d, "momentum", W(1, (divdamp ? 6 : 0) + 12), [&] {
                 if (MX) k_momentum_lc<<<grid_lc, blk, 0, st>>>(g, f, divdamp, times, lc);
+                else if (lw) k_momentum_lw<<<grid_lc, blk, 0, st>>>(g, f, divdamp, times, lc);
                 else if (ml && d.ml_nl == 2) k_momentum_ml<2><<<grid_ml(2), blk, 0, st>>>(g, f, divdamp, times);
                 else if (ml) k_momentum_ml<4><<<grid_ml(4), blk, 0, st>>>(g, f, divdamp, times);
                 else k_momentum<MX><<<grid_t2, blk, 0, st>>>(g, f, divdamp, times);
@@ -1111,6 +1133,15 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
         if (v == 1 || v == 2 || v == 4) d.cp_lv = v;
     }
     if (const char *e = std::getenv("THOR_PREPARE_SPLIT")) d.prep_split = d.prep_split && std::atoi(e) != 0;
+    // FP64 operators as weights: the production build (the parity build keeps
+    // the reference's operation order). The switches below choose among kernels
+    // in that order, so setting one of them keeps it too.
+#ifndef THOR_PORTABLE_MATH
+    d.lw = !d.mixed;
+    for (const char *k : {"THOR_SLOW_CHUNKED", "THOR_FP64_MULTILEVEL", "THOR_ML_LEVELS", "THOR_PREPARE_LC64",
+                          "THOR_DIFF2_SPLIT64"})
+        if (std::getenv(k)) d.lw = false;
+#endif
     if (const char *e = std::getenv("THOR_FP64_MULTILEVEL")) d.fp64_ml = std::atoi(e) != 0;
     if (const char *e = std::getenv("THOR_ML_LEVELS")) {
         const int v = std::atoi(e);
@@ -1183,6 +1214,22 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
         }
         if (e != hipSuccess)
             return cleanup_fail(fail(THOR_ERR_HIP, std::string("thor_dyn_create: level table: ") + hipGetErrorString(e)));
+    }
+    if (d.lw) {
+        double *wlap = nullptr, *wdd = nullptr, *udd = nullptr, *et = nullptr, *wdt = nullptr, *wgt = nullptr;
+        A(&wlap, (size_t)6 * S); A(&wdd, (size_t)63 * S); A(&udd, (size_t)21 * S);
+        A(&et, (size_t)6 * S); A(&wdt, (size_t)42 * S); A(&wgt, (size_t)14 * S);
+        if (e == hipSuccess) {
+            Geo gu = g;
+            gu.deep = 0;  // rscale = 1
+            k_probe_weights64<<<(P + 255) / 256, 256, 0, d.stream>>>(gu, wlap, wdd, udd, et, wdt, wgt);
+            e = hipGetLastError();
+            if (e == hipSuccess) e = hipStreamSynchronize(d.stream);
+            g.wlap64 = wlap; g.wdd64 = wdd; g.udd64 = udd;
+            g.et64 = et; g.wdt64 = wdt; g.wgt64 = wgt;
+        }
+        if (e != hipSuccess)
+            return cleanup_fail(fail(THOR_ERR_HIP, std::string("thor_dyn_create: operator weights: ") + hipGetErrorString(e)));
     }
     if (d.mixed) {
         auto F = [&](float **ptr, size_t n) {

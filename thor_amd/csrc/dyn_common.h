@@ -44,6 +44,16 @@ struct Geo {
     const float *wlap;  // [7][S]
     const float *wdd;   // [63][S]
     const float *udd;   // [21][S]
+    // FP64 form of the production build: the same operators as FP64 weights
+    // (k_probe_weights64): Laplacian slots 1..6, divergence damping, and the
+    // tangent basis of each point with the tangential components of the
+    // damping and of the gradient.
+    const double *wlap64;  // [6][S]
+    const double *wdd64;   // [63][S]
+    const double *udd64;   // [21][S]
+    const double *et64;    // [6][S]
+    const double *wdt64;   // [42][S]
+    const double *wgt64;   // [14][S]
     // Mixed precision only: per-level FP32 constants [4][nv]: rscale, rscale^2,
     // 1 / (Alth[lev] - Alth[lev + 1]) and Kdhz.
     const float *lvc;
