@@ -254,3 +254,41 @@ def test_concurrent_fallback_equals_sequential(built):
         assert np.array_equal(a[k], b[k]), k
     assert np.array_equal(qa, qb)
     m.close()
+
+
+@pytest.mark.parametrize("nin,nout,rows", [(3, 1, 1), (33, 16, 31), (97, 48, 257), (128, 64, 2100)])
+def test_fused_training_kernels_match_oracle(built, nin, nout, rows):
+    """The two-launch training form (n_hidden 256, n_in <= 128, n_out <= 64) at the
+    edges of its 32-row groups and 32 x 32 gradient tiles, against the oracle;
+    tolerances as test_gradients_match_oracle. Then Adam's first step: the
+    parameters move by at most lr, against the gradient's sign where the
+    gradient is not near zero, and the operand copies follow (the next
+    forward uses the new parameters)."""
+    from oracle import mlp_oracle as mo
+    capi = built
+    dims = (nin, 256, nout)
+    print(f"case: MLP {nin}-256-256-{nout} gradients and one Adam step, {rows} rows", flush=True)
+    m = capi.MLP(*dims, seed=9)
+    rng = np.random.default_rng(rows)
+    X = rng.standard_normal((rows, nin)).astype(np.float32)
+    T = rng.standard_normal((rows, nout)).astype(np.float32)
+    g, loss = m.gradients(X, T)
+    lo, go = mo.loss_and_grad(m.params(), X, T, dims, bf=True)
+    assert abs(loss / lo - 1) < 1e-3
+    bg, bo = _blocks(g, dims), _blocks(go, dims)
+    for k in bg:
+        e = np.linalg.norm(bg[k] - bo[k]) / np.linalg.norm(bo[k])
+        print(f"  d{k}: relative L2 diff {e:.2e}")
+        assert e < 3e-2, k
+    p0 = m.params()
+    m.set_data(X, T)
+    first = m.train_epoch(rows, 1e-3, 3)
+    assert abs(first / loss - 1) < 1e-6
+    d = m.params() - p0
+    assert np.abs(d).max() < 1.01e-3
+    big = np.abs(g) > 0.1 * np.abs(g).max()
+    assert (np.sign(d[big]) == -np.sign(g[big])).all()
+    Y = m.forward(X)
+    Yo, _ = mo.forward(m.params(), X, dims, bf=True)
+    assert np.abs(Y - Yo).max() / np.abs(Yo).max() < 1e-2
+    m.close()

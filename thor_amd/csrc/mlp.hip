@@ -6,6 +6,7 @@
 #include "common.h"
 #include "mlp_internal.h"
 #include "mlp_kernels.h"
+#include "mlp_train.h"
 
 #include <hip/hip_runtime.h>
 
@@ -34,6 +35,13 @@ struct Net {
     int kpad = 0;
     int ncu = 0;  // compute units of the device: inference blocks
     uint16_t *wt1 = nullptr, *wt2 = nullptr, *wt3 = nullptr;
+    // the fused training kernels' operands: W2 and W3 by rows, and per group of
+    // 32 rows the fragments of inputs, activations and deltas, the bias sums
+    // and the squared errors (tcap groups, tparts error sums)
+    uint16_t *wa2 = nullptr, *wa3 = nullptr, *tfrag = nullptr;
+    float *tbias = nullptr;
+    double *tpart = nullptr;
+    long tcap = 0, tparts = 0;
     long step = 0;
     // activations for up to cap rows
     long cap = 0;
@@ -151,24 +159,91 @@ static void backward(Net &n, long rows, int loss_slot) {
 }
 
 static void refresh_bf16(Net &n) {
+    if (n.fused) {
+        struct { const float *src; int K, N; uint16_t *dst; int Kp, Np, byrow; } c[5] = {
+            {n.w + n.oW1(), n.nin, n.nh, n.wt1, n.kpad, n.nh, 0}, {n.w + n.oW2(), n.nh, n.nh, n.wt2, n.nh, n.nh, 0},
+            {n.w + n.oW3(), n.nh, n.nout, n.wt3, n.nh, 64, 0},    {n.w + n.oW2(), n.nh, n.nh, n.wa2, n.nh, n.nh, 1},
+            {n.w + n.oW3(), n.nout, n.nh, n.wa3, 64, n.nh, 1}};
+        for (const auto &f : c)
+            k_frag_bf16<<<(unsigned)(((long)f.Np * f.Kp + 255) / 256), 256, 0, n.stream>>>(f.src, f.K, f.N, f.dst, f.Kp,
+                                                                                         f.Np, f.byrow);
+        return;
+    }
     const long nw[3] = {(long)n.nin * n.nh, (long)n.nh * n.nh, (long)n.nh * n.nout};
     const long src[3] = {n.oW1(), n.oW2(), n.oW3()}, dst[3] = {n.bW1(), n.bW2(), n.bW3()};
     for (int i = 0; i < 3; i++)
         k_to_bf16<<<(unsigned)((nw[i] + 255) / 256), 256, 0, n.stream>>>(n.w + src[i], n.wb + dst[i], nw[i]);
-    if (n.fused) {
-        const int K[3] = {n.nin, n.nh, n.nh}, N[3] = {n.nh, n.nh, n.nout};
-        const int Kp[3] = {n.kpad, n.nh, n.nh}, Np[3] = {n.nh, n.nh, 64};
-        uint16_t *wt[3] = {n.wt1, n.wt2, n.wt3};
-        for (int i = 0; i < 3; i++) {
-            const long cnt = (long)Np[i] * Kp[i];
-            k_frag_bf16<<<(unsigned)((cnt + 255) / 256), 256, 0, n.stream>>>(n.w + src[i], K[i], N[i], wt[i], Kp[i],
-                                                                             Np[i]);
-        }
-    }
 }
 
 static InferWeights infer_weights(const Net &n) {
     return InferWeights{n.wt1, n.wt2, n.wt3, n.w + n.ob1(), n.w + n.ob2(), n.w + n.ob3(), n.nin, n.nout, n.kpad};
+}
+
+// Room for a fused batch of `groups` 32-row groups and `parts` error sums.
+static hipError_t ensure_train(Net &n, long groups, long parts) {
+    auto grow = [&](auto **p, size_t count) {
+        if (*p) {
+            auto it = std::find(n.allocs.begin(), n.allocs.end(), (void *)*p);
+            if (it != n.allocs.end()) n.allocs.erase(it);
+            (void)hipFree(*p);
+            *p = nullptr;
+        }
+        return alloc(n, p, count);
+    };
+    hipError_t e = hipSuccess;
+    if (groups > n.tcap) {
+        n.tcap = 0;
+        e = grow(&n.tfrag, (size_t)groups * (n.kpad / 16 + 4 * 16 + 4) * 512);
+        if (e == hipSuccess) e = grow(&n.tbias, (size_t)groups * kBiasCols);
+        if (e == hipSuccess) n.tcap = groups;
+    }
+    if (e == hipSuccess && parts > n.tparts) {
+        n.tparts = 0;
+        e = grow(&n.tpart, (size_t)parts);
+        if (e == hipSuccess) n.tparts = parts;
+    }
+    return e;
+}
+
+// One fused batch: rows idx[0..rows) (null: 0..rows) of X, Y; the groups' error
+// sums into part; Adam's update (adam.m set) or the gradients into n.grad.
+static void train_batch(Net &n, const float *X, const float *Y, const int *idx, long rows, double *part,
+                        const AdamArgs &adam) {
+    const long nb = (rows + 31) / 32;
+    uint16_t *f = n.tfrag;
+    auto take = [&](int tiles) {
+        uint16_t *p = f;
+        f += (size_t)n.tcap * tiles * 512;
+        return p;
+    };
+    TrainArgs t{};
+    t.X = X;
+    t.Y = Y;
+    t.idx = idx;
+    t.rows = rows;
+    t.w = infer_weights(n);
+    t.wa2 = n.wa2;
+    t.wa3 = n.wa3;
+    t.scale = 2.0f / (float)(rows * n.nout);
+    t.fX = take(n.kpad / 16);
+    t.fH1 = take(16);
+    t.fH2 = take(16);
+    t.fZ1 = take(16);
+    t.fZ2 = take(16);
+    t.fY = take(4);
+    t.bpart = n.tbias;
+    t.part = part;
+    auto go = [&](auto kern) { kern<<<(unsigned)nb, kInferThreads, 0, n.stream>>>(t); };
+    switch (n.kpad / 32) {
+    case 1: go(k_train_rows<1>); break;
+    case 2: go(k_train_rows<2>); break;
+    case 3: go(k_train_rows<3>); break;
+    default: go(k_train_rows<4>); break;
+    }
+    GradArgs g{t.fX, t.fH1, t.fH2, t.fZ1, t.fZ2, t.fY, t.bpart, (int)nb, n.nin, n.nout, n.kpad, n.grad, adam,
+               n.wt1, n.wt2, n.wt3, n.wa2, n.wa3};
+    const int tiles = (n.nin + 31) / 32 * 8 + 64 + 8 * ((n.nout + 31) / 32);
+    k_train_weights<<<(unsigned)(tiles + kBiasCols / 64), 256, 0, n.stream>>>(g);
 }
 
 // Inference over rows of X0 into Y: the fused kernel when the shape allows it,
@@ -188,9 +263,9 @@ static void infer(Net &n, long rows) {
     }
 }
 
-static double sum_loss(Net &n, int slots) {
+static double sum_loss(Net &n, const double *dev, long slots) {
     std::vector<double> part((size_t)slots);
-    (void)hipMemcpyAsync(part.data(), n.loss_part, slots * sizeof(double), hipMemcpyDeviceToHost, n.stream);
+    (void)hipMemcpyAsync(part.data(), dev, slots * sizeof(double), hipMemcpyDeviceToHost, n.stream);
     (void)hipStreamSynchronize(n.stream);
     double s = 0.0;
     for (double v : part) s += v;
@@ -255,6 +330,8 @@ extern "C" thor_status thor_mlp_create(int n_in, int n_hidden, int n_out, unsign
         if (e == hipSuccess) e = alloc(n, &n.wt1, (size_t)256 * n.kpad);
         if (e == hipSuccess) e = alloc(n, &n.wt2, (size_t)256 * 256);
         if (e == hipSuccess) e = alloc(n, &n.wt3, (size_t)64 * 256);
+        if (e == hipSuccess) e = alloc(n, &n.wa2, (size_t)256 * 256);
+        if (e == hipSuccess) e = alloc(n, &n.wa3, (size_t)256 * 64);
     }
     if (e != hipSuccess) {
         thor_mlp_destroy(m);
@@ -335,7 +412,13 @@ extern "C" thor_status thor_mlp_train_epoch(thor_mlp *m, int batch, float lr, un
     Net &n = *m;
     const long nb = (n.ndata + batch - 1) / batch;
     MLP_TRY(wait_users(n));
-    MLP_TRY(ensure_cap(n, batch));
+    const long rmax = std::min<long>(batch, n.ndata), gpb = (rmax + 31) / 32;  // 32-row groups per batch
+    if (n.fused) {
+        if (gpb > n.tcap || nb * gpb > n.tparts) MLP_TRY(hipStreamSynchronize(n.stream));
+        MLP_TRY(ensure_train(n, gpb, nb * gpb));
+    } else {
+        MLP_TRY(ensure_cap(n, batch));
+    }
     // seeded shuffle on the host
     std::vector<int> perm((size_t)n.ndata);
     std::iota(perm.begin(), perm.end(), 0);
@@ -346,6 +429,13 @@ extern "C" thor_status thor_mlp_train_epoch(thor_mlp *m, int batch, float lr, un
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     for (long b = 0; b < nb; b++) {
         const long r0 = b * batch, rows = std::min<long>(batch, n.ndata - r0);
+        if (n.fused) {
+            n.step++;
+            const AdamArgs a{n.w, n.gm, n.gv, lr, b1, b2, eps, 1.0f - std::pow(b1, (float)n.step),
+                             1.0f - std::pow(b2, (float)n.step)};
+            train_batch(n, n.Xall, n.Yall, n.idx + r0, rows, n.tpart + b * gpb, a);
+            continue;
+        }
         k_gather<<<(unsigned)((rows * std::max(n.nin, n.nout) + 255) / 256), 256, 0, n.stream>>>(
             n.Xall, n.Yall, n.idx + r0, rows, n.nin, n.nout, n.X0, n.T);
         forward(n, rows);
@@ -357,8 +447,11 @@ extern "C" thor_status thor_mlp_train_epoch(thor_mlp *m, int batch, float lr, un
                                                                      bc1, bc2);
         refresh_bf16(n);
         MLP_TRY(hipGetLastError());
-        total += sum_loss(n, (int)((rows * n.nout + 255) / 256));  // sum of squared errors of the batch
+        total += sum_loss(n, n.loss_part, (rows * n.nout + 255) / 256);  // sum of squared errors of the batch
     }
+    MLP_TRY(hipGetLastError());
+    // fused: every batch left its groups' sums (the last batch has the fewest)
+    if (n.fused) total = sum_loss(n, n.tpart, (nb - 1) * gpb + (n.ndata - (nb - 1) * batch + 31) / 32);
     if (loss) *loss = total / (double)n.ndata / n.nout;
     return THOR_OK;
 }
@@ -389,12 +482,19 @@ extern "C" thor_status thor_mlp_gradients(thor_mlp *m, const float *X, const flo
     Net &net = *m;
     MLP_TRY(wait_users(net));
     MLP_TRY(ensure_cap(net, n));
+    const long groups = (n + 31) / 32;
+    if (net.fused) MLP_TRY(ensure_train(net, groups, groups));
     float *dX = nullptr;
     MLP_TRY(hipMalloc((void **)&dX, (size_t)n * net.nin * sizeof(float)));
     hipError_t e = hipMemcpyAsync(dX, X, (size_t)n * net.nin * sizeof(float), hipMemcpyHostToDevice, net.stream);
     if (e == hipSuccess) e = hipMemcpyAsync(net.T, Y, (size_t)n * net.nout * sizeof(float), hipMemcpyHostToDevice, net.stream);
-    if (e == hipSuccess) e = hipMemsetAsync(net.loss_part, 0, net.nloss_part * sizeof(double), net.stream);
-    if (e == hipSuccess) {
+    if (e == hipSuccess && net.fused) {
+        train_batch(net, dX, net.T, nullptr, n, net.tpart, AdamArgs{});
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess && !net.fused)
+        e = hipMemsetAsync(net.loss_part, 0, net.nloss_part * sizeof(double), net.stream);
+    if (e == hipSuccess && !net.fused) {
         k_to_bf16<<<(unsigned)((n * net.nin + 255) / 256), 256, 0, net.stream>>>(dX, net.X0, n * net.nin);
         forward(net, n);
         backward(net, n, 0);
@@ -404,7 +504,9 @@ extern "C" thor_status thor_mlp_gradients(thor_mlp *m, const float *X, const flo
     if (e == hipSuccess) e = hipStreamSynchronize(net.stream);
     (void)hipFree(dX);
     if (e != hipSuccess) return fail(THOR_ERR_HIP, std::string("thor_mlp_gradients: ") + hipGetErrorString(e));
-    if (loss) *loss = sum_loss(net, (int)((n * net.nout + 255) / 256)) / (double)(n * net.nout);
+    if (loss)
+        *loss = (net.fused ? sum_loss(net, net.tpart, groups) : sum_loss(net, net.loss_part, (n * net.nout + 255) / 256))
+                / (double)(n * net.nout);
     return THOR_OK;
 }
 

@@ -160,8 +160,9 @@ template <int KT1> __global__ __launch_bounds__(kInferThreads, 1) void k_mlp_inf
 // read their MFMA B operands: for each 32 x 16 tile (kt, nt) of W, lane l's
 // eight values W[32 kt + 8 (l / 16) + e][16 nt + l % 16], e = 0..7, are at
 // ((nt * Kpad / 32 + kt) * 64 + l) * 8 + e, so a wave's operand load is 1024
-// contiguous bytes. Zero beyond K and N.
-__global__ void k_frag_bf16(const float *src, int K, int N, uint16_t *dst, int Kpad, int Npad) {
+// contiguous bytes. Zero beyond K and N. byrow: W is stored [N][K] (the
+// operand of the transposed product in training).
+__global__ void k_frag_bf16(const float *src, int K, int N, uint16_t *dst, int Kpad, int Npad, int byrow) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (long)Npad * Kpad) return;
     const int KT = Kpad / 32;
@@ -169,7 +170,7 @@ __global__ void k_frag_bf16(const float *src, int K, int N, uint16_t *dst, int K
     const long tile = i >> 9;
     const int kt = (int)(tile % KT), nt = (int)(tile / KT);
     const int n = 16 * nt + (l & 15), k = 32 * kt + 8 * (l >> 4) + e;
-    dst[i] = (n < N && k < K) ? f2bf(src[(size_t)k * N + n]) : (uint16_t)0;
+    dst[i] = (n < N && k < K) ? f2bf(src[byrow ? (size_t)n * K + k : (size_t)k * N + n]) : (uint16_t)0;
 }
 
 __global__ void k_to_bf16(const float *src, uint16_t *dst, long n) {
