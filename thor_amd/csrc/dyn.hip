@@ -116,6 +116,8 @@ struct Dyn {
     float *dmbuf = nullptr;  // mixed form: DivM of the slow modes, [3][nv][S], when overlapped
     bool slow_lc64 = false;  // FP64 path: k_divm1_ml + k_slow_lc2<false> in place of k_slow<false>
     bool lw = false;       // FP64 path: horizontal operators as FP64 weights over level chunks (*_lw kernels)
+    bool rows64 = false;   // FP64 path with lw: the mixed form's vertical solve (all rows sweep, one power per
+                           // cell) and its split flux divergence, in FP64 storage
     bool fp64_ml = true;   // FP64 path: horizontal stencils over several levels per block (*_ml kernels)
     int ml_nl = 4;         // FP64 path: levels per block of the divergence-damping pass 0 and momentum (2 or 4)
     bool diff2_split64 = true;  // FP64 path: the last hyperdiffusion pass and the stage divergence-damping pass 0
@@ -410,7 +412,7 @@ template <bool MX> static int thor_step_t(Dyn &d) {
         auto factor = [&](hipStream_t on) {
             launch(d, "thomas_factor", 5 * B, [&] {
                 const int fseg = (d.nv - 1 + 7) / 8;  // interfaces per row of the segment form (32 columns)
-                if (MX && d.fseg && d.nv > 1 && fseg <= 8) {
+                if ((MX || d.rows64) && d.fseg && d.nv > 1 && fseg <= 8) {
                     const dim3 gs((d.P + 31) / 32);
                     if (fseg <= 6) k_thomas_factor_seg<32, 6><<<gs, 256, 0, on>>>(g, f, times);
                     else k_thomas_factor_seg<32, 8><<<gs, 256, 0, on>>>(g, f, times);
@@ -552,7 +554,10 @@ template <bool MX> static int thor_step_t(Dyn &d) {
                 });
             // booked as the reference's slow modes with DivM pass 1 (as the per-level kernel)
             launch(d, "slow_modes", W(19 + (rk ? 16 : 0), (divdamp ? 6 : 0) + 21 + (rk ? 3 : 0)),
-                   [&] { k_slow_lc2<false><<<grid_ls, blk, 0, st>>>(g, f, f.diff, divdamp, rk, lcs); });
+                   [&] {
+                       if (d.rows64) k_slow_lc2<false, true><<<grid_ls, blk, 0, st>>>(g, f, f.diff, divdamp, rk, lcs);
+                       else k_slow_lc2<false><<<grid_ls, blk, 0, st>>>(g, f, f.diff, divdamp, rk, lcs);
+                   });
         } else {
             launch(d, "slow_modes", W(19 + (rk ? 16 : 0), (divdamp ? 6 : 0) + 21 + (rk ? 3 : 0)),
                    [&] { k_slow<MX><<<grid_t2, blk, 0, st>>>(g, f, divdamp, rk); });
@@ -586,6 +591,7 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             launch(d, "prepare", MX && d.prep_split ? W(4, 5) : W(7, 3), [&] {
                 if (MX && d.prep_split) k_prepare_lc<true><<<grid_lc, blk, 0, st>>>(g, f, lc);
                 else if (MX) k_prepare_lc<false><<<grid_lc, blk, 0, st>>>(g, f, lc);
+                else if (d.rows64) k_prepare_lw<<<grid_lc, blk, 0, st>>>(g, f, lc);
                 else if (ml && d.prep64) k_prepare_lc64<<<grid_lc, blk, 0, st>>>(g, f, lc);
                 else if (ml) k_prepare_ml<2><<<grid_ml(2), blk, 0, st>>>(g, f);
                 else k_prepare<MX><<<grid_t2, blk, 0, st>>>(g, f);
@@ -596,14 +602,22 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             const dim3 grid_th((d.P + d.tcb - 1) / d.tcb);
             // segment kernel: rows of (nv - 1 + NROW - 1) / NROW interfaces
             const int seg16 = (d.nv - 1 + 15) / 16, seg32 = (d.nv - 1 + 7) / 8;
-            // mixed: 16 or 32 columns (rows chained); FP64: 16 columns (one-lane sweeps)
-            const int cbs = MX ? d.tseg : d.tseg64;
+            // mixed: 16 or 32 columns (rows chained); FP64: 16 columns (rows chained, or one-lane sweeps)
+            const bool rows64 = !MX && d.rows64;
+            const int cbs = MX ? d.tseg : rows64 ? 16 : d.tseg64;
             const bool tseg = d.nv > 1 && (MX ? d.f.thomas_rows && (cbs == 16 ? seg16 <= 4 : cbs == 32 && seg32 <= 8)
                                               : cbs == 16 && seg16 <= 4);
             const size_t lds_seg = ((size_t)(d.nv + 1) * cbs + 2 * 256) * sizeof(double);
             auto seg_solve = [&](auto dp) {
                 constexpr bool DP = decltype(dp)::value;
                 const dim3 gs((d.P + cbs - 1) / cbs);
+                if constexpr (!MX) {
+                    if (rows64) {
+                        if (seg16 <= 3) k_thomas_dp_seg<16, 3, DP, false, true><<<gs, 256, lds_seg, st>>>(g, f, times);
+                        else k_thomas_dp_seg<16, 4, DP, false, true><<<gs, 256, lds_seg, st>>>(g, f, times);
+                        return;
+                    }
+                }
                 if (cbs == 16 && seg16 <= 3) k_thomas_dp_seg<16, 3, DP, MX><<<gs, 256, lds_seg, st>>>(g, f, times);
                 else if (cbs == 16) k_thomas_dp_seg<16, 4, DP, MX><<<gs, 256, lds_seg, st>>>(g, f, times);
                 else if (seg32 <= 6) k_thomas_dp_seg<32, 6, DP, MX><<<gs, 256, lds_seg, st>>>(g, f, times);
@@ -629,8 +643,11 @@ template <bool MX> static int thor_step_t(Dyn &d) {
                 const thor_step_view v = view(f);
                 if (d.hooks.dyn_core_loop_fast_modes(d.hooks.user, (void *)st, nstep, times, &v))
                     return hook_fail("dyn_core_loop_fast_modes");
-                launch(d, "density_pressure", W(18, 4),
-                       [&] { k_dp<MX><<<dim3((d.P + kTile - 1) / kTile, d.nv), blk, 0, st>>>(g, f, times); });
+                launch(d, "density_pressure", W(18, 4), [&] {
+                    const dim3 gd((d.P + kTile - 1) / kTile, d.nv);
+                    if (rows64) k_dp<MX, true><<<gd, blk, 0, st>>>(g, f, times);
+                    else k_dp<MX, MX><<<gd, blk, 0, st>>>(g, f, times);
+                });
             }
             // next substep's divergence-damping pass 0
             if (next) divm0();
@@ -1141,6 +1158,10 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
     for (const char *k : {"THOR_SLOW_CHUNKED", "THOR_FP64_MULTILEVEL", "THOR_ML_LEVELS", "THOR_PREPARE_LC64",
                           "THOR_DIFF2_SPLIT64"})
         if (std::getenv(k)) d.lw = false;
+    // rows of up to four interfaces in the vertical solve, the entropy equation (the energy equation's branch
+    // spills at five waves per SIMD); its other kernels by their switches
+    d.rows64 = d.lw && d.slow_lc64 && !g.energy && (nv - 1 + 15) / 16 <= 4 && !std::getenv("THOR_THOMAS_SEG64")
+               && !std::getenv("THOR_THOMAS_COLUMNS");
 #endif
     if (const char *e = std::getenv("THOR_FP64_MULTILEVEL")) d.fp64_ml = std::atoi(e) != 0;
     if (const char *e = std::getenv("THOR_ML_LEVELS")) {
@@ -1186,7 +1207,7 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
     A(&f.SlowMh, n3); A(&f.SlowWh, ni); A(&f.SlowRho, n1); A(&f.Slowp, n1);
     A(&f.Sp, n1); A(&f.Sd, n1); A(&f.hflx_r, n1); A(&f.hflx_pt, n1); A(&f.tAA, n1); A(&f.tCC, n1); A(&f.tTT, n1);
     A(&f.Qheat, n1); A(&f.dMh, n3); A(&f.dWh, ni);
-    if (d.mixed) A(&f.hflx_ptk, n1);
+    if (d.mixed || d.rows64) A(&f.hflx_ptk, n1);
     if (g.energy) A(&f.Etot, n1);
     const bool diff_mid = prm->HyDiff && prm->HyDiffOrder >= 6;  // intermediate passes alternate two arrays
     if (diff_mid && !d.mixed) A(&f.diffx, 6 * n1);
