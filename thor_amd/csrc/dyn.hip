@@ -7,6 +7,7 @@
 #include "dyn_kernels.h"
 #include "dyn_kernels_lw.h"
 #include "dyn_kernels_ml.h"
+#include "dyn_kernels_solve.h"
 #include "mlp_internal.h"
 #include "tracer_kernels.h"
 
@@ -125,7 +126,7 @@ struct Dyn {
     bool prep64 = true;    // FP64 path: level-chunked prepare k_prepare_lc64 (false: k_prepare_ml; 107.7 -> 63.6 us
                            // at g6 L48; at three blocks per CU it spills, 95 us)
     int tur = 2;           // unroll of the level loops of the fused Thomas kernel (1 or 2; 64 columns)
-    int tseg = 16;         // mixed path: columns per block of the segment Thomas kernel (16 or 32; 0: off)
+    int tseg = 16;         // mixed path: 16: k_solve; 32: the segment Thomas kernel of 32 columns; 0: neither
     bool fseg = true;      // mixed path: segment form of the stage's Thomas factorisation
     int tseg64 = 0;        // FP64 path: segment Thomas kernel, 16 columns per block (0: the 64-column kernel;
                            // the segment form is bit for bit the same but slower: its one-lane sweeps run
@@ -602,26 +603,28 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             const dim3 grid_th((d.P + d.tcb - 1) / d.tcb);
             // segment kernel: rows of (nv - 1 + NROW - 1) / NROW interfaces
             const int seg16 = (d.nv - 1 + 15) / 16, seg32 = (d.nv - 1 + 7) / 8;
-            // mixed: 16 or 32 columns (rows chained); FP64: 16 columns (rows chained, or one-lane sweeps)
-            const bool rows64 = !MX && d.rows64;
-            const int cbs = MX ? d.tseg : rows64 ? 16 : d.tseg64;
-            const bool tseg = d.nv > 1 && (MX ? d.f.thomas_rows && (cbs == 16 ? seg16 <= 4 : cbs == 32 && seg32 <= 8)
-                                              : cbs == 16 && seg16 <= 4);
+            // up to 65 levels: k_solve (mixed, FP64 of the production build)
+            const bool solve = d.nv > 1 && seg16 <= 4 && (MX ? d.f.thomas_rows && d.tseg == 16 : d.rows64);
+            // else mixed: 32 columns (rows chained); FP64: 16 columns (one-lane sweeps)
+            const int cbs = MX ? d.tseg : d.tseg64;
+            const bool tseg = solve
+                              || (d.nv > 1 && (MX ? d.f.thomas_rows && cbs == 32 && seg32 <= 8 : cbs == 16 && seg16 <= 4));
             const size_t lds_seg = ((size_t)(d.nv + 1) * cbs + 2 * 256) * sizeof(double);
             auto seg_solve = [&](auto dp) {
                 constexpr bool DP = decltype(dp)::value;
-                const dim3 gs((d.P + cbs - 1) / cbs);
-                if constexpr (!MX) {
-                    if (rows64) {
-                        if (seg16 <= 3) k_thomas_dp_seg<16, 3, DP, false, true><<<gs, 256, lds_seg, st>>>(g, f, times);
-                        else k_thomas_dp_seg<16, 4, DP, false, true><<<gs, 256, lds_seg, st>>>(g, f, times);
-                        return;
-                    }
+                const dim3 gs((d.P + (solve ? 16 : cbs) - 1) / (solve ? 16 : cbs));
+                if (solve) {
+                    if (seg16 <= 1) k_solve<1, DP, MX><<<gs, 256, 0, st>>>(g, f, times);
+                    else if (seg16 == 2) k_solve<2, DP, MX><<<gs, 256, 0, st>>>(g, f, times);
+                    else if (seg16 == 3) k_solve<3, DP, MX><<<gs, 256, 0, st>>>(g, f, times);
+                    else k_solve<4, DP, MX><<<gs, 256, 0, st>>>(g, f, times);
+                } else if constexpr (MX) {
+                    if (seg32 <= 6) k_thomas_dp_seg<32, 6, DP, MX><<<gs, 256, lds_seg, st>>>(g, f, times);
+                    else k_thomas_dp_seg<32, 8, DP, MX><<<gs, 256, lds_seg, st>>>(g, f, times);
+                } else {
+                    if (seg16 <= 3) k_thomas_dp_seg<16, 3, DP, MX><<<gs, 256, lds_seg, st>>>(g, f, times);
+                    else k_thomas_dp_seg<16, 4, DP, MX><<<gs, 256, lds_seg, st>>>(g, f, times);
                 }
-                if (cbs == 16 && seg16 <= 3) k_thomas_dp_seg<16, 3, DP, MX><<<gs, 256, lds_seg, st>>>(g, f, times);
-                else if (cbs == 16) k_thomas_dp_seg<16, 4, DP, MX><<<gs, 256, lds_seg, st>>>(g, f, times);
-                else if (seg32 <= 6) k_thomas_dp_seg<32, 6, DP, MX><<<gs, 256, lds_seg, st>>>(g, f, times);
-                else k_thomas_dp_seg<32, 8, DP, MX><<<gs, 256, lds_seg, st>>>(g, f, times);
             };
             if (!d.hooks.dyn_core_loop_fast_modes && tseg) {
                 launch(d, "thomas_dp", W(12 + 18, 4), [&] { seg_solve(std::true_type{}); });
@@ -645,8 +648,8 @@ template <bool MX> static int thor_step_t(Dyn &d) {
                     return hook_fail("dyn_core_loop_fast_modes");
                 launch(d, "density_pressure", W(18, 4), [&] {
                     const dim3 gd((d.P + kTile - 1) / kTile, d.nv);
-                    if (rows64) k_dp<MX, true><<<gd, blk, 0, st>>>(g, f, times);
-                    else k_dp<MX, MX><<<gd, blk, 0, st>>>(g, f, times);
+                    if (solve) k_dp_solve<MX><<<gd, blk, 0, st>>>(g, f, times);
+                    else k_dp<MX><<<gd, blk, 0, st>>>(g, f, times);
                 });
             }
             // next substep's divergence-damping pass 0
@@ -1232,6 +1235,14 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
             k_slow_levels<<<(nv + 63) / 64, 64, 0, d.stream>>>(g, slv);
             e = hipGetLastError();
             g.slv = slv;
+        }
+        // and of the vertical solve (nv <= 127)
+        double *tlv = nullptr;
+        if (e == hipSuccess) e = dalloc(d, &tlv, (size_t)6 * (nv + 1));
+        if (e == hipSuccess) {
+            k_solve_levels<<<1, 128, 0, d.stream>>>(g, tlv);
+            e = hipGetLastError();
+            g.tlv = tlv;
         }
         if (e != hipSuccess)
             return cleanup_fail(fail(THOR_ERR_HIP, std::string("thor_dyn_create: level table: ") + hipGetErrorString(e)));

@@ -3434,9 +3434,7 @@ __global__ __launch_bounds__(256) void k_thomas_factor_seg(Geo g, Fields f, doub
 // (whs(k) = Whs at interface k).
 // rhos, pss, slowrho: Rhos, ps and SlowRho of the cell, read by the caller
 // (the segment kernel keeps them from its right-hand-side phase).
-// FAST: the update with one power (below), in the mixed form and the FP64 form
-// of the production build (entropy equation only).
-template <bool MX, bool FAST, class GetW>
+template <bool MX, class GetW>
 __device__ __forceinline__ void dp_column_in(const Geo &g, const Fields &f, int p, int lev, bool pole, double dt,
                                              double nflxr, double nflxpt, GetW whs, double rhos, double pss,
                                              double slowrho) {
@@ -3479,7 +3477,7 @@ __device__ __forceinline__ void dp_column_in(const Geo &g, const Fields &f, int 
     const double rhosn = rhos + (slowrho - nflxr) * dt;
     LV(f.Rhos, lev) = rhosn;
     double psn;
-    if constexpr (!MX && !FAST) {
+    if constexpr (!MX) {
         if (g.energy) {
             // total energy (thor_fastmodes.h:501-533): advance it, then the
             // pressure from it less the potential and kinetic energy of the
@@ -3503,7 +3501,7 @@ __device__ __forceinline__ void dp_column_in(const Geo &g, const Fields &f, int 
             return;
         }
     }
-    if constexpr (FAST) {
+    if constexpr (MX) {
         // The same update with one power. With pf = pss + pkv, q = (pf / P_Ref)^(Cv/Cp)
         // and x = -Rd (nflxpt + dwptdz) dt / (P_Ref q): Rd aux / P_Ref = q (1 + x),
         // so pnew = pf (1 + x)^(Cp/Cv) and pnew - pkv = pss + pf ((1 + x)^(Cp/Cv) - 1),
@@ -3536,11 +3534,11 @@ __device__ __forceinline__ void dp_column_in(const Geo &g, const Fields &f, int 
     if (isnan(psn)) atomicOr(f.flags, FLAG_NAN_P);
 }
 
-template <bool MX, bool FAST, class GetW>
+template <bool MX, class GetW>
 __device__ __forceinline__ void dp_column(const Geo &g, const Fields &f, int p, int lev, bool pole, double dt,
                                           double nflxr, double nflxpt, GetW whs) {
     const size_t S = g.S;
-    dp_column_in<MX, FAST>(g, f, p, lev, pole, dt, nflxr, nflxpt, whs, LV(f.Rhos, lev), LV(f.ps, lev),
+    dp_column_in<MX>(g, f, p, lev, pole, dt, nflxr, nflxpt, whs, LV(f.Rhos, lev), LV(f.ps, lev),
                      LV(f.SlowRho, lev));
 }
 
@@ -3761,7 +3759,7 @@ __global__ __launch_bounds__(256) void k_thomas_dp(Geo g, Fields f, double delta
     const bool pole = p >= g.P - 2;
 #pragma unroll UR
     for (int lev = row; lev < nv; lev += NROW)
-        dp_column<MX, MX>(g, f, p, lev, pole, deltat, LV(f.hflx_r, lev), LV(f.hflx_pt, lev),
+        dp_column<MX>(g, f, p, lev, pole, deltat, LV(f.hflx_r, lev), LV(f.hflx_pt, lev),
                       [&](int k) { return sD[k * CB + c]; });
 }
 
@@ -3779,15 +3777,10 @@ __global__ __launch_bounds__(256) void k_thomas_dp(Geo g, Fields f, double delta
 // equals k_thomas_dp<.., false> bit for bit.
 // SEG: interfaces per row at most; the host launches it with
 // (nv - 1 + NROW - 1) / NROW <= SEG. DP = false: the vertical solve alone
-// (Whs written; k_dp applies the update after a physics hook). Up to three
-// interfaces per row at 16 columns: five waves per SIMD (96 VGPRs, no spills;
-// 79 against 83 us at g6 L48 with four, and six spill); longer rows spill at
-// five and keep the compiler's choice. ROWS: both sweeps on all rows and the
-// one-power update (the mixed form, and the FP64 form of the production build:
-// 96 -> 79 us there, 26 -> 23 at 10 242 x 40); without it, the reference's order.
-template <int CB, int SEG, bool DP = true, bool MX = true, bool ROWS = MX>
-__global__ __launch_bounds__(256, (ROWS && CB == 16 && SEG <= 3) ? 5 : 1) void k_thomas_dp_seg(Geo g, Fields f,
-                                                                                               double deltat) {
+// (Whs written; k_dp applies the update after a physics hook). Up to 65 levels
+// both forms of the production build take k_solve instead.
+template <int CB, int SEG, bool DP = true, bool MX = true>
+__global__ __launch_bounds__(256) void k_thomas_dp_seg(Geo g, Fields f, double deltat) {
     constexpr int NROW = 256 / CB;
     extern __shared__ double sm[];
     double *sD = sm;
@@ -3813,15 +3806,15 @@ __global__ __launch_bounds__(256, (ROWS && CB == 16 && SEG <= 3) ? 5 : 1) void k
         cS[i] = in ? LV(f.SlowRho, lev) : 0.0;
         cF[i] = in ? LV(f.hflx_r, lev) : 0.0;
         cSp[i] = in ? LV(f.Sp, lev) : 0.0;
-        if constexpr (!ROWS) cD[i] = in ? LV(f.Sd, lev) : 0.0;  // written by k_prepare_lc64
+        if constexpr (!MX) cD[i] = in ? LV(f.Sd, lev) : 0.0;  // written by k_prepare_lc64
     }
 #pragma unroll
     for (int i = 1; i <= SEG; i++) {
         const int lev = lo - 1 + i;  // interface
         if (valid && i < ncell) {
             const double alth = Alth[lev], alt = Alt[lev], altl = Alt[lev - 1];
-            const double Sp = cSp[i], Sd = ROWS ? -cF[i] + cS[i] : cD[i], pr = cP[i], r = cR[i];
-            const double Spl = cSp[i - 1], Sdl = ROWS ? -cF[i - 1] + cS[i - 1] : cD[i - 1], pl = cP[i - 1],
+            const double Sp = cSp[i], Sd = MX ? -cF[i] + cS[i] : cD[i], pr = cP[i], r = cR[i];
+            const double Spl = cSp[i - 1], Sdl = MX ? -cF[i - 1] + cS[i - 1] : cD[i - 1], pl = cP[i - 1],
                          rl = cR[i - 1];
             const double dzh = 1.0 / (alt - altl);
             const double CRdd = (CRdd_c * (alt - alth) + CRdd_c * (alth - altl)) / (alt - altl);
@@ -3856,7 +3849,7 @@ __global__ __launch_bounds__(256, (ROWS && CB == 16 && SEG <= 3) ? 5 : 1) void k
     }
     __syncthreads();
     const Plane AA{f.tAA, S, p}, CC{f.tCC, S, p}, TT{f.tTT, S, p};
-    if constexpr (ROWS) {
+    if constexpr (MX) {
         thomas_sweeps_rows<CB, SEG>(sD, sm + (size_t)(nv + 1) * CB, AA, CC, TT, nv, c, row, valid);
     } else if (row == 0 && valid) {
         // one lane per column: forward elimination and back substitution in
@@ -3893,18 +3886,18 @@ __global__ __launch_bounds__(256, (ROWS && CB == 16 && SEG <= 3) ? 5 : 1) void k
     for (int i = 0; i < SEG + 1; i++) {
         const int lev = lo - 1 + i;
         if (i < nlast)
-            dp_column_in<MX, ROWS>(g, f, p, lev, pole, deltat, cF[i], LV(f.hflx_pt, lev),
+            dp_column_in<MX>(g, f, p, lev, pole, deltat, cF[i], LV(f.hflx_pt, lev),
                                [&](int k) { return sD[k * CB + c]; }, cR[i], cP[i], cS[i]);
     }
 }
 
 // Column part of Density_Pressure_Eqs after a separate vertical solve
 // (k_thomas_dp<.., false>): one thread per (point, level), Whs from HBM.
-template <bool MX, bool FAST> __global__ __launch_bounds__(256) void k_dp(Geo g, Fields f, double deltat) {
+template <bool MX> __global__ __launch_bounds__(256) void k_dp(Geo g, Fields f, double deltat) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x, lev = blockIdx.y;
     if (p >= g.P) return;
     const size_t S = g.S;
-    dp_column<MX, FAST>(g, f, p, lev, p >= g.P - 2, deltat, LV(f.hflx_r, lev), LV(f.hflx_pt, lev),
+    dp_column<MX>(g, f, p, lev, p >= g.P - 2, deltat, LV(f.hflx_r, lev), LV(f.hflx_pt, lev),
                   [&](int k) { return LVP(f.Whs, k, p); });
 }
 
