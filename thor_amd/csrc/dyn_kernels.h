@@ -27,8 +27,12 @@ namespace thor {
 #ifndef THOR_SLOT_UNROLL
 #define THOR_SLOT_UNROLL 1
 #endif
-#define PRAGMA_STR(x) _Pragma(#x)
-#define SLOT_UNROLL(n) PRAGMA_STR(unroll n)
+// The two poles gather their slots from global memory: with the sums unrolled
+// (kPoleUnroll) all loads of a pole are in flight at once. Rolled, each of the
+// 20 to 60 terms waited for its own load, and the pole block was the last to
+// finish on small grids (us per launch at 2 562 x 20 and 10 242 x 40, mixed: advection
+// 20.2 -> 8.8 and 28 -> 18.7, prepare 9.2 -> 5.4 and 12.4 -> 9.8).
+constexpr int kPoleUnroll = 8;
 
 // pow inside the dynamical-core step (the equation of state in the column
 // preparation and the density/pressure update, r^2 and r^3 of the deep
@@ -841,7 +845,7 @@ __global__ __launch_bounds__(256) void k_energy_prep(Geo g, Fields f) {
 // added to the vertical part, and the first Laplacian pass of the 4th-order
 // hyperdiffusion (Diffusion_Op stepnum 0, thor_diff.h:54-522) of rho, u, v,
 // w = M/rho, W/rho and Rd*T.
-template <bool MX, class GetM, class GetV, class GetR, class GetW, class GetT>
+template <bool MX, int U = THOR_SLOT_UNROLL, class GetM, class GetV, class GetR, class GetW, class GetT>
 __device__ __forceinline__ void adv_diff1_point(const Geo &g, const Fields &f, int p, int lev, int nf, int hydiff,
                                                 GetM M, GetV v, GetR rho, GetW W, GetT T) {
     const size_t S = g.S;
@@ -853,7 +857,7 @@ __device__ __forceinline__ void adv_diff1_point(const Geo &g, const Fields &f, i
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             double sum = g.div[(size_t)(0 * 3 + kk) * S + p] * v(0, c) * M(0, kk);
-SLOT_UNROLL(THOR_SLOT_UNROLL)
+#pragma unroll U
             for (int s = 1; s < 7; s++) sum = sum + g.div[(size_t)(s * 3 + kk) * S + p] * v(s, c) * M(s, kk);
             nf3[c] += rs * sum;
         }
@@ -1222,10 +1226,13 @@ template <bool MX>
 __device__ __forceinline__ void slow_tail(const Geo &g, const Fields &f, int p, int lev, bool pole, int rk,
                                           const double DivM[3], const double nflxv_in[3], double nflxr, double nflxp,
                                           double pv0, double M0x, double M0y, double M0z);
+// slow_sums: the operator sums from the stencil values, then the tail.
+template <bool MX, int U = THOR_SLOT_UNROLL, class GetP, class GetH, class GetM>
+__device__ __forceinline__ void slow_sums(const Geo &g, const Fields &f, int p, int lev, bool pole, int rk,
+                                          const double DivM[3], GetP pv, GetH hv, GetM mv);
 template <bool MX, class GetG, class GetP, class GetH, class GetM>
 __device__ __forceinline__ void slow_point(const Geo &g, const Fields &f, int p, int lev, int nf, bool pole,
                                            int divdamp, int rk, GetG dg, GetP pv, GetH hv, GetM mv) {
-    const size_t S = g.S;
     double DivM[3] = {0.0, 0.0, 0.0};
     if (divdamp) {
         if constexpr (MX) {
@@ -1237,6 +1244,13 @@ __device__ __forceinline__ void slow_point(const Geo &g, const Fields &f, int p,
             divm_nf<true>(g, p, lev, nf, pole, dg, none, none, DivM);
         }
     }
+    slow_sums<MX>(g, f, p, lev, pole, rk, DivM, pv, hv, mv);
+}
+
+template <bool MX, int U, class GetP, class GetH, class GetM>
+__device__ __forceinline__ void slow_sums(const Geo &g, const Fields &f, int p, int lev, bool pole, int rk,
+                                          const double DivM[3], GetP pv, GetH hv, GetM mv) {
+    const size_t S = g.S;
     const double rscale = rscale_at(g, lev);
     double nflxv[3], nflxr = 0.0, nflxp = 0.0;
 #pragma unroll
@@ -1244,7 +1258,7 @@ __device__ __forceinline__ void slow_point(const Geo &g, const Fields &f, int p,
         double sg = g.grad[(size_t)(0 * 3 + k) * S + p] * pv(0);
         double sr = g.div[(size_t)(0 * 3 + k) * S + p] * mv(0, k);
         double sp = g.div[(size_t)(0 * 3 + k) * S + p] * mv(0, k) * hv(0);
-SLOT_UNROLL(THOR_SLOT_UNROLL)
+#pragma unroll U
         for (int s = 1; s < 7; s++) {
             const double gd = g.grad[(size_t)(s * 3 + k) * S + p], dd = g.div[(size_t)(s * 3 + k) * S + p];
             sg = sg + gd * pv(s);
@@ -1268,7 +1282,21 @@ __device__ __forceinline__ void slow_tail(const Geo &g, const Fields &f, int p, 
     const double fx = g.fr[p], fy = g.fr[S + p], fz = g.fr[2 * S + p];
     const double *Alt = g.Alt, *Alth = g.Alth;
     const double nflxv[3] = {nflxv_in[0], nflxv_in[1], nflxv_in[2]};
+    // everything the cell reads, before its first store
     const auto *Adv = FS<MX>::Adv(f);
+    const auto *diffmh = FS<MX>::diffmh(f), *diffw = FS<MX>::diffw(f);
+    double v_dmh[3], v_dmv[3], v_dM[3], v_y[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        v_dmh[k] = VEC(diffmh, k, lev, p);
+        v_dmv[k] = f.diffmv ? VEC(f.diffmv, k, lev, p) : 0.0;
+        v_dM[k] = VEC(f.dMh, k, lev, p);
+        if (rk) v_y[k] = VEC(f.Mh, k, lev, p);
+    }
+    const double v_dw = LV(diffw, lev), v_dwl = lev ? (double)LV(diffw, lev - 1) : 0.0, v_dWh = LV(f.dWh, lev),
+                 v_drh = LV(FS<MX>::diffrh(f), lev), v_dpr = LV(FS<MX>::diffpr(f), lev), v_gtil = LV(f.gtil, lev),
+                 v_q = LV(f.Qheat, lev), v_rho = rk ? LV(f.Rho, lev) : 0.0, v_p = rk ? LV(f.p, lev) : 0.0,
+                 v_wh = rk ? LV(f.Wh, lev) : 0.0, v_whk = LV(f.Whk, lev);
     double advx = VEC(Adv, 0, lev, p), advy = VEC(Adv, 1, lev, p), advz = VEC(Adv, 2, lev, p);
     const double rho = LV(f.Rhok, lev);
     double advrl = 0, rhol = 0, altl = 0, pressurel = 0;
@@ -1320,11 +1348,9 @@ __device__ __forceinline__ void slow_tail(const Geo &g, const Fields &f, int p, 
     const double dpr = nflxv[0] * fx + nflxv[1] * fy + nflxv[2] * fz;
     const double fv[3] = {fx, fy, fz}, ad[3] = {advx, advy, advz};
     auto *SlowMh = FS<MX>::SlowMh(f);
-    const auto *diffmh = FS<MX>::diffmh(f);
 #pragma unroll
     for (int k = 0; k < 3; k++)
-        VEC(SlowMh, k, lev, p) = -(nflxv[k] - dpr * fv[k]) - ad[k] + DivM[k] + VEC(diffmh, k, lev, p)
-                                 + (f.diffmv ? VEC(f.diffmv, k, lev, p) : 0.0) + VEC(f.dMh, k, lev, p);
+        VEC(SlowMh, k, lev, p) = -(nflxv[k] - dpr * fv[k]) - ad[k] + DivM[k] + v_dmh[k] + v_dmv[k] + v_dM[k];
     if (lev == 0) {
         LV(f.SlowWh, 0) = 0.0;
         LV(f.SlowWh, nv) = 0.0;
@@ -1344,22 +1370,21 @@ __device__ __forceinline__ void slow_tail(const Geo &g, const Fields &f, int p, 
             else
                 swr = (rhol * Gravit) * intt + (rho * Gravit) * intl;
         }
-        const auto *diffw = FS<MX>::diffw(f);
-        if (g.nonhydro) swr += (-LV(diffw, lev - 1) - 0.0) * intt + (-LV(diffw, lev) - 0.0) * intl;
+        if (g.nonhydro) swr += (-v_dwl - 0.0) * intt + (-v_dw - 0.0) * intl;
         const double dzl = alt - altl;
         const double dpdz = (pv0 - pressurel) / dzl;
         swr += dpdz;
-        swr -= LV(f.dWh, lev);
+        swr -= v_dWh;
         LV(f.SlowWh, lev) = -swr;
     }
     nflxr += dwdz;
-    LV(f.SlowRho, lev) = -nflxr + LV(FS<MX>::diffrh(f), lev) + 0.0;
+    LV(f.SlowRho, lev) = -nflxr + v_drh + 0.0;
     const double r = 1.0 / rho;
     const double vgp =
         (nflxv[0] - dpr * fx) * M0x * r + (nflxv[1] - dpr * fy) * M0y * r + (nflxv[2] - dpr * fz) * M0z * r;
-    double sp = (Rd / Cv) * (-nflxp - LV(f.gtil, lev) - dwhdz + vgp + LV(f.Qheat, lev));
-    if (g.energy) sp += Rd / Cv * (LV(FS<MX>::diffpr(f), lev) + 0.0);  // thor_slowmodes.h:375-377
-    else sp += LV(FS<MX>::diffpr(f), lev) + 0.0;
+    double sp = (Rd / Cv) * (-nflxp - v_gtil - dwhdz + vgp + v_q);
+    if (g.energy) sp += Rd / Cv * (v_dpr + 0.0);  // thor_slowmodes.h:375-377
+    else sp += v_dpr + 0.0;
     LV(f.Slowp, lev) = sp;
 
     // Deviations at the start of the stage.
@@ -1372,14 +1397,14 @@ __device__ __forceinline__ void slow_tail(const Geo &g, const Fields &f, int p, 
         LV(f.Whs, lev) = 0.0;
         if (lev == nv - 1) LV(f.Whs, nv) = 0.0;
     } else {
-        const double Mx = VEC(f.Mh, 0, lev, p) - M0x, My = VEC(f.Mh, 1, lev, p) - M0y, Mz = VEC(f.Mh, 2, lev, p) - M0z;
+        const double Mx = v_y[0] - M0x, My = v_y[1] - M0y, Mz = v_y[2] - M0z;
         const double aux = Mx * fx + My * fy + Mz * fz;
         VEC(Mhs, 0, lev, p) = Mx - aux * fx;
         VEC(Mhs, 1, lev, p) = My - aux * fy;
         VEC(Mhs, 2, lev, p) = Mz - aux * fz;
-        LV(f.Rhos, lev) = LV(f.Rho, lev) - rho;
-        LV(f.ps, lev) = LV(f.p, lev) - pv0;
-        LV(f.Whs, lev) = lev == 0 ? 0.0 : LV(f.Wh, lev) - LV(f.Whk, lev);
+        LV(f.Rhos, lev) = v_rho - rho;
+        LV(f.ps, lev) = v_p - pv0;
+        LV(f.Whs, lev) = lev == 0 ? 0.0 : v_wh - v_whk;
         if (lev == nv - 1) LV(f.Whs, nv) = 0.0;
     }
 }
@@ -1483,7 +1508,7 @@ template <bool MX> __global__ STENCIL_BOUNDS void k_divm0(Geo g, Fields f) {
 template <bool MX>
 __device__ __forceinline__ void momentum_tail(const Geo &g, const Fields &f, int p, int lev, const double nf3[3],
                                               const double DivM[3], double dt);
-template <bool MX, class GetG, class GetS>
+template <bool MX, int U = THOR_SLOT_UNROLL, class GetG, class GetS>
 __device__ __forceinline__ void momentum_point(const Geo &g, const Fields &f, int p, int lev, int nf, bool pole,
                                                int divdamp, double dt, GetG dg, GetS pv) {
     const size_t S = g.S;
@@ -1503,7 +1528,7 @@ __device__ __forceinline__ void momentum_point(const Geo &g, const Fields &f, in
 #pragma unroll
     for (int k = 0; k < 3; k++) {
         double s0 = g.grad[(size_t)(0 * 3 + k) * S + p] * pv(0);
-SLOT_UNROLL(THOR_SLOT_UNROLL)
+#pragma unroll U
         for (int s = 1; s < 7; s++) s0 = s0 + g.grad[(size_t)(s * 3 + k) * S + p] * pv(s);
         nf3[k] = rs * s0;
     }
@@ -1617,11 +1642,11 @@ __device__ __forceinline__ void prepare_point_w(const Geo &g, const Fields &f, i
     LV(f.hflx_pt, lev) = SPLIT ? dpt + dptk : dpt;
 }
 
-template <class GetM, class GetH, class GetV1, class GetPt>
+template <int U = THOR_SLOT_UNROLL, class GetM, class GetH, class GetV1, class GetPt>
 __device__ __forceinline__ void prepare_point(const Geo &g, const Fields &f, int p, int lev, GetM mv, GetH hv,
                                               GetV1 v1, GetPt ptv) {
     const size_t S = g.S;
-    prepare_point_w<THOR_SLOT_UNROLL>(
+    prepare_point_w<U>(
         g, f, p, lev, [&](int s, int k) { return g.div[(size_t)(s * 3 + k) * S + p]; }, mv, hv, v1, ptv,
         LV(f.Slowp, lev), LV(f.SlowRho, lev), rscale_at(g, lev));
 }
@@ -1776,7 +1801,7 @@ __global__ __launch_bounds__(256, 3) void k_momentum_lc(Geo g, Fields f, int div
         PoleCtx c;
         int lev;
         if (pole_ctx_lc(g, l0, l1, c, lev))
-            momentum_point<true>(
+            momentum_point<true, kPoleUnroll>(
                 g, f, c.p, lev, 5, true, divdamp, dt, [&](int s, int k) { return VEC(divg, k, lev, c.gi(s)); },
                 [&](int s) { return LVP(f.ps, lev, c.gi(s)); });
         return;
@@ -1902,7 +1927,7 @@ __global__ __launch_bounds__(256, SPLIT ? THOR_PREP_LC_MINB : 2) void k_prepare_
         PoleCtx c;
         int lev;
         if (pole_ctx_lc(g, l0, l1, c, lev))
-            prepare_point(
+            prepare_point<kPoleUnroll>(
                 g, f, c.p, lev, [&](int s, int k) { return (double)VEC(Mhs, k, lev, c.gi(s)); },
                 [&](int s) { return LVP(f.h, lev, c.gi(s)); },
                 [&](int s, int k) { return (double)VEC(Mhs, k, lev, c.gi(s)) + VEC(f.Mhk, k, lev, c.gi(s)); },
@@ -2042,7 +2067,7 @@ __global__ __launch_bounds__(256, 2) void k_prepare_lc64(Geo g, Fields f, int lc
         PoleCtx c;
         int lev;
         if (pole_ctx_lc(g, l0, l1, c, lev))
-            prepare_point(
+            prepare_point<kPoleUnroll>(
                 g, f, c.p, lev, [&](int s, int k) { return VEC(Mhs, k, lev, c.gi(s)); },
                 [&](int s) { return LVP(f.h, lev, c.gi(s)); },
                 [&](int s, int k) { return VEC(Mhs, k, lev, c.gi(s)) + VEC(f.Mhk, k, lev, c.gi(s)); },
@@ -2360,13 +2385,23 @@ __global__ __launch_bounds__(256, THOR_DIVM0_LC_MINB) void k_divm0_lc(Geo g, Fie
 
 // Divergence-damping pass 1 of the slow part (the DivM term of
 // Compute_Slow_Modes, thor_slowmodes.h:82-105) in FP32 over level chunks, with
-// the operation order of divm_w<true>, written to dm [3][nv] for k_slow_lc.
-// Tiles only: the pole block of k_slow_lc forms its own DivM.
+// the operation order of divm_w<true>, written to dm [3][nv] for k_slow_lc and
+// k_slow_lc2.
 __global__ __launch_bounds__(256, 3) void k_divm1_lc(Geo g, Fields f, float *dm, int lc) {
     int r, l0, l1;
-    if (!block_tile_lc(g, lc, r, l0, l1) || r == g.nr) return;
+    if (!block_tile_lc(g, lc, r, l0, l1)) return;
     const size_t S = g.S;
     const int nv = g.nv;
+    if (r == g.nr) {
+        PoleCtx c;
+        int lev;
+        if (!pole_ctx_lc(g, l0, l1, c, lev)) return;
+        float o3[3];
+        divm_w<true>(g, c.p, lev, [&](int s, int k) { return VEC(f.mdivg, k, lev, c.gi(s)); }, [](int) { return 0.f; }, o3);
+#pragma unroll
+        for (int k = 0; k < 3; k++) VEC(dm, k, lev, c.p) = o3[k];
+        return;
+    }
     __shared__ float sG[2][3][NHL2], sL[4][kLcMax];
     stage_lvc(g, l0, l1, sL);
     const LcThread T = lc_thread(g, r);
@@ -2771,11 +2806,18 @@ __global__ __launch_bounds__(256, MX ? 2 : 1) void k_slow_lc2(Geo g, Fields f, c
         PoleCtx c;
         int lev;
         if (pole_ctx_lc(g, l0, l1, c, lev)) {
-            const auto *divg = FS<MX>::divg(f);
-            slow_point<MX>(
-                g, f, c.p, lev, 5, true, divdamp, rk, [&](int s, int k) { return VEC(divg, k, lev, c.gi(s)); },
-                [&](int s) { return LVP(f.pk, lev, c.gi(s)); }, [&](int s) { return LVP(f.h, lev, c.gi(s)); },
-                [&](int s, int k) { return VEC(f.Mhk, k, lev, c.gi(s)); });
+            double DivM[3] = {0.0, 0.0, 0.0};
+            if constexpr (MX || PTK) {  // dm holds the poles' DivM too
+                if (divdamp)
+                    for (int k = 0; k < 3; k++) DivM[k] = VEC(dm, k, lev, c.p);
+            } else if (divdamp) {
+                auto none = [&](int) { return 0.0; };
+                divm_nf<true>(g, c.p, lev, 5, true, [&](int s, int k) { return VEC(f.divg, k, lev, c.gi(s)); }, none,
+                              none, DivM);
+            }
+            slow_sums<MX, kPoleUnroll>(
+                g, f, c.p, lev, true, rk, DivM, [&](int s) { return LVP(f.pk, lev, c.gi(s)); },
+                [&](int s) { return LVP(f.h, lev, c.gi(s)); }, [&](int s, int k) { return VEC(f.Mhk, k, lev, c.gi(s)); });
         }
         return;
     }
@@ -3107,7 +3149,7 @@ __global__ __launch_bounds__(256, 3) void k_adv_diff1_lc(Geo g, Fields f, int hy
                 const double rho = LVP(f.Rhok, lev, q), w = LVP(f.Wk, lev, q);
                 return VEC(f.Mhk, k, lev, q) / rho + (w / rho) * g.fr[(size_t)k * S + q];
             };
-            adv_diff1_point<true>(
+            adv_diff1_point<true, kPoleUnroll>(
                 g, f, c.p, lev, 5, hydiff, [&](int s, int k) { return VEC(f.Mhk, k, lev, c.gi(s)); },
                 [&](int s, int k) { return vel(c.gi(s), k); }, [&](int s) { return LVP(f.Rhok, lev, c.gi(s)); },
                 [&](int s) { return LVP(f.Wk, lev, c.gi(s)); }, [&](int s) { return LVP(f.T, lev, c.gi(s)); });
@@ -3934,22 +3976,25 @@ __global__ __launch_bounds__(256) void k_update_rk2(Geo g, Fields f) {
         return (lev == 0 || lev == nv) ? 0.0 : LV(f.Whk, lev) + LV(f.Whs, lev);
     };
     const auto *Mhs = FS<MX>::Mhs(f);
+#pragma unroll 2
     for (int lev = l0; lev < l1; lev++) {
+        // every load before the first store
         const double Mx = VEC(Mhs, 0, lev, p) + VEC(f.Mhk, 0, lev, p);
         const double My = VEC(Mhs, 1, lev, p) + VEC(f.Mhk, 1, lev, p);
         const double Mz = VEC(Mhs, 2, lev, p) + VEC(f.Mhk, 2, lev, p);
+        const double rho = LV(f.Rhok, lev) + LV(f.Rhos, lev), pr = LV(f.pk, lev) + LV(f.ps, lev);
+        const double wl = whk_new(lev), wt = whk_new(lev + 1);
+        const double althl = lev == 0 ? 0 : g.Alth[lev];
+        const double altht = g.Alth[lev + 1];
+        const double xi = g.Alt[lev], xim = althl, xip = altht;
         const double aux = Mx * fx + My * fy + Mz * fz;
         VEC(f.Mhk_out, 0, lev, p) = Mx - aux * fx;
         VEC(f.Mhk_out, 1, lev, p) = My - aux * fy;
         VEC(f.Mhk_out, 2, lev, p) = Mz - aux * fz;
-        LV(f.Rhok_out, lev) = LV(f.Rhok, lev) + LV(f.Rhos, lev);
-        LV(f.pk_out, lev) = LV(f.pk, lev) + LV(f.ps, lev);
-        const double wl = whk_new(lev), wt = whk_new(lev + 1);
+        LV(f.Rhok_out, lev) = rho;
+        LV(f.pk_out, lev) = pr;
         LV(f.Whk_out, lev) = wl;
         if (lev == nv - 1) LV(f.Whk_out, nv) = wt;
-        const double althl = lev == 0 ? 0 : g.Alth[lev];
-        const double altht = g.Alth[lev + 1];
-        const double xi = g.Alt[lev], xim = althl, xip = altht;
         const double intt = (xi - xip) / (xim - xip), intl = (xi - xim) / (xip - xim);
         LV(f.Wk_out, lev) = wl * intt + wt * intl;
     }

@@ -112,6 +112,7 @@ __global__ __launch_bounds__(256, 2) void k_divm0_lw(Geo g, Fields f, int lc) {
         const int p = c.p;
         const double rs = rscale_at(g, lev), rs2 = rs * rs, rdz = rs / (g.Alth[lev] - g.Alth[lev + 1]);
         double o[3] = {0.0, 0.0, 0.0};
+#pragma unroll
         for (int s = 0; s < 7; s++) {
             const int q = c.gi(s);
             const double dw = (LVP(Wv, lev, q) - LVP(Wv, lev + 1, q)) * rdz;
@@ -208,6 +209,7 @@ __global__ __launch_bounds__(256, 2) void k_momentum_lw(Geo g, Fields f, int div
         double t[2];
         for (int e = 0; e < 2; e++) {
             double sg = 0.0, sd = 0.0, sm = 0.0;
+#pragma unroll
             for (int s = 0; s < 7; s++) {
                 const int q = c.gi(s);
                 sg += g.wgt64[(size_t)(e * 7 + s) * S + p] * LVP(f.ps, lev, q);
@@ -300,14 +302,31 @@ __global__ __launch_bounds__(256, 2) void k_momentum_lw(Geo g, Fields f, int div
 }
 
 // Divergence-damping pass 1 of the slow part (thor_slowmodes.h:82-105) into dm
-// [3][nv], for k_slow_lc2<false>. Tiles only: the pole block of the slow modes
-// forms its own.
+// [3][nv], for k_slow_lc2<false>.
 __global__ __launch_bounds__(256, 3) void k_divm1_lw(Geo g, Fields f, double *dm, int lc) {
 #pragma clang fp contract(fast)
     int r, l0, l1;
-    if (!block_tile_lc(g, lc, r, l0, l1) || r == g.nr) return;
+    if (!block_tile_lc(g, lc, r, l0, l1)) return;
     const size_t S = g.S;
     const int nv = g.nv;
+    if (r == g.nr) {
+        PoleCtx c;
+        int lev;
+        if (!pole_ctx_lc(g, l0, l1, c, lev)) return;
+        const double rs = rscale_at(g, lev), kz = -(rs * rs) * g.Kdhz[lev];
+        double t[2] = {0.0, 0.0};
+#pragma unroll
+        for (int s = 0; s < 7; s++)
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                const double a = VEC(f.divg, k, lev, c.gi(s));
+                t[0] += g.wdt64[(size_t)(s * 3 + k) * S + c.p] * a;
+                t[1] += g.wdt64[(size_t)(21 + s * 3 + k) * S + c.p] * a;
+            }
+        for (int k = 0; k < 3; k++)
+            VEC(dm, k, lev, c.p) = kz * (t[0] * g.et64[(size_t)k * S + c.p] + t[1] * g.et64[(size_t)(3 + k) * S + c.p]);
+        return;
+    }
     __shared__ double2 sA[2][NHL2];
     __shared__ double sB[2][NHL2], sKz[kLcMax];
     if ((int)threadIdx.x < l1 - l0) {
@@ -386,6 +405,7 @@ __global__ __launch_bounds__(256, 2) void k_adv_diff1_lw(Geo g, Fields f, int hy
         const int p = c.p;
         const double rs = rscale_at(g, lev);
         double adv[3] = {0.0, 0.0, 0.0}, lap[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, a0[6];
+#pragma unroll
         for (int s = 0; s < 7; s++) {
             const int q = c.gi(s);
             const double rho = LVP(f.Rhok, lev, q), wr = LVP(f.Wk, lev, q) / rho;
@@ -516,6 +536,7 @@ __global__ __launch_bounds__(256, 3) void k_diff_lw(Geo g, Fields f, const doubl
         const int p = c.p;
         const double rs = rscale_at(g, lev);
         double out[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, a0[6];
+#pragma unroll
         for (int s = 0; s < 7; s++) {
             const int q = c.gi(s);
             const double rho = LAST ? LVP(f.Rhok, lev, q) : 1.0;
@@ -638,7 +659,7 @@ __global__ __launch_bounds__(256, 2) void k_prepare_lw(Geo g, Fields f, int lc) 
         PoleCtx c;
         int lev;
         if (pole_ctx_lc(g, l0, l1, c, lev))
-            prepare_point(
+            prepare_point<kPoleUnroll>(
                 g, f, c.p, lev, [&](int s, int k) { return VEC(f.Mhs, k, lev, c.gi(s)); },
                 [&](int s) { return LVP(f.h, lev, c.gi(s)); },
                 [&](int s, int k) { return VEC(f.Mhs, k, lev, c.gi(s)) + VEC(f.Mhk, k, lev, c.gi(s)); },
