@@ -112,3 +112,84 @@ def test_row_solve_equals_the_one_lane_solve(built, nv, extra, precision):
         print(f"  {k}: {err:.2e}")
         assert err < (1e-9 if precision else 1e-12), k
         assert np.array_equal(a[k], c[k]), ("hook split", k)
+
+
+@pytest.mark.parametrize("precision,nv,extra", [
+    (0, 20, {}), (1, 20, {}), (0, 3, {}), (1, 33, dict(DeepModel=0, NonHydro=0, GravHeightVar=1)),
+    (0, 33, dict(DeepModel=0, NonHydro=0, GravHeightVar=1)), (1, 23, dict(DivDampP=0)), (0, 23, dict(HyDiff=0)),
+    (0, 21, dict(thermo_equation=1)), (0, 20, dict(VertHyDiff=1, VertHyDiffOrder=6, Diffc_v=2e-3)),
+])
+def test_slow_modes_equal_the_reference_order(built, precision, nv, extra):
+    """k_slow_w (weights in registers, constants from a table, the first stage's
+    momentum written with the slow tendencies) against the kernels in the
+    reference's order (THOR_SLOW_CHUNKED), one step with given forcing arrays.
+    FP64: sums of at most 21 products in another order, 1e-12 of the field's
+    scale. Mixed: the first stage's momentum is rounded to FP32 once instead of
+    twice, so 2^-24 of rho c_s in the momenta and what that moves, 1e-7."""
+    capi = built
+    print(f"case: precision {precision} g4 L{nv} {extra}: k_slow_w vs the reference order, 1 step", flush=True)
+    g = grid(capi, 4, nv)
+    p = earth_params(capi, 4, dt=600.0, ns=6, precision=precision, **extra)
+    st = capi.ic_rest(g, p, seed=2340 + nv, temperature_noise=1e-3, wind_noise=1.0)
+    rng = np.random.default_rng(nv)
+    tend = {"profx_Qheat": 1e-3 * rng.standard_normal((g.P, nv)), "profx_dMh": 1e-5 * rng.standard_normal((g.P, nv, 3)),
+            "profx_dWh": 1e-6 * rng.standard_normal((g.P, nv + 1))}
+    out = []
+    for env in ({}, {"THOR_SLOW_CHUNKED": "1"}):
+        for k, v in env.items():
+            os.environ[k] = v
+        try:
+            d = capi.Dyn(g, p)
+        finally:
+            for k in env:
+                os.environ.pop(k, None)
+        d.set_state(st)
+        for k, v in tend.items():
+            d.set_field(k, v)
+        d.thor()
+        d.sync()
+        out.append(d.get_state())
+        d.close()
+    a, b = out
+    cs = np.sqrt(p.Cp / (p.Cp - p.Rd) * p.Rd * p.Tmean)
+    for k in STATE:
+        scale = np.abs(b["Rho"]).max() * cs if k in ("Mh", "Wh", "W") else np.abs(b[k]).max()
+        err = np.abs(a[k] - b[k]).max() / scale
+        print(f"  {k}: {err:.2e}")
+        assert err < (1e-7 if precision else 1e-12), k
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_known_zero_tendencies_equal_zeros_read(built, precision):
+    """Arrays of forcing tendencies that are known to be zero are not read:
+    the same states as with zeros written to them, before and after a forcing
+    that fills them (double-gray heating), ProfX clearing them again."""
+    from common import hj_grid, hj_params, rt_params
+    capi = built
+    print(f"case: precision {precision} g4 L20: known zero tendencies", flush=True)
+    g, p = hj_grid(capi, 4, 20), hj_params(capi, 4, precision=precision)
+    st = capi.ic_rest(g, p, seed=2440, temperature_noise=1.0, wind_noise=1.0)
+    z = {"profx_Qheat": np.zeros((g.P, 20)), "profx_dMh": np.zeros((g.P, 20, 3)), "profx_dWh": np.zeros((g.P, 21))}
+    nr = capi.NewtonianParams(1600.0, 600.0, 0.0, 1e2, 1e7, 1e6, 1e4, 1e7)
+    out = []
+    for written in (False, True):
+        d = capi.Dyn(g, p)
+        d.set_newtonian(nr)
+        d.set_rt(rt_params(capi))
+        d.set_state(st)
+        res = []
+        for forcing in (capi.FORCING_NONE, capi.FORCING_NEWTONIAN, capi.FORCING_DOUBLE_GRAY, capi.FORCING_NEWTONIAN,
+                        capi.FORCING_NONE):
+            d.profx(forcing)
+            if written:
+                for k, v in z.items():
+                    d.set_field(k, d.get_field(k) if k == "profx_Qheat" else v)
+            d.thor()
+            d.sync()
+            res.append(dict(d.get_state(), q=d.get_field("profx_Qheat")))
+        out.append(res)
+        d.close()
+    for i, (a, b) in enumerate(zip(*out)):
+        for k in a:
+            assert np.array_equal(a[k], b[k]), (i, k)
+    assert np.abs(out[0][2]["q"]).max() > 0 and np.abs(out[0][3]["q"]).max() == 0

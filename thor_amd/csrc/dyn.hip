@@ -7,6 +7,7 @@
 #include "dyn_kernels.h"
 #include "dyn_kernels_lw.h"
 #include "dyn_kernels_ml.h"
+#include "dyn_kernels_slow.h"
 #include "dyn_kernels_solve.h"
 #include "mlp_internal.h"
 #include "tracer_kernels.h"
@@ -117,6 +118,11 @@ struct Dyn {
     float *dmbuf = nullptr;  // mixed form: DivM of the slow modes, [3][nv][S], when overlapped
     bool slow_lc64 = false;  // FP64 path: k_divm1_ml + k_slow_lc2<false> in place of k_slow<false>
     bool lw = false;       // FP64 path: horizontal operators as FP64 weights over level chunks (*_lw kernels)
+    bool slow_w = false;   // k_slow_w for the slow tendencies (production build, both forms)
+    // Host-side knowledge of the forcing tendencies: the arrays still hold the
+    // zeros they were created with (dMh and dWh) or that ProfX last wrote (Qheat),
+    // so the step's kernels need not read them.
+    bool zero_dm = true, zero_q = true;
     bool rows64 = false;   // FP64 path with lw: the mixed form's vertical solve (all rows sweep, one power per
                            // cell) and its split flux divergence, in FP64 storage
     bool fp64_ml = true;   // FP64 path: horizontal stencils over several levels per block (*_ml kernels)
@@ -383,6 +389,8 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             k_rk_arrays<<<(unsigned)((rk_count + 255) / 256), blk, 0, st>>>(d.rka, mode);
         });
     };
+    // the explicit sponge writes the tendencies in every stage
+    if (d.sponge_on && d.spg.mode != 0) d.zero_dm = d.zero_q = false;
     if (d.hooks.dyn_core_loop_init) {
         const thor_step_view v = view(stage_fields(d, 0));
         if (d.hooks.dyn_core_loop_init(d.hooks.user, (void *)st, nstep, &v)) return hook_fail("dyn_core_loop_init");
@@ -392,6 +400,8 @@ template <bool MX> static int thor_step_t(Dyn &d) {
         const double times = rk == 0 ? d.prm.timestep / 3.0 : d.prm.timestep / (double)ns_total;
         Fields f = stage_fields(d, rk);
         const Geo g = d.g;
+        if (d.zero_dm) f.dMh = f.dWh = nullptr;
+        if (d.zero_q) f.Qheat = nullptr;
         // second stream: the divergence-damping passes of the slow modes need
         // only the stage values, the factorisation only the column preparation
         const bool ovl = overlap_ok;
@@ -542,7 +552,8 @@ template <bool MX> static int thor_step_t(Dyn &d) {
                 launch(d, "divm1", W(0, 6), [&] { k_divm1_lc<<<grid_lc, blk, 0, st>>>(g, f, dm, lc); });
             launch(d, "slow_modes", W(19 + (rk ? 16 : 0), (divdamp ? 6 : 0) + 21 + (rk ? 3 : 0)),
                    [&] {
-                       if (d.slow_v2) k_slow_lc2<true><<<grid_ls, blk, 0, st>>>(g, f, dm, divdamp, rk, lcs);
+                       if (d.slow_w) k_slow_w<true><<<grid_ls, blk, 0, st>>>(g, f, dm, divdamp, rk, times, lcs);
+                       else if (d.slow_v2) k_slow_lc2<true><<<grid_ls, blk, 0, st>>>(g, f, dm, divdamp, rk, lcs);
                        else k_slow_lc<<<grid_ls, blk, 0, st>>>(g, f, dm, divdamp, rk, lcs);
                    });
         } else if (!MX && d.slow_lc64) {
@@ -556,7 +567,7 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             // booked as the reference's slow modes with DivM pass 1 (as the per-level kernel)
             launch(d, "slow_modes", W(19 + (rk ? 16 : 0), (divdamp ? 6 : 0) + 21 + (rk ? 3 : 0)),
                    [&] {
-                       if (d.rows64) k_slow_lc2<false, true><<<grid_ls, blk, 0, st>>>(g, f, f.diff, divdamp, rk, lcs);
+                       if (d.slow_w) k_slow_w<false><<<grid_ls, blk, 0, st>>>(g, f, f.diff, divdamp, rk, times, lcs);
                        else k_slow_lc2<false><<<grid_ls, blk, 0, st>>>(g, f, f.diff, divdamp, rk, lcs);
                    });
         } else {
@@ -573,12 +584,14 @@ template <bool MX> static int thor_step_t(Dyn &d) {
                 else k_divm0<MX><<<grid_t2, blk, 0, st>>>(g, f);
             });
         };
-        if (divdamp) divm0();
+        // the first stage starts from zero deviations: k_slow_w has written its momentum
+        const bool started = d.slow_w && rk == 0;
+        if (divdamp && !started) divm0();
         if (ovl) hipStreamWaitEvent(st, d.ev_s[3], 0);
         else factor(st);
         for (int ns = 0; ns < ns_it; ns++) {
             const int next = divdamp && ns < ns_it - 1;
-            launch(d, "momentum", W(1, (divdamp ? 6 : 0) + 12), [&] {
+            if (!(started && ns == 0)) launch(d, "momentum", W(1, (divdamp ? 6 : 0) + 12), [&] {
                 if (MX) k_momentum_lc<<<grid_lc, blk, 0, st>>>(g, f, divdamp, times, lc);
                 else if (lw) k_momentum_lw<<<grid_lc, blk, 0, st>>>(g, f, divdamp, times, lc);
                 else if (ml && d.ml_nl == 2) k_momentum_ml<2><<<grid_ml(2), blk, 0, st>>>(g, f, divdamp, times);
@@ -733,23 +746,29 @@ static int profx(Dyn &d, int forcing) {
     if (d.bl.on && forcing != THOR_FORCING_HELD_SUAREZ && forcing != THOR_FORCING_NEWTONIAN)
         launch(d, "boundary_layer", 8 * B, [&] { k_bl_rayleigh<<<grid_c, blk, 0, d.stream>>>(g, f, d.bl, dt); });
     if (forcing == THOR_FORCING_HELD_SUAREZ) {
+        const int zq = d.zero_q ? 0 : 1;
+        d.zero_q = true;
         launch(d, "profx_held_suarez", 24 * B, [&] {
-            if (d.small) k_profx_relax<THOR_FORCING_HELD_SUAREZ, 16><<<grid_c16, blk, 0, d.stream>>>(g, f, dt, 1, d.nr, d.bl);
-            else k_profx_relax<THOR_FORCING_HELD_SUAREZ, 64><<<grid_c, blk, 0, d.stream>>>(g, f, dt, 1, d.nr, d.bl);
+            if (d.small) k_profx_relax<THOR_FORCING_HELD_SUAREZ, 16><<<grid_c16, blk, 0, d.stream>>>(g, f, dt, zq, d.nr, d.bl);
+            else k_profx_relax<THOR_FORCING_HELD_SUAREZ, 64><<<grid_c, blk, 0, d.stream>>>(g, f, dt, zq, d.nr, d.bl);
         });
     } else if (forcing == THOR_FORCING_NEWTONIAN) {
         if (!d.nr_set) return fail(THOR_ERR_BAD_ARG, "profx: Newtonian forcing parameters not set");
         // W, T, relaxation and pressure per cell: Wh 2, p, rho, Mh untouched -> 4 in, W, p, Qheat out
+        const int zq = d.zero_q ? 0 : 1;
+        d.zero_q = true;
         launch(d, "profx_newtonian", 7 * B, [&] {
-            if (d.small) k_profx_relax<THOR_FORCING_NEWTONIAN, 16><<<grid_c16, blk, 0, d.stream>>>(g, f, dt, 1, d.nr, d.bl);
-            else k_profx_relax<THOR_FORCING_NEWTONIAN, 64><<<grid_c, blk, 0, d.stream>>>(g, f, dt, 1, d.nr, d.bl);
+            if (d.small) k_profx_relax<THOR_FORCING_NEWTONIAN, 16><<<grid_c16, blk, 0, d.stream>>>(g, f, dt, zq, d.nr, d.bl);
+            else k_profx_relax<THOR_FORCING_NEWTONIAN, 64><<<grid_c, blk, 0, d.stream>>>(g, f, dt, zq, d.nr, d.bl);
         });
     } else if (forcing == THOR_FORCING_DOUBLE_GRAY) {
         if (!d.rt_set) return fail(THOR_ERR_BAD_ARG, "profx: RT parameters not set");
         // Wh 2, p, rho in; W, T, Qheat, p out; two flux planes written and read twice
+        d.zero_q = false;
         launch(d, "profx_double_gray", 14 * B, [&] { launch_rt(d, g, f, dt); });
     } else if (forcing == THOR_FORCING_RT_SURROGATE) {
         if (!d.rt_set || !d.sur) return fail(THOR_ERR_BAD_ARG, "profx: RT surrogate not set");
+        d.zero_q = false;
         const bool judge = d.judge_every > 0 && d.sur_calls % d.judge_every == 0;
         int *cnt = d.sur_cnt + (d.sur_calls & 1), *cnt_next = d.sur_cnt + ((d.sur_calls & 1) ^ 1);
         d.sur_calls++;
@@ -1136,6 +1155,8 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
     }
     if (const char *e = std::getenv("THOR_SLOW_V2")) d.slow_v2 = std::atoi(e) != 0;
     d.prep_split = d.slow_lc;
+    // k_slow_w unless a switch asks for the kernels in the reference's order
+    d.slow_w = d.slow_lc && !std::getenv("THOR_SLOW_CHUNKED") && !std::getenv("THOR_SLOW_V2");
     if (const char *e = std::getenv("THOR_DIFF2_CHUNKED")) d.diff2_lc = std::atoi(e) != 0;
     d.f.thomas_rows = 1;
     if (const char *e = std::getenv("THOR_THOMAS_ROWS")) d.f.thomas_rows = std::atoi(e) != 0;
@@ -1165,6 +1186,7 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
     // spills at five waves per SIMD); its other kernels by their switches
     d.rows64 = d.lw && d.slow_lc64 && !g.energy && (nv - 1 + 15) / 16 <= 4 && !std::getenv("THOR_THOMAS_SEG64")
                && !std::getenv("THOR_THOMAS_COLUMNS");
+    if (!d.mixed) d.slow_w = d.lw && d.slow_lc64;
 #endif
     if (const char *e = std::getenv("THOR_FP64_MULTILEVEL")) d.fp64_ml = std::atoi(e) != 0;
     if (const char *e = std::getenv("THOR_ML_LEVELS")) {
@@ -1210,7 +1232,7 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
     A(&f.SlowMh, n3); A(&f.SlowWh, ni); A(&f.SlowRho, n1); A(&f.Slowp, n1);
     A(&f.Sp, n1); A(&f.Sd, n1); A(&f.hflx_r, n1); A(&f.hflx_pt, n1); A(&f.tAA, n1); A(&f.tCC, n1); A(&f.tTT, n1);
     A(&f.Qheat, n1); A(&f.dMh, n3); A(&f.dWh, ni);
-    if (d.mixed || d.rows64) A(&f.hflx_ptk, n1);
+    if (d.mixed || d.slow_w) A(&f.hflx_ptk, n1);
     if (g.energy) A(&f.Etot, n1);
     const bool diff_mid = prm->HyDiff && prm->HyDiffOrder >= 6;  // intermediate passes alternate two arrays
     if (diff_mid && !d.mixed) A(&f.diffx, 6 * n1);
@@ -1243,6 +1265,14 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
             k_solve_levels<<<1, 128, 0, d.stream>>>(g, tlv);
             e = hipGetLastError();
             g.tlv = tlv;
+        }
+        // and of k_slow_w
+        double *scl = nullptr;
+        if (e == hipSuccess) e = dalloc(d, &scl, (size_t)kSlowConst * (nv + 1));
+        if (e == hipSuccess) {
+            k_slow_consts<<<1, 128, 0, d.stream>>>(g, scl);
+            e = hipGetLastError();
+            g.scl = scl;
         }
         if (e != hipSuccess)
             return cleanup_fail(fail(THOR_ERR_HIP, std::string("thor_dyn_create: level table: ") + hipGetErrorString(e)));
@@ -1380,6 +1410,7 @@ extern "C" thor_status thor_dyn_step(thor_dyn *h, const thor_state *state, const
         transpose_async(d, user[i], dev[i], nlev[i], ncomp[i], true);
     }
     if (forcing) {
+        d.zero_q = d.zero_dm = false;
         transpose_async(d, forcing->Qheat, d.f.Qheat, d.nv, 1, true);
         transpose_async(d, forcing->dMh, d.f.dMh, d.nv, 3, true);
         transpose_async(d, forcing->dWh, d.f.dWh, d.nv + 1, 1, true);
@@ -1658,6 +1689,8 @@ extern "C" thor_status thor_dyn_set_field(thor_dyn *h, const char *name, const d
     int nlev, ncomp;
     if (!field_ptr(*h, name, dev, nlev, ncomp)) return fail(THOR_ERR_BAD_ARG, std::string("set_field: unknown ") + name);
     if (n != (long)h->P * nlev * ncomp) return fail(THOR_ERR_BAD_ARG, "set_field: size mismatch");
+    if (!std::strcmp(name, "profx_Qheat")) h->zero_q = false;
+    if (!std::strcmp(name, "profx_dMh") || !std::strcmp(name, "profx_dWh")) h->zero_dm = false;
     HIP_TRY(hipStreamSynchronize(h->stream));
     return copy_field(*h, dev, nlev, ncomp, const_cast<double *>(src), true, false);
 }

@@ -60,6 +60,7 @@ struct Geo {
     // Mixed precision only: per-level FP64 constants of the chunked slow modes
     // [6][nv]: r2p, r2m, r2l, rscale, dr2dz, (A / (A + Alt))^2 (k_slow_levels).
     const double *slv;
+    const double *scl;  // per-level constants of the slow tendencies [9][nv + 1] (k_slow_consts)
     const double *tlv;  // per-level constants of the vertical solve [6][nv + 1] (k_solve_levels)
     double A, Omega, Gravit, P_Ref, Rd, Cp;
     int deep, nonhydro, ghv;
@@ -90,7 +91,7 @@ struct Fields {
     double *hflx_r, *hflx_pt;             // horizontal flux divergences of the density / pressure update [nv]
     double *hflx_ptk;                     // split flux divergence: the stage part rs sum_k div_k(Mhk_k pt) of hflx_pt [nv]
     double *tAA, *tCC, *tTT;              // Thomas factorisation of the stage [nv]
-    double *Qheat, *dMh, *dWh;            // ProfX tendencies
+    double *Qheat, *dMh, *dWh;            // ProfX tendencies (null in the step's kernels: all zero)
     unsigned int *flags;                  // bit 0: NaN pressure, bit 1: NaN temperature
     int skip_w;                           // ProfX: W already set (by the sponge), do not recompute it from Wh
     int thomas_rows;                      // mixed path: both sweeps of the vertical solve on all rows of the block

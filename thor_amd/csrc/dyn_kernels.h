@@ -1290,12 +1290,12 @@ __device__ __forceinline__ void slow_tail(const Geo &g, const Fields &f, int p, 
     for (int k = 0; k < 3; k++) {
         v_dmh[k] = VEC(diffmh, k, lev, p);
         v_dmv[k] = f.diffmv ? VEC(f.diffmv, k, lev, p) : 0.0;
-        v_dM[k] = VEC(f.dMh, k, lev, p);
+        v_dM[k] = f.dMh ? VEC(f.dMh, k, lev, p) : 0.0;
         if (rk) v_y[k] = VEC(f.Mh, k, lev, p);
     }
-    const double v_dw = LV(diffw, lev), v_dwl = lev ? (double)LV(diffw, lev - 1) : 0.0, v_dWh = LV(f.dWh, lev),
+    const double v_dw = LV(diffw, lev), v_dwl = lev ? (double)LV(diffw, lev - 1) : 0.0, v_dWh = f.dWh ? LV(f.dWh, lev) : 0.0,
                  v_drh = LV(FS<MX>::diffrh(f), lev), v_dpr = LV(FS<MX>::diffpr(f), lev), v_gtil = LV(f.gtil, lev),
-                 v_q = LV(f.Qheat, lev), v_rho = rk ? LV(f.Rho, lev) : 0.0, v_p = rk ? LV(f.p, lev) : 0.0,
+                 v_q = f.Qheat ? LV(f.Qheat, lev) : 0.0, v_rho = rk ? LV(f.Rho, lev) : 0.0, v_p = rk ? LV(f.p, lev) : 0.0,
                  v_wh = rk ? LV(f.Wh, lev) : 0.0, v_whk = LV(f.Whk, lev);
     double advx = VEC(Adv, 0, lev, p), advy = VEC(Adv, 1, lev, p), advz = VEC(Adv, 2, lev, p);
     const double rho = LV(f.Rhok, lev);
@@ -2542,10 +2542,10 @@ __global__ __launch_bounds__(256, 1) void k_slow_lc(Geo g, Fields f, const float
                rPt = rsrc(f.pt, nv * pl8),
                rAdv = rsrc(f.mAdv, 3 * nv * pl4), rRk = rsrc(f.Rhok, nv * pl8),
                rWk = rsrc(f.Whk, (nv + 1) * pl8), rHh = rsrc(f.hh, (nv + 1) * pl8),
-               rDmh = rsrc(f.mdiffmh, 3 * nv * pl4), rdM = rsrc(f.dMh, 3 * nv * pl8),
-               rDw = rsrc(f.mdiffw, nv * pl4), rdW = rsrc(f.dWh, (nv + 1) * pl8),
+               rDmh = rsrc(f.mdiffmh, 3 * nv * pl4), rdM = rsrc(f.dMh, f.dMh ? 3 * nv * pl8 : 0),
+               rDw = rsrc(f.mdiffw, nv * pl4), rdW = rsrc(f.dWh, f.dWh ? (nv + 1) * pl8 : 0),
                rDr = rsrc(f.mdiffrh, nv * pl4), rDp = rsrc(f.mdiffpr, nv * pl4), rGt = rsrc(f.gtil, nv * pl8),
-               rQ = rsrc(f.Qheat, nv * pl8), rDM = rsrc(dm, 3 * nv * pl4), rM = rsrc(f.Mh, 3 * nv * pl8),
+               rQ = rsrc(f.Qheat, f.Qheat ? nv * pl8 : 0), rDM = rsrc(dm, 3 * nv * pl4), rM = rsrc(f.Mh, 3 * nv * pl8),
                rR = rsrc(f.Rho, nv * pl8), rPr = rsrc(f.p, nv * pl8), rW = rsrc(f.Wh, (nv + 1) * pl8);
     struct Stg {  // staged tile values: own point and halo point, two levels ahead
         double om[3], op, oh, ot, hm[3], hp, hh, ht;
@@ -2792,9 +2792,8 @@ __global__ __launch_bounds__(256, 1) void k_slow_lc(Geo g, Fields f, const float
 // two, and the values used late in a level are read at its start. The
 // arithmetic is slow_point's, so the results equal k_slow<MX>'s bit for bit.
 // dm: DivM (divergence-damping pass 1) of the tile points, from k_divm1_lc
-// (mixed), k_divm1_lw or k_divm1_ml (FP64). PTK: also form the stage part of
-// the substeps' pressure flux divergence, f.hflx_ptk.
-template <bool MX, bool PTK = MX>
+// (mixed) or k_divm1_ml (FP64).
+template <bool MX>
 __global__ __launch_bounds__(256, MX ? 2 : 1) void k_slow_lc2(Geo g, Fields f, const typename FS<MX>::R *dm,
                                                               int divdamp, int rk, int lc) {
     using R = typename FS<MX>::R;
@@ -2807,7 +2806,7 @@ __global__ __launch_bounds__(256, MX ? 2 : 1) void k_slow_lc2(Geo g, Fields f, c
         int lev;
         if (pole_ctx_lc(g, l0, l1, c, lev)) {
             double DivM[3] = {0.0, 0.0, 0.0};
-            if constexpr (MX || PTK) {  // dm holds the poles' DivM too
+            if constexpr (MX) {  // dm holds the poles' DivM too
                 if (divdamp)
                     for (int k = 0; k < 3; k++) DivM[k] = VEC(dm, k, lev, c.p);
             } else if (divdamp) {
@@ -2815,7 +2814,7 @@ __global__ __launch_bounds__(256, MX ? 2 : 1) void k_slow_lc2(Geo g, Fields f, c
                 divm_nf<true>(g, c.p, lev, 5, true, [&](int s, int k) { return VEC(f.divg, k, lev, c.gi(s)); }, none,
                               none, DivM);
             }
-            slow_sums<MX, kPoleUnroll>(
+            slow_sums<MX, 3>(
                 g, f, c.p, lev, true, rk, DivM, [&](int s) { return LVP(f.pk, lev, c.gi(s)); },
                 [&](int s) { return LVP(f.h, lev, c.gi(s)); }, [&](int s, int k) { return VEC(f.Mhk, k, lev, c.gi(s)); });
         }
@@ -2848,10 +2847,10 @@ __global__ __launch_bounds__(256, MX ? 2 : 1) void k_slow_lc2(Geo g, Fields f, c
                rPt = rsrc(f.pt, nv * pl8),
                rAdv = rsrc(FS<MX>::Adv(f), 3 * nv * plR), rRk = rsrc(f.Rhok, nv * pl8),
                rWk = rsrc(f.Whk, (nv + 1) * pl8), rHh = rsrc(f.hh, (nv + 1) * pl8),
-               rDmh = rsrc(FS<MX>::diffmh(f), 3 * nv * plR), rdM = rsrc(f.dMh, 3 * nv * pl8),
-               rDw = rsrc(FS<MX>::diffw(f), nv * plR), rdW = rsrc(f.dWh, (nv + 1) * pl8),
+               rDmh = rsrc(FS<MX>::diffmh(f), 3 * nv * plR), rdM = rsrc(f.dMh, f.dMh ? 3 * nv * pl8 : 0),
+               rDw = rsrc(FS<MX>::diffw(f), nv * plR), rdW = rsrc(f.dWh, f.dWh ? (nv + 1) * pl8 : 0),
                rDr = rsrc(FS<MX>::diffrh(f), nv * plR), rDp = rsrc(FS<MX>::diffpr(f), nv * plR),
-               rGt = rsrc(f.gtil, nv * pl8), rQ = rsrc(f.Qheat, nv * pl8), rDM = rsrc(dm, 3 * nv * plR),
+               rGt = rsrc(f.gtil, nv * pl8), rQ = rsrc(f.Qheat, f.Qheat ? nv * pl8 : 0), rDM = rsrc(dm, 3 * nv * plR),
                rM = rsrc(f.Mh, 3 * nv * pl8),
                rR = rsrc(f.Rho, nv * pl8), rPr = rsrc(f.p, nv * pl8), rW = rsrc(f.Wh, (nv + 1) * pl8);
     struct Stg {  // staged tile values: own point and halo point, two levels ahead
@@ -2872,7 +2871,7 @@ __global__ __launch_bounds__(256, MX ? 2 : 1) void k_slow_lc2(Geo g, Fields f, c
         v.hp = ldb_d(rPk, T.h8, l8);
         v.oh = ldb_d(rH, T.o8, l8);
         v.hh = ldb_d(rH, T.h8, l8);
-        if constexpr (PTK) {  // pt: the stage part of the substeps' pressure flux divergence
+        if constexpr (MX) {  // pt: the stage part of the substeps' pressure flux divergence
             v.ot = ldb_d(rPt, T.o8, l8);
             v.ht = ldb_d(rPt, T.h8, l8);
         } else {
@@ -2995,7 +2994,7 @@ __global__ __launch_bounds__(256, MX ? 2 : 1) void k_slow_lc2(Geo g, Fields f, c
             nflxp += rscale * sp3[k];
             dptk += rscale * st3[k];
         }
-        if constexpr (PTK) LV(f.hflx_ptk, lev) = dptk;
+        if constexpr (MX) LV(f.hflx_ptk, lev) = dptk;
         double whl, wht, hhl, hht;
         if (lev == 0) {
             whl = 0.0;
@@ -3513,7 +3512,7 @@ __device__ __forceinline__ void dp_column_in(const Geo &g, const Fields &f, int 
     const double dwdz = pole ? (wht * r2p - whl * r2l) / (dz * r2m) : (wht * r2p - whl * r2l) / (dr2dz);
     const double dwptdz = (wht2 * pht * r2p - whl2 * phl * r2l) / (dz * r2m);
     double aux = -(nflxpt + dwptdz) * dt;
-    const double pkv = LV(f.pk, lev);
+    const double pkv = LV(f.pk, lev), v_q = f.Qheat ? LV(f.Qheat, lev) : 0.0;
     const double r = LV(f.Rhok, lev) + rhos;
     nflxr += dwdz;
     const double rhosn = rhos + (slowrho - nflxr) * dt;
@@ -3527,7 +3526,7 @@ __device__ __forceinline__ void dp_column_in(const Geo &g, const Fields &f, int 
             // momentum (the new Whs + Whk interpolated to the centre)
             const double *Alt = g.Alt, *Alth = g.Alth, Gravit = g.Gravit;
             const int nv = g.nv;
-            aux += LV(f.Etot, lev) + (LV(f.diffpr, lev) + 0.0) * dt + LV(f.Qheat, lev) * dt;
+            aux += LV(f.Etot, lev) + (LV(f.diffpr, lev) + 0.0) * dt + v_q * dt;
             LV(f.Etot, lev) = aux;
             const double w =
                 (whl2 * (Alth[lev + 1] - Alt[lev]) + wht2 * (Alt[lev] - Alth[lev])) / (Alth[lev + 1] - Alth[lev]);
@@ -3565,12 +3564,12 @@ __device__ __forceinline__ void dp_column_in(const Geo &g, const Fields &f, int 
         } else {
             g1 = pm::pow(1.0 + x, gam) - 1.0;
         }
-        psn = pss + pf * g1 + (LV(FS<MX>::diffpr(f), lev) + 0.0) * dt + Rd / Cv * LV(f.Qheat, lev) * dt;
+        psn = pss + pf * g1 + (LV(FS<MX>::diffpr(f), lev) + 0.0) * dt + Rd / Cv * v_q * dt;
     } else {
         const double ptc = (P_Ref / (Rd * r)) * XPOW((pss + pkv) / P_Ref, Cv / Cp);
         aux += ptc * r;
         const double pnew = P_Ref * XPOW(Rd * aux / P_Ref, Cp / Cv);
-        psn = pnew - pkv + (LV(FS<MX>::diffpr(f), lev) + 0.0) * dt + Rd / Cv * LV(f.Qheat, lev) * dt;
+        psn = pnew - pkv + (LV(FS<MX>::diffpr(f), lev) + 0.0) * dt + Rd / Cv * v_q * dt;
     }
     LV(f.ps, lev) = psn;
     if (isnan(psn)) atomicOr(f.flags, FLAG_NAN_P);
