@@ -92,7 +92,10 @@ def measured_traffic(kernel: str, workload: str):
 # kernel symbol (demangled, rocprofv3) -> launch name of the library's per-kernel timing
 TRAFFIC_NAMES = [
     (r"k_profx_relax<1>", "profx_held_suarez"),
-    (r"k_column_prep", "column_prep"),
+    (r"k_column_consts", None),  # level tables, once per handle
+    (r"k_solve_levels", None),
+    (r"k_slow_consts", None),
+    (r"k_column_", "column_prep"),
     (r"k_adv_diff1", "adv_diff1"),
     (r"k_diff2_divm0", "diff2_divm0"),
     (r"k_diff2_lc", "diff2"),
@@ -104,7 +107,7 @@ TRAFFIC_NAMES = [
     (r"k_thomas_factor", "thomas_factor"),
     (r"k_momentum", "momentum"),
     (r"k_prepare", "prepare"),
-    (r"k_thomas_dp", "thomas_dp"),
+    (r"k_thomas_dp|k_solve", "thomas_dp"),
     (r"k_update_rk2", "update_rk2"),
 ]
 

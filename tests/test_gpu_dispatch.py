@@ -193,3 +193,46 @@ def test_known_zero_tendencies_equal_zeros_read(built, precision):
         for k in a:
             assert np.array_equal(a[k], b[k]), (i, k)
     assert np.abs(out[0][2]["q"]).max() > 0 and np.abs(out[0][3]["q"]).max() == 0
+
+
+@pytest.mark.parametrize("nv,extra", [
+    (3, {}), (16, {}), (17, dict(DeepModel=0)), (31, dict(GravHeightVar=1)), (32, dict(NonHydro=0)),
+    (33, dict(DeepModel=0, NonHydro=0, GravHeightVar=1)), (48, {}), (63, {}), (64, dict(GravHeightVar=1)), (65, {}),
+    (20, dict(thermo_equation=1)),
+])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_column_kernel_equals_the_separate_kernels(built, nv, extra, precision):
+    """Stage update, column preparation and factorisation in one kernel (rows of
+    one to four cells, constants from a table, pivots by scanned Moebius maps)
+    against the three kernels (THOR_COLPREP_LEVELS), one step; above 64 levels
+    both are the three. Bound: a few FP64 roundings per value and the powers'
+    2.5 (1 + |y log x|) ulp, 1e-12 of a field's scale (gtilh differences two
+    pressures, H / dz <= 20 times that); mixed: the advection's FP32 rounding
+    may fall the other way, 1e-9. The energy equation has the FP64 form only."""
+    capi = built
+    if precision and extra.get("thermo_equation"):
+        return
+    print(f"case: precision {precision} g4 L{nv} {extra}: column kernel vs separate kernels, 1 step", flush=True)
+    g = grid(capi, 4, nv)
+    p = earth_params(capi, 4, dt=600.0, ns=6, precision=precision, **extra)
+    st = capi.ic_rest(g, p, seed=2540 + nv, temperature_noise=1e-3, wind_noise=1.0)
+    out = []
+    for env in ({}, {"THOR_COLPREP_LEVELS": "2"}):
+        os.environ.update(env)
+        try:
+            d = capi.Dyn(g, p)
+        finally:
+            for k in env:
+                os.environ.pop(k, None)
+        d.set_state(st)
+        d.run(1)
+        d.sync()
+        out.append(dict(d.get_state(), **{k: d.get_field(k) for k in ("temperature", "h", "pt", "hh", "pth", "gtilh")}))
+        d.close()
+    a, b = out
+    cs = np.sqrt(p.Cp / (p.Cp - p.Rd) * p.Rd * p.Tmean)
+    for k in a:
+        scale = np.abs(b["Rho"]).max() * cs if k in ("Mh", "Wh", "W") else np.abs(b[k]).max()
+        err = np.abs(a[k] - b[k]).max() / scale
+        print(f"  {k}: {err:.2e}")
+        assert err < (1e-9 if precision else 2e-11 if k == "gtilh" else 1e-12), k

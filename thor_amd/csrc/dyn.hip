@@ -5,6 +5,7 @@
 #include "../../include/thor_mlp.h"
 #include "common.h"
 #include "dyn_kernels.h"
+#include "dyn_kernels_column.h"
 #include "dyn_kernels_lw.h"
 #include "dyn_kernels_ml.h"
 #include "dyn_kernels_slow.h"
@@ -118,6 +119,7 @@ struct Dyn {
     float *dmbuf = nullptr;  // mixed form: DivM of the slow modes, [3][nv][S], when overlapped
     bool slow_lc64 = false;  // FP64 path: k_divm1_ml + k_slow_lc2<false> in place of k_slow<false>
     bool lw = false;       // FP64 path: horizontal operators as FP64 weights over level chunks (*_lw kernels)
+    bool col_w = false;    // k_column_w at the start of a stage (production build, both forms)
     bool slow_w = false;   // k_slow_w for the slow tendencies (production build, both forms)
     // Host-side knowledge of the forcing tendencies: the arrays still hold the
     // zeros they were created with (dMh and dWh) or that ProfX last wrote (Qheat),
@@ -415,7 +417,23 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             launch(d, "divm1", W(0, 6), [&] { k_divm1_lc<<<grid_lc, blk, 0, s2>>>(g, f, d.dmbuf, lc); }, s2);
             hipEventRecord(d.ev_s[1], s2);  // DivM ready
         }
-        launch(d, "column_prep", W(12 + 5, 6), [&] {
+        // the update of the stage before with this stage's column preparation and
+        // factorisation, or the column preparation alone
+        if (d.col_w)
+            launch(d, "column_prep", W(12 + 5, 6) + (rk ? W(16, 3) : 0.0), [&] {
+                const dim3 gc((d.P + 15) / 16);
+                auto go = [&](auto seg) {
+                    constexpr int SEG = decltype(seg)::value;
+                    if (rk) k_column_w<SEG, true, MX><<<gc, 256, 0, st>>>(g, stage_fields(d, rk - 1), times);
+                    else k_column_w<SEG, false, MX><<<gc, 256, 0, st>>>(g, f, times);
+                };
+                const int seg = (d.nv + 15) / 16;
+                if (seg == 1) go(std::integral_constant<int, 1>{});
+                else if (seg == 2) go(std::integral_constant<int, 2>{});
+                else if (seg == 3) go(std::integral_constant<int, 3>{});
+                else go(std::integral_constant<int, 4>{});
+            });
+        else launch(d, "column_prep", W(12 + 5, 6), [&] {
             if (d.cp_lv == 4) k_column_prep_lv<MX, 4><<<grid_c4, blk, 0, st>>>(g, f);
             else if (d.cp_lv == 2) k_column_prep_lv<MX, 2><<<grid_c2, blk, 0, st>>>(g, f);
             else k_column_prep<MX><<<grid_c, blk, 0, st>>>(g, f);
@@ -588,7 +606,7 @@ template <bool MX> static int thor_step_t(Dyn &d) {
         const bool started = d.slow_w && rk == 0;
         if (divdamp && !started) divm0();
         if (ovl) hipStreamWaitEvent(st, d.ev_s[3], 0);
-        else factor(st);
+        else if (!d.col_w) factor(st);
         for (int ns = 0; ns < ns_it; ns++) {
             const int next = divdamp && ns < ns_it - 1;
             if (!(started && ns == 0)) launch(d, "momentum", W(1, (divdamp ? 6 : 0) + 12), [&] {
@@ -668,7 +686,8 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             // next substep's divergence-damping pass 0
             if (next) divm0();
         }
-        launch(d, "update_rk2", W(16, 3), [&] {
+        // with k_column_w the next stage's launch updates this one
+        if (!d.col_w || rk == 2) launch(d, "update_rk2", W(16, 3), [&] {
             const unsigned nc = (unsigned)((d.P + kTile - 1) / kTile);
             if (d.small) k_update_rk2<1, MX><<<dim3(nc, d.nv), blk, 0, st>>>(g, f);
             else k_update_rk2<kLC, MX><<<dim3(nc, (d.nv + kLC - 1) / kLC), blk, 0, st>>>(g, f);
@@ -1187,6 +1206,11 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
     d.rows64 = d.lw && d.slow_lc64 && !g.energy && (nv - 1 + 15) / 16 <= 4 && !std::getenv("THOR_THOMAS_SEG64")
                && !std::getenv("THOR_THOMAS_COLUMNS");
     if (!d.mixed) d.slow_w = d.lw && d.slow_lc64;
+    // up to four cells per row; offsets are 32 bits over a vector field. The
+    // switches choose among the kernels that k_column_w replaces.
+    d.col_w = (d.mixed || d.lw) && nv >= 2 && nv <= 64 && (size_t)24 * nv * d.S < 0x7fffffffu;
+    for (const char *k : {"THOR_COLPREP_LEVELS", "THOR_FACTOR_SEG", "THOR_STAGE_OVERLAP"})
+        if (std::getenv(k)) d.col_w = false;
 #endif
     if (const char *e = std::getenv("THOR_FP64_MULTILEVEL")) d.fp64_ml = std::atoi(e) != 0;
     if (const char *e = std::getenv("THOR_ML_LEVELS")) {
@@ -1273,6 +1297,14 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
             k_slow_consts<<<1, 128, 0, d.stream>>>(g, scl);
             e = hipGetLastError();
             g.scl = scl;
+        }
+        // and of k_column_w
+        double *ccl = nullptr;
+        if (e == hipSuccess) e = dalloc(d, &ccl, (size_t)kColConst * (nv + 1));
+        if (e == hipSuccess) {
+            k_column_consts<<<1, 128, 0, d.stream>>>(g, ccl);
+            e = hipGetLastError();
+            g.ccl = ccl;
         }
         if (e != hipSuccess)
             return cleanup_fail(fail(THOR_ERR_HIP, std::string("thor_dyn_create: level table: ") + hipGetErrorString(e)));

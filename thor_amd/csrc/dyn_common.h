@@ -60,6 +60,7 @@ struct Geo {
     // Mixed precision only: per-level FP64 constants of the chunked slow modes
     // [6][nv]: r2p, r2m, r2l, rscale, dr2dz, (A / (A + Alt))^2 (k_slow_levels).
     const double *slv;
+    const double *ccl;  // per-level constants of the stage's column kernel [13][nv + 1] (k_column_consts)
     const double *scl;  // per-level constants of the slow tendencies [9][nv + 1] (k_slow_consts)
     const double *tlv;  // per-level constants of the vertical solve [6][nv + 1] (k_solve_levels)
     double A, Omega, Gravit, P_Ref, Rd, Cp;
