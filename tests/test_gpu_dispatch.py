@@ -4,12 +4,13 @@ the states are equal bit for bit, whole chunks or not.
 """
 from __future__ import annotations
 
+import ctypes as C
 import os
 
 import numpy as np
 import pytest
 
-from common import STATE, earth_params, grid
+from common import HIP_D2H, HIP_H2D, STATE, earth_params, grid, hip_runtime
 
 pytestmark = pytest.mark.gpu
 
@@ -236,3 +237,39 @@ def test_column_kernel_equals_the_separate_kernels(built, nv, extra, precision):
         err = np.abs(a[k] - b[k]).max() / scale
         print(f"  {k}: {err:.2e}")
         assert err < (1e-9 if precision else 2e-11 if k == "gtilh" else 1e-12), k
+
+
+@pytest.mark.parametrize("glevel,nv", [(4, 3), (4, 21), (4, 22), (4, 64), (4, 65), (5, 97)])
+def test_device_layout_equals_the_host_one(built, glevel, nv):
+    """The state between device arrays in THOR's layout and the planes (tiles of
+    32 points x at most 64 values of a point's row: remainders of both, one to
+    five chunks per field) equals the conversion on the host, bit for bit, in both
+    directions."""
+    capi = built
+    print(f"case: g{glevel} L{nv}: device layout", flush=True)
+    hip = hip_runtime()
+    g = grid(capi, glevel, nv)
+    d = capi.Dyn(g, earth_params(capi, glevel, dt=600.0, ns=4))
+    rng = np.random.default_rng(nv)
+    st = {k: rng.standard_normal((g.P, nv + (k == "Wh")) + ((3,) if k == "Mh" else ())) for k in STATE}
+    ptrs = {}
+    try:
+        for k in STATE:
+            ptr = C.c_void_p()
+            assert hip.hipMalloc(C.byref(ptr), st[k].nbytes) == 0
+            ptrs[k] = ptr.value
+            assert hip.hipMemcpy(ptrs[k], st[k].ctypes.data, st[k].nbytes, HIP_H2D) == 0
+        s = capi.State(1, *(C.cast(C.c_void_p(ptrs[k]), capi._dp) for k in STATE))
+        d._chk(d.L.thor_dyn_set_state(d._h, C.byref(s)))
+        back = d.get_state()
+        d.set_state({k: -st[k] for k in STATE})
+        d._chk(d.L.thor_dyn_get_state(d._h, C.byref(s)))
+        for k in STATE:
+            out = np.empty_like(st[k])
+            assert hip.hipMemcpy(out.ctypes.data, ptrs[k], out.nbytes, HIP_D2H) == 0
+            assert np.array_equal(back[k].reshape(st[k].shape), st[k]), ("set", k)
+            assert np.array_equal(out, -st[k]), ("get", k)
+    finally:
+        d.close()
+        for ptr in ptrs.values():
+            hip.hipFree(ptr)

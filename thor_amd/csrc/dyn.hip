@@ -905,18 +905,9 @@ static bool field_ptr(Dyn &d, const std::string &n, double *&ptr, int &nlev, int
     return true;
 }
 
-static int copy_field(Dyn &d, double *dev, int nlev, int ncomp, double *user, bool to_device, bool user_on_device) {
-    const long n = (long)d.P * nlev * ncomp;
+// A field between the caller's host array in THOR's layout and its planes.
+static int copy_field(Dyn &d, double *dev, int nlev, int ncomp, double *user, bool to_device) {
     const size_t plane = (size_t)ncomp * nlev * d.S;
-    if (user_on_device) {
-        const int tb = 256;
-        const long nb = (n + tb - 1) / tb;
-        if (to_device) k_aos_to_soa<<<nb, tb, 0, d.stream>>>(user, dev, d.P, d.S, nlev, ncomp);
-        else k_soa_to_aos<<<nb, tb, 0, d.stream>>>(dev, user, d.P, d.S, nlev, ncomp);
-        HIP_TRY(hipGetLastError());
-        HIP_TRY(hipStreamSynchronize(d.stream));
-        return THOR_OK;
-    }
     std::vector<double> tmp(plane, 0.0);
     if (to_device) {
         for (int p = 0; p < d.P; p++)
@@ -986,13 +977,34 @@ static int set_timestep(Dyn &d, double dt) {
     return THOR_OK;
 }
 
-// Caller's array in THOR's layout <-> the library's level-planar copy, in
-// stream order on the handle's stream (no host synchronisation).
-static void transpose_async(Dyn &d, const double *src, double *dst, int nlev, int ncomp, bool to_planar) {
-    const long n = (long)d.P * nlev * ncomp;
-    const unsigned nb = (unsigned)((n + 255) / 256);
-    if (to_planar) k_aos_to_soa<<<nb, 256, 0, d.stream>>>(src, dst, d.P, d.S, nlev, ncomp);
-    else k_soa_to_aos<<<nb, 256, 0, d.stream>>>(src, dst, d.P, d.S, nlev, ncomp);
+// The caller's device arrays in THOR's layout <-> the library's level-planar
+// copies: the five state fields (Mh, Wh, W, Rho, pressure) and, with forcing,
+// its three tendencies, in stream order on the handle's stream (no host
+// synchronisation).
+static int layout_async(Dyn &d, double *const user[5], const thor_forcing *forcing, bool to_planar) {
+    static const char *const names[5] = {"Mh", "Wh", "W", "Rho", "pressure"};
+    Layout L{};
+    auto add = [&](double *caller, double *planes, int nlev, int ncomp) {
+        const int len = nlev * ncomp, n = (len + kLayoutRow - 1) / kLayoutRow;
+        L.f[L.n++] = {to_planar ? caller : planes, to_planar ? planes : caller, nlev, ncomp, L.chunks, (len + n - 1) / n};
+        L.chunks += n;
+    };
+    for (int i = 0; i < 5; i++) {
+        double *dev;
+        int nlev, ncomp;
+        field_ptr(d, names[i], dev, nlev, ncomp);
+        add(user[i], dev, nlev, ncomp);
+    }
+    if (forcing) {
+        add(const_cast<double *>(forcing->Qheat), d.f.Qheat, d.nv, 1);
+        add(const_cast<double *>(forcing->dMh), d.f.dMh, d.nv, 3);
+        add(const_cast<double *>(forcing->dWh), d.f.dWh, d.nv + 1, 1);
+    }
+    const unsigned nb = (unsigned)((d.P + kLayoutPts - 1) / kLayoutPts) * (unsigned)L.chunks;
+    if (to_planar) k_state_layout<true><<<nb, 256, 0, d.stream>>>(L, d.P, d.S);
+    else k_state_layout<false><<<nb, 256, 0, d.stream>>>(L, d.P, d.S);
+    HIP_TRY(hipGetLastError());
+    return THOR_OK;
 }
 
 } // namespace thor
@@ -1393,12 +1405,19 @@ static thor_status state_io(thor_dyn *h, const thor_state *s, bool to_device) {
     if (!h || !s) return fail(THOR_ERR_BAD_ARG, "state: null argument");
     double *user[5] = {s->Mh, s->Wh, s->W, s->Rho, s->pressure};
     const char *names[5] = {"Mh", "Wh", "W", "Rho", "pressure"};
+    for (double *u : user)
+        if (!u) return fail(THOR_ERR_BAD_ARG, "state: null field pointer");
+    if (s->on_device) {
+        const int rc = layout_async(*h, user, nullptr, to_device);
+        if (rc != THOR_OK) return rc;
+        HIP_TRY(hipStreamSynchronize(h->stream));
+        return THOR_OK;
+    }
     for (int i = 0; i < 5; i++) {
-        if (!user[i]) return fail(THOR_ERR_BAD_ARG, "state: null field pointer");
         double *dev;
         int nlev, ncomp;
         field_ptr(*h, names[i], dev, nlev, ncomp);
-        int rc = copy_field(*h, dev, nlev, ncomp, user[i], to_device, s->on_device != 0);
+        int rc = copy_field(*h, dev, nlev, ncomp, user[i], to_device);
         if (rc != THOR_OK) return rc;
     }
     return THOR_OK;
@@ -1434,27 +1453,12 @@ extern "C" thor_status thor_dyn_step(thor_dyn *h, const thor_state *state, const
     const hipStream_t cs = (hipStream_t)stream;
     HIP_TRY(hipEventRecord(d.ev_in, cs));
     HIP_TRY(hipStreamWaitEvent(d.stream, d.ev_in, 0));
-    const char *names[5] = {"Mh", "Wh", "W", "Rho", "pressure"};
-    double *dev[5];
-    int nlev[5], ncomp[5];
-    for (int i = 0; i < 5; i++) {
-        field_ptr(d, names[i], dev[i], nlev[i], ncomp[i]);
-        transpose_async(d, user[i], dev[i], nlev[i], ncomp[i], true);
-    }
-    if (forcing) {
-        d.zero_q = d.zero_dm = false;
-        transpose_async(d, forcing->Qheat, d.f.Qheat, d.nv, 1, true);
-        transpose_async(d, forcing->dMh, d.f.dMh, d.nv, 3, true);
-        transpose_async(d, forcing->dWh, d.f.dWh, d.nv + 1, 1, true);
-    }
-    HIP_TRY(hipGetLastError());
-    const int rc = thor_step(d);
+    if (forcing) d.zero_q = d.zero_dm = false;
+    int rc = layout_async(d, user, forcing, true);
+    if (rc == THOR_OK) rc = thor_step(d);
+    // the step swapped y(n) with the stage arrays
+    if (rc == THOR_OK) rc = layout_async(d, user, nullptr, false);
     if (rc != THOR_OK) return rc;
-    for (int i = 0; i < 5; i++) {
-        field_ptr(d, names[i], dev[i], nlev[i], ncomp[i]);  // the step swapped y(n) with the stage arrays
-        transpose_async(d, dev[i], user[i], nlev[i], ncomp[i], false);
-    }
-    HIP_TRY(hipGetLastError());
     // the caller's later work on its stream sees the new state
     HIP_TRY(hipEventRecord(d.ev_out, d.stream));
     HIP_TRY(hipStreamWaitEvent(cs, d.ev_out, 0));
@@ -1711,7 +1715,7 @@ extern "C" thor_status thor_dyn_get_field(thor_dyn *h, const char *name, double 
     if (!field_ptr(*h, name, dev, nlev, ncomp)) return fail(THOR_ERR_BAD_ARG, std::string("get_field: unknown ") + name);
     if (n != (long)h->P * nlev * ncomp) return fail(THOR_ERR_BAD_ARG, "get_field: size mismatch");
     HIP_TRY(hipStreamSynchronize(h->stream));
-    return copy_field(*h, dev, nlev, ncomp, dst, false, false);
+    return copy_field(*h, dev, nlev, ncomp, dst, false);
 }
 
 extern "C" thor_status thor_dyn_set_field(thor_dyn *h, const char *name, const double *src, long n) {
@@ -1724,7 +1728,7 @@ extern "C" thor_status thor_dyn_set_field(thor_dyn *h, const char *name, const d
     if (!std::strcmp(name, "profx_Qheat")) h->zero_q = false;
     if (!std::strcmp(name, "profx_dMh") || !std::strcmp(name, "profx_dWh")) h->zero_dm = false;
     HIP_TRY(hipStreamSynchronize(h->stream));
-    return copy_field(*h, dev, nlev, ncomp, const_cast<double *>(src), true, false);
+    return copy_field(*h, dev, nlev, ncomp, const_cast<double *>(src), true);
 }
 
 extern "C" thor_status thor_dyn_set_sponge(thor_dyn *h, const thor_sponge_params *q) {

@@ -4952,26 +4952,67 @@ __global__ __launch_bounds__(1024) void k_globdiag(Geo g, Fields f, double *part
 }
 
 // ============================================================ layout changes
-// THOR layout <-> level-planar layout, on the device.
-__global__ void k_aos_to_soa(const double *src, double *dst, int P, int S, int nlev, int ncomp) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;  // index into src
-    const long n = (long)P * nlev * ncomp;
-    if (i >= n) return;
-    const int c = (int)(i % ncomp);
-    const long r = i / ncomp;
-    const int lev = (int)(r % nlev);
-    const int p = (int)(r / nlev);
-    dst[((size_t)c * nlev + lev) * S + p] = src[i];
-}
-__global__ void k_soa_to_aos(const double *src, double *dst, int P, int S, int nlev, int ncomp) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long n = (long)P * nlev * ncomp;
-    if (i >= n) return;
-    const int c = (int)(i % ncomp);
-    const long r = i / ncomp;
-    const int lev = (int)(r % nlev);
-    const int p = (int)(r / nlev);
-    dst[i] = src[((size_t)c * nlev + lev) * S + p];
+// THOR layout [(p nlev + lev) ncomp + c] <-> level-planar layout [(c nlev +
+// lev) S + p], on the device, all fields of a state in one launch. A block takes
+// 32 points x up to 64 values of a point's row: the row's values by the lanes
+// of a wave (contiguous on THOR's side), the points by half waves (256 bytes of
+// a plane), transposed through LDS, eight loads of a thread in flight. One
+// thread per value and one launch per field, which this replaces, wrote (or
+// read) the planes with a stride: 141 us for a state into the planes and 109
+// back at 40 962 x 48, 38 and 30 at 10 242 x 40, 16 and 14 at 2 562 x 20. Here 64 and
+// 39 (memory: 47 for its 220 MB), 12 and 9, 5.2 and 4.4.
+constexpr int kLayoutPts = 32, kLayoutRow = 64, kLayoutMax = 8;
+struct LayoutField {
+    const double *src;
+    double *dst;
+    int nlev, ncomp, first, chunk;  // the field's first chunk of the launch; values per chunk
+};
+struct Layout {
+    LayoutField f[kLayoutMax];
+    int n, chunks;
+};
+template <bool PLANAR> __global__ __launch_bounds__(256) void k_state_layout(Layout L, int P, int S) {
+    __shared__ double s[kLayoutPts][kLayoutRow + 1];
+    const int ch = blockIdx.x % L.chunks, p0 = (blockIdx.x / L.chunks) * kLayoutPts;
+    int q = 0;
+    while (q + 1 < L.n && ch >= L.f[q + 1].first) q++;
+    const LayoutField F = L.f[q];
+    const int len = F.nlev * F.ncomp, j0 = (ch - F.first) * F.chunk, nj = min(F.chunk, len - j0);
+    const int t = threadIdx.x, j = t & 63, w = t >> 6, pp = t & 31, h = t >> 5;
+    auto plane = [&](int k) {  // of value k of a point's row
+        const int c = F.ncomp == 3 ? k % 3 : k % F.ncomp, lev = F.ncomp == 3 ? k / 3 : k / F.ncomp;
+        return ((size_t)c * F.nlev + lev) * S + p0 + pp;
+    };
+    double v[8];
+    if constexpr (PLANAR) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int r = w + 4 * i;
+            v[i] = j < nj && p0 + r < P ? F.src[(size_t)(p0 + r) * len + j0 + j] : 0.0;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) s[w + 4 * i][j] = v[i];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int k = h + 8 * i;
+            if (k < nj && p0 + pp < P) F.dst[plane(j0 + k)] = s[pp][k];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int k = h + 8 * i;
+            v[i] = k < nj && p0 + pp < P ? F.src[plane(j0 + k)] : 0.0;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) s[pp][h + 8 * i] = v[i];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const int r = w + 4 * i;
+            if (j < nj && p0 + r < P) F.dst[(size_t)(p0 + r) * len + j0 + j] = s[r][j];
+        }
+    }
 }
 
 } // namespace thor
