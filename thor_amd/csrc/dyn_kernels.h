@@ -3132,8 +3132,13 @@ __global__ void k_slow_levels(Geo g, double *out) {
 // and Rd T (the reference's variables 0..5), formed once per point from the
 // FP64 stage values and rounded to FP32, so no quotient is recomputed per
 // stencil slot. The horizontal advection is added to Adv (which holds the
-// vertical part from k_column_prep).
-__global__ __launch_bounds__(256, 3) void k_adv_diff1_lc(Geo g, Fields f, int hydiff, int lc) {
+// vertical part from the column preparation): per slot the mass flux through the
+// weights, sum_k w_k M_k, once, times the three velocity components. A staged
+// point is three 16-byte LDS words. Bound by arithmetic (the flux formed anew for
+// each component, four FP64 divisions per point and 84 4-byte LDS reads per cell:
+// 73 us at 40 962 x 48, 19.4 at 10 242 x 40, 9.3 at 2 562 x 20; here 65, 17 and 8.8
+// at two blocks per CU: at three it spills 12 registers, 73 and 18.8 us).
+__global__ __launch_bounds__(256, 2) void k_adv_diff1_lc(Geo g, Fields f, int hydiff, int lc) {
 #pragma clang fp contract(fast)
     int r, l0, l1;
     if (!block_tile_lc(g, lc, r, l0, l1)) return;
@@ -3155,7 +3160,9 @@ __global__ __launch_bounds__(256, 3) void k_adv_diff1_lc(Geo g, Fields f, int hy
         }
         return;
     }
-    __shared__ float sM[2][3][NHL2], sV[2][3][NHL2], sA[2][6][NHL2], sL[4][kLcMax];
+    // staged point: (M, rho), (v, W / rho), (M / rho, Rd T)
+    __shared__ float4 sM[2][NHL2], sV[2][NHL2], sU[2][NHL2];
+    __shared__ float sL[4][kLcMax];
     stage_lvc(g, l0, l1, sL);
     const LcThread T = lc_thread(g, r);
     const int p = T.p;
@@ -3197,17 +3204,11 @@ __global__ __launch_bounds__(256, 3) void k_adv_diff1_lc(Geo g, Fields f, int hy
     };
     // one staged point: M, v, and the six diffused variables
     auto put1 = [&](int b, int pos, const double m[3], double rho, double w, double t, const float fr[3]) {
-        const double wr = w / rho;
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            const double u = m[k] / rho;
-            sM[b][k][pos] = (float)m[k];
-            sV[b][k][pos] = (float)(u + wr * fr[k]);
-            sA[b][1 + k][pos] = (float)u;
-        }
-        sA[b][0][pos] = (float)rho;
-        sA[b][4][pos] = (float)wr;
-        sA[b][5][pos] = (float)(Rd * t);
+        const double inv = 1.0 / rho, wr = w * inv, u[3] = {m[0] * inv, m[1] * inv, m[2] * inv};
+        sM[b][pos] = make_float4((float)m[0], (float)m[1], (float)m[2], (float)rho);
+        sV[b][pos] = make_float4((float)(u[0] + wr * fr[0]), (float)(u[1] + wr * fr[1]), (float)(u[2] + wr * fr[2]),
+                                 (float)wr);
+        sU[b][pos] = make_float4((float)u[0], (float)u[1], (float)u[2], (float)(Rd * t));
     };
     auto put = [&](const In &v, int b) {
         put1(b, T.ir, v.om, v.orho, v.ow, v.ot, ofr);
@@ -3215,10 +3216,7 @@ __global__ __launch_bounds__(256, 3) void k_adv_diff1_lc(Geo g, Fields f, int hy
             if (qh >= 0) {
                 put1(b, T.hp, v.hm, v.hrho, v.hw, v.ht, hfr);
             } else {
-#pragma unroll
-                for (int k = 0; k < 3; k++) sM[b][k][T.hp] = sV[b][k][T.hp] = 0.f;
-#pragma unroll
-                for (int k = 0; k < 6; k++) sA[b][k][T.hp] = 0.f;
+                sM[b][T.hp] = sV[b][T.hp] = sU[b][T.hp] = make_float4(0.f, 0.f, 0.f, 0.f);
             }
         }
     };
@@ -3229,27 +3227,32 @@ __global__ __launch_bounds__(256, 3) void k_adv_diff1_lc(Geo g, Fields f, int hy
         load(L, min(lev + 2, l1 - 1));
         const int b = (lev - l0) & 1;
         const float rs = sL[0][lev - l0], rs2 = sL[1][lev - l0];
+        const float4 m0 = sM[b][T.pos[0]], v0 = sV[b][T.pos[0]], u0 = sU[b][T.pos[0]];
+        const float f0 = wd[0] * m0.x + wd[1] * m0.y + wd[2] * m0.z;
+        float sum[3] = {f0 * v0.x, f0 * v0.y, f0 * v0.z}, df[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int c = 0; c < 3; c++) {
-            float sum = 0.f;
-#pragma unroll
-            for (int kk = 0; kk < 3; kk++) {
-                float sk = wd[kk] * sV[b][c][T.pos[0]] * sM[b][kk][T.pos[0]];
-#pragma unroll
-                for (int s = 1; s < 7; s++) sk += wd[s * 3 + kk] * sV[b][c][T.pos[s]] * sM[b][kk][T.pos[s]];
-                sum += rs * sk;
+        for (int s = 1; s < 7; s++) {
+            const float4 m = sM[b][T.pos[s]], v = sV[b][T.pos[s]];
+            const float fl = wd[s * 3] * m.x + wd[s * 3 + 1] * m.y + wd[s * 3 + 2] * m.z;
+            sum[0] += fl * v.x;
+            sum[1] += fl * v.y;
+            sum[2] += fl * v.z;
+            if (hydiff) {
+                const float4 u = sU[b][T.pos[s]];
+                const float w = wl[s - 1];
+                df[0] += w * (m.w - m0.w);
+                df[1] += w * (u.x - u0.x);
+                df[2] += w * (u.y - u0.y);
+                df[3] += w * (u.z - u0.z);
+                df[4] += w * (v.w - v0.w);
+                df[5] += w * (u.w - u0.w);
             }
-            stb_f(rAd, T.o4, (unsigned)((c * nv + lev) * pl4), sum + adv[c]);
         }
+#pragma unroll
+        for (int c = 0; c < 3; c++) stb_f(rAd, T.o4, (unsigned)((c * nv + lev) * pl4), rs * sum[c] + adv[c]);
         if (hydiff) {
 #pragma unroll
-            for (int var = 0; var < 6; var++) {
-                const float a0 = sA[b][var][T.pos[0]];
-                float sum = wl[0] * (sA[b][var][T.pos[1]] - a0);
-#pragma unroll
-                for (int s = 2; s < 7; s++) sum += wl[s - 1] * (sA[b][var][T.pos[s]] - a0);
-                stb_f(rDf, T.o4, (unsigned)((var * nv + lev) * pl4), rs2 * sum);
-            }
+            for (int var = 0; var < 6; var++) stb_f(rDf, T.o4, (unsigned)((var * nv + lev) * pl4), rs2 * df[var]);
         }
         if (lev + 1 < l1) put(R, b ^ 1);
         __syncthreads();

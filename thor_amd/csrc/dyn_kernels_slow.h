@@ -42,8 +42,8 @@ __global__ void k_slow_consts(Geo g, double *out) {
 // k_slow_lc2 (the reference's order, 24 weight planes in LDS, about 30 buffer
 // descriptors, a dozen divisions per cell) spilled 24 vector and 245 scalar
 // registers at two blocks per CU: 168 us (mixed) and 228 (FP64) at 40 962 x 48,
-// 38.6 and 52.7 at 10 242 x 40, 16.5 and 18.9 at 2 562 x 20; here 136, 145, 27.6,
-// 33.4, 11.7 and 13.5 (110 and 140 for the traffic at 40 962 x 48).
+// 38.6 and 52.7 at 10 242 x 40, 16.5 and 18.9 at 2 562 x 20; here 135, 142, 27.1,
+// 33.1, 11.4 and 13.1 (110 and 140 for the traffic at 40 962 x 48).
 // dm: the damping pass 1 (k_divm1_lc, k_divm1_lw). At the first stage the
 // deviations start from zero, so the first substep's damping and pressure
 // gradient vanish and its momentum equation is Mhs = dt SlowMh (tangential):
@@ -136,9 +136,10 @@ __global__ __launch_bounds__(256, 2) void k_slow_w(Geo g, Fields f, const typena
     auto dot = [](const double a[3], const double c[3]) {
         return __builtin_fma(a[2], c[2], __builtin_fma(a[1], c[1], a[0] * c[0]));
     };
-    // the cell below: radial advection (or its hydrostatic form), rho, p, vertical diffusion
-    double c_advr = 0.0, c_rho = 0.0, c_p = 0.0, c_dw = 0.0;
+    // the cell below: radial advection (or its hydrostatic form), rho, p, vertical diffusion, gravity
+    double c_advr = 0.0, c_rho = 0.0, c_p = 0.0, c_dw = 0.0, c_g = 0.0;
     if (l0 > 0) {
+        c_g = g.scl[SC_G * N + l0 - 1];
         const unsigned o8 = T.o8 + (unsigned)(l0 - 1) * p8, oR = (unsigned)(T.p * sizeof(R)) + (unsigned)(l0 - 1) * pR;
         c_rho = ld(f.Rhok, 0, 0, o8);
         c_p = ld(f.pk, 0, 0, o8);
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(256, 2) void k_slow_w(Geo g, Fields f, const typena
         // vertical momentum at the interface below
         if (lev > 0) {
             const double wl = sK[SC_WL][i], wu = sK[SC_WU][i];
-            double lo = c_rho * (i ? sK[SC_G][i - 1] : g.scl[SC_G * N + lev - 1]), up = rho * sK[SC_G][i];
+            double lo = c_rho * c_g, up = rho * sK[SC_G][i];
             if (g.deep) {
                 lo += c_advr;
                 up += advr;
@@ -242,6 +243,7 @@ __global__ __launch_bounds__(256, 2) void k_slow_w(Geo g, Fields f, const typena
             st(f.SlowWh, 0, 0, o8, 0.0);
             LV(f.SlowWh, nv) = 0.0;
         }
+        c_g = sK[SC_G][i];
         const double ul = whl * sK[SC_R2][i], ut = wht * sK[SC_R2][i + 1];
         st(f.SlowRho, 0, 0, o8, v_drh - (rs * nr + (ut - ul) * sK[SC_IDR][i]));
         double sp = RoC * (v_q + vgp / rho - rs * nh - v_gt - (ut * hht - ul * hhl) * sK[SC_IDZ][i]);
