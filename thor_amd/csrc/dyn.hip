@@ -1374,6 +1374,49 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
         if (e != hipSuccess)
             return cleanup_fail(fail(THOR_ERR_HIP, std::string("thor_dyn_create: mixed-precision set-up: ") + hipGetErrorString(e)));
     }
+    {
+        // packed copies of the weights, [ceil(n / W)][S]
+        auto pack = [&](auto **dst, int n) {
+            using V = std::remove_const_t<std::remove_pointer_t<std::remove_pointer_t<decltype(dst)>>>;
+            const int W = sizeof(V) / sizeof(V::x);
+            void *v = nullptr;
+            if (e == hipSuccess) e = hipMalloc(&v, (size_t)((n + W - 1) / W) * S * sizeof(V));
+            if (e == hipSuccess) {
+                d.allocs.push_back(v);
+                e = hipMemsetAsync(v, 0, (size_t)((n + W - 1) / W) * S * sizeof(V), d.stream);
+            }
+            *dst = (V *)v;
+            return (V *)v;
+        };
+        auto put = [&](auto *v, const auto *src, int n, int off) {
+            if (e != hipSuccess) return;
+            k_pack_weights<<<(unsigned)((S + 255) / 256), 256, 0, d.stream>>>(src, v, (size_t)S, n, off);
+            e = hipGetLastError();
+        };
+        put(pack(&g.pdiv, 21), g.div, 21, 0);
+        double2 *gr = pack(&g.pgrad, 24);
+        put(gr, g.grad, 21, 0);
+        put(gr, g.div, 3, 21);
+        if (d.mixed) {
+            put(pack(&g.pwd, 63), g.wdd, 63, 0);
+            float4 *wg = pack(&g.pwg, 24), *wa = pack(&g.pwa, 27);
+            put(wg, g.grad, 21, 0);
+            put(wg, g.fr, 3, 21);
+            put(wa, g.div, 21, 0);
+            put(wa, g.wlap + S, 6, 21);
+        }
+        if (d.lw) {
+            put(pack(&g.pwd64, 63), g.wdd64, 63, 0);
+            put(pack(&g.pwu64, 21), g.udd64, 21, 0);
+            put(pack(&g.pwt64, 42), g.wdt64, 42, 0);
+            double2 *wg = pack(&g.pwg64, 20);
+            put(wg, g.wgt64, 14, 0);
+            put(wg, g.et64, 6, 14);
+        }
+        if (e == hipSuccess) e = hipStreamSynchronize(d.stream);
+        if (e != hipSuccess)
+            return cleanup_fail(fail(THOR_ERR_HIP, std::string("thor_dyn_create: packed weights: ") + hipGetErrorString(e)));
+    }
     *out = h;
     return THOR_OK;
 }

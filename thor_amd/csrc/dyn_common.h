@@ -54,6 +54,12 @@ struct Geo {
     const double *et64;    // [6][S]
     const double *wdt64;   // [42][S]
     const double *wgt64;   // [14][S]
+    // The same weights (and, from areas, the gradient and divergence) again with
+    // 16 bytes of a point together, [ceil(n / W)][S] of W values (k_pack_weights):
+    // what a level-chunked stencil loads in its prologue.
+    const float4 *pwd, *pwg, *pwa;                  // mixed: wdd 63; grad 21, fr 3; div 21, wlap 1..6
+    const double2 *pdiv, *pgrad;                    // div 21; grad 21, div of slot 0 (3)
+    const double2 *pwd64, *pwu64, *pwt64, *pwg64;   // FP64 weights: wdd 63; udd 21; wdt 42; wgt 14, et 6
     // Mixed precision only: per-level FP32 constants [4][nv]: rscale, rscale^2,
     // 1 / (Alth[lev] - Alth[lev + 1]) and Kdhz.
     const float *lvc;

@@ -137,10 +137,8 @@ __global__ __launch_bounds__(256, 2) void k_divm0_lw(Geo g, Fields f, int lc) {
     const LcThread T = lc_thread(g, r);
     const int p = T.p;
     double wd[63], wu[21];
-#pragma unroll
-    for (int i = 0; i < 63; i++) wd[i] = g.wdd64[(size_t)i * S + p];
-#pragma unroll
-    for (int i = 0; i < 21; i++) wu[i] = g.udd64[(size_t)i * S + p];
+    load_packed(g.pwd64, S, p, wd);
+    load_packed(g.pwu64, S, p, wu);
     const size_t pl8 = S * 8;
     const auto rM = rsrc(Mv, 3 * nv * pl8), rW = rsrc(Wv, (nv + 1) * pl8), rD = rsrc(f.divg, 3 * nv * pl8);
     struct In {
@@ -235,13 +233,10 @@ __global__ __launch_bounds__(256, 2) void k_momentum_lw(Geo g, Fields f, int div
     }
     const LcThread T = lc_thread(g, r);
     const int p = T.p;
-    double wd[42], wg[14], e[6];
-#pragma unroll
-    for (int i = 0; i < 42; i++) wd[i] = divdamp ? g.wdt64[(size_t)i * S + p] : 0.0;
-#pragma unroll
-    for (int i = 0; i < 14; i++) wg[i] = g.wgt64[(size_t)i * S + p];
-#pragma unroll
-    for (int i = 0; i < 6; i++) e[i] = g.et64[(size_t)i * S + p];
+    double wd[42] = {}, wg[20];  // wg: gradient, then the tangent basis
+    if (divdamp) load_packed(g.pwt64, S, p, wd);
+    load_packed(g.pwg64, S, p, wg);
+    const double *e = wg + 14;
     const size_t pl8 = S * 8;
     // without damping the divg loads fall outside an empty buffer and return 0
     const auto rG = rsrc(f.divg, divdamp ? 3 * nv * pl8 : 0), rP = rsrc(f.ps, nv * pl8), rS = rsrc(f.SlowMh, 3 * nv * pl8),
@@ -337,8 +332,7 @@ __global__ __launch_bounds__(256, 3) void k_divm1_lw(Geo g, Fields f, double *dm
     const LcThread T = lc_thread(g, r);
     const int p = T.p;
     double wd[42], e[6];
-#pragma unroll
-    for (int i = 0; i < 42; i++) wd[i] = g.wdt64[(size_t)i * S + p];
+    load_packed(g.pwt64, S, p, wd);
 #pragma unroll
     for (int i = 0; i < 6; i++) e[i] = g.et64[(size_t)i * S + p];
     const size_t pl8 = S * 8;
@@ -434,8 +428,7 @@ __global__ __launch_bounds__(256, 2) void k_adv_diff1_lw(Geo g, Fields f, int hy
     const LcThread T = lc_thread(g, r);
     const int p = T.p;
     double wd[21], wl[6];
-#pragma unroll
-    for (int i = 0; i < 21; i++) wd[i] = g.div[(size_t)i * S + p];
+    load_packed(g.pdiv, S, p, wd);
 #pragma unroll
     for (int s = 0; s < 6; s++) wl[s] = g.wlap64[(size_t)s * S + p];
     const int qh = T.hp >= 0 ? g.halo[r * NHALO + threadIdx.x] : -1;
@@ -673,8 +666,7 @@ __global__ __launch_bounds__(256, 2) void k_prepare_lw(Geo g, Fields f, int lc) 
     const LcThread T = lc_thread(g, r);
     const int p = T.p;
     double wv[21];
-#pragma unroll
-    for (int i = 0; i < 21; i++) wv[i] = g.div[(size_t)i * S + p];
+    load_packed(g.pdiv, S, p, wv);
     const size_t pl8 = S * 8;
     const auto rM = rsrc(f.Mhs, 3 * nv * pl8), rH = rsrc(f.h, nv * pl8), rPt = rsrc(f.pt, nv * pl8),
                rSp = rsrc(f.Slowp, nv * pl8), rPk = rsrc(f.hflx_ptk, nv * pl8), wSp = rsrc(f.Sp, nv * pl8),

@@ -84,11 +84,9 @@ __global__ __launch_bounds__(256, 2) void k_slow_w(Geo g, Fields f, const typena
         sK[i / (l1 - l0 + 1)][i % (l1 - l0 + 1)] = g.scl[(i / (l1 - l0 + 1)) * N + l0 + i % (l1 - l0 + 1)];
     const LcThread T = lc_thread(g, r);
     const int p = T.p;
-    double w[21], wd0[3];
-#pragma unroll
-    for (int i = 0; i < 21; i++) w[i] = g.grad[(size_t)i * S + p];
-#pragma unroll
-    for (int k = 0; k < 3; k++) wd0[k] = g.div[(size_t)k * S + p];
+    double w[24];  // gradient, then the divergence weights of slot 0
+    load_packed(g.pgrad, S, p, w);
+    const double *wd0 = w + 21;
     const double fr[3] = {g.fr[p], g.fr[S + p], g.fr[2 * S + p]};
     const unsigned p8 = (unsigned)S * 8u, pR = (unsigned)(S * sizeof(R));  // bytes of a level plane
     const size_t c8 = (size_t)nv * p8, cR = (size_t)nv * pR;               // of a component
