@@ -273,3 +273,30 @@ def test_device_layout_equals_the_host_one(built, glevel, nv):
         d.close()
         for ptr in ptrs.values():
             hip.hipFree(ptr)
+
+
+@pytest.mark.parametrize("ns", [0.0, 0.96, 0.99])
+@pytest.mark.parametrize("mode,temp", [(0, 0), (0, 1), (1, 1), (3, 0)])
+def test_sponge_from_any_level_bitwise(built, ns, mode, temp):
+    """The sponge's zonal means are formed at the damped levels only (Alt / top >=
+    ns): all of the levels, the top one, none. Parity build, two steps against the
+    oracle, which forms them everywhere: bit for bit."""
+    from common import hj_grid, hj_params, nr_params
+    from oracle.oracle import Oracle
+    capi = built
+    print(f"case: parity build, hot Jupiter g4 L20, sponge above {ns}, mode {mode}, temperature {temp}", flush=True)
+    g, p = hj_grid(capi, 4, 20), hj_params(capi, 4)
+    st = capi.ic_rest(g, p, seed=2640, temperature_noise=1.0, wind_noise=20.0)
+    q = capi.SpongeParams(ns, 2e-4, 1e-4, 16, 1, 1, temp, 3e-4 if temp else 0.0, mode)
+    d, o = capi.Dyn(g, p, variant="pm"), Oracle(g, p, variant="pm")
+    for x in (d, o):
+        x.set_state(st)
+        x.set_newtonian(nr_params(capi))
+        x.set_sponge(q)
+    d.run(2, capi.FORCING_NEWTONIAN)
+    d.sync()
+    o.run(2, capi.FORCING_NEWTONIAN)
+    a, b = d.get_state(), o.get_state()
+    d.close()
+    for k in STATE:
+        assert np.array_equal(a[k], b[k]), k

@@ -545,14 +545,16 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             fz.p = f.pk;
             const SpongePar sp = d.spg;
             const dim3 gpl((d.P + kTile - 1) / kTile, d.nv);
-            if (rk == 0 || sp.mode == 3) {
+            const int nl = d.nv - sp.l0;  // levels with a zonal mean
+            const dim3 gpz((d.P + kTile - 1) / kTile, nl);
+            if (nl > 0 && (rk == 0 || sp.mode == 3)) {
                 const int nc = sp.ncomp();
                 launch(d, "sponge_zonal", 6 * B, [&] {
-                    k_sponge_zonal<<<gpl, blk, 0, st>>>(g, fz, sp, d.ztab, d.ztmp);
+                    k_sponge_zonal<<<gpz, blk, 0, st>>>(g, fz, sp, d.ztab, d.ztmp);
                 });
                 launch(d, "sponge_mean", 8.0 * nc * sp.nlat * d.nv * sp.max_count, [&] {
-                    k_sponge_reduce<<<d.nv * nc * sp.nlat, 1024, 0, st>>>(sp, d.nv, d.ztmp, d.zout);
-                    k_sponge_vbar<<<(nc * sp.nlat * d.nv + 255) / 256, 256, 0, st>>>(sp, d.nv, d.zout, d.vbar);
+                    k_sponge_reduce<<<nl * nc * sp.nlat, 1024, 0, st>>>(sp, d.nv, d.ztmp, d.zout);
+                    k_sponge_vbar<<<(nc * sp.nlat * nl + 255) / 256, 256, 0, st>>>(sp, d.nv, d.zout, d.vbar);
                 });
             }
             launch(d, "sponge_drag", 12 * B, [&] {
@@ -741,15 +743,17 @@ static int profx(Dyn &d, int forcing) {
     if (d.sponge_on && d.spg.mode == 0) {
         const SpongePar sp = d.spg;
         const dim3 gpl((d.P + kTile - 1) / kTile, d.nv);
+        const int nl = d.nv - sp.l0;  // levels with a zonal mean
+        const dim3 gpz((d.P + kTile - 1) / kTile, nl);
         // Wh 2, Mh 3, rho in; W and the three zonal slots out
-        launch(d, "sponge_zonal", 10 * B, [&] {
-            k_sponge_zonal<<<gpl, blk, 0, d.stream>>>(g, f, sp, d.ztab, d.ztmp);
+        if (nl > 0) launch(d, "sponge_zonal", 10 * B, [&] {
+            k_sponge_zonal<<<gpz, blk, 0, d.stream>>>(g, f, sp, d.ztab, d.ztmp);
         });
-        if (sp.dmu || sp.dmw || sp.dmt) {
+        if (nl > 0 && (sp.dmu || sp.dmw || sp.dmt)) {
             const int nc = sp.ncomp();
             launch(d, "sponge_mean", 8.0 * nc * sp.nlat * d.nv * sp.max_count, [&] {
-                k_sponge_reduce<<<d.nv * nc * sp.nlat, 1024, 0, d.stream>>>(sp, d.nv, d.ztmp, d.zout);
-                k_sponge_vbar<<<(nc * sp.nlat * d.nv + 255) / 256, 256, 0, d.stream>>>(sp, d.nv, d.zout, d.vbar);
+                k_sponge_reduce<<<nl * nc * sp.nlat, 1024, 0, d.stream>>>(sp, d.nv, d.ztmp, d.zout);
+                k_sponge_vbar<<<(nc * sp.nlat * nl + 255) / 256, 256, 0, d.stream>>>(sp, d.nv, d.zout, d.vbar);
             });
         }
         // Mh 3, W, rho in; Mh 3, W out; then W 2 in, Wh out
@@ -1817,6 +1821,7 @@ extern "C" thor_status thor_dyn_set_sponge(thor_dyn *h, const thor_sponge_params
     SpongePar sp{q->ns, q->Ruv, q->Rw, nlat, q->damp_uv_to_mean != 0, q->damp_w_to_mean != 0, max_count,
                  (max_count + 2047) / 2048, q->temp_sponge != 0, q->temp_sponge ? q->RT_sponge : 0.0,
                  q->raysp_calc_mode};
+    while (sp.l0 < nv && !(h->alt_host[sp.l0] / h->alth_host[nv] >= q->ns)) sp.l0++;
     // (re)allocate the tables; the zonal slots beyond each bin's count stay zero
     for (void *ptr : {(void *)h->ztab, (void *)h->ztmp, (void *)h->zout, (void *)h->vbar, (void *)h->ztrig,
                       (void *)h->zkf, (void *)h->zcnt, (void *)h->zdw}) {

@@ -4705,6 +4705,7 @@ struct SpongePar {
     int dmt;                            // temperature sponge (RayleighSpongeT)
     double RT;
     int mode;                           // raysp_calc_mode: 0 imp, 1 exp1, 3 exp3
+    int l0;                             // the first level at or above ns: below it the rates are 0, no mean is formed
     const double *trig;                 // [4][S]: sin, cos of the longitude (in [0, 2 pi)) and of the latitude
     const double *kf;                   // [nv]: sin^2(pi/2 (n - ns) / (1 - ns)) above ns, else 0
     const int *cnt;                     // [nlat]: points per latitude bin
@@ -4741,20 +4742,29 @@ __device__ __forceinline__ void sponge_uv(const Geo &g, const Fields &f, const S
     v = (m0 * (-sa * cl) + m1 * (-sa * sl) + m2 * (ca)) / rho;
 }
 
+// W at the layer centre (Recompute_W, profx_auxiliary.h:110-130).
+__device__ __forceinline__ double sponge_w(const Geo &g, const Fields &f, int p, int lev) {
+    const size_t S = g.S;
+    const double whl = LV(f.Wh, lev), wht = LV(f.Wh, lev + 1);
+    const double xi = g.Alt[lev], xim = g.Alth[lev], xip = g.Alth[lev + 1];
+    const double intt = (xi - xip) / (xim - xip), intl = (xi - xim) / (xip - xim);
+    return whl * intt + wht * intl;
+}
+
 // ztab: [3][S] latitude bin, points in the bin, index within the bin;
 // tmp: [ncomp][nlat][nv][max_count] (u, v, w, T), zero beyond each bin's count.
+// Levels l0 .. nv - 1 (blockIdx.y), here and in the reduction: a mean below them is
+// multiplied by the rate 0. All levels before: 142 us (and 69 for the reduction) at
+// 163 842 x 48, 8.9 (13.1) at 10 242 x 40; with a quarter of the levels damped 38
+// (20) and 5.4 (5.6).
 __global__ __launch_bounds__(256) void k_sponge_zonal(Geo g, Fields f, SpongePar sp, const int *ztab, double *tmp) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x, lev = blockIdx.y;
+    const int p = blockIdx.x * blockDim.x + threadIdx.x, lev = sp.l0 + blockIdx.y;
     if (p >= g.P) return;
     const size_t S = g.S;
     const int nv = g.nv;
-    const double *Alt = g.Alt, *Alth = g.Alth;
     double w;
     if (sp.mode == 0) {  // Recompute_W first (profx_driver.cu:92)
-        const double whl = LV(f.Wh, lev), wht = LV(f.Wh, lev + 1);
-        const double xi = Alt[lev], xim = Alth[lev], xip = Alth[lev + 1];
-        const double intt = (xi - xip) / (xim - xip), intl = (xi - xim) / (xip - xim);
-        w = whl * intt + wht * intl;
+        w = sponge_w(g, f, p, lev);
         LV(f.W, lev) = w;
     } else {  // explicit modes: the stage's W (the caller passes Wk as f.W)
         w = LV(f.W, lev);
@@ -4779,7 +4789,8 @@ __global__ __launch_bounds__(256) void k_sponge_zonal(Geo g, Fields f, SpongePar
 // below the count has the sum +0.
 __global__ __launch_bounds__(1024) void k_sponge_reduce(SpongePar sp, int nv, const double *tmp, double *out) {
     __shared__ double ds[2048];
-    const int t = threadIdx.x, lev = blockIdx.x % nv, cb = blockIdx.x / nv;  // cb = component * nlat + bin
+    const int nl = nv - sp.l0, t = threadIdx.x, lev = sp.l0 + blockIdx.x % nl;
+    const int cb = blockIdx.x / nl;  // component * nlat + bin
     const long L = sp.max_count, n = min(L, (long)sp.cnt[cb % sp.nlat]);
     const double *row = tmp + ((size_t)cb * nv + lev) * L;
     double *o = out + ((size_t)cb * nv + lev) * sp.nb;
@@ -4805,8 +4816,9 @@ __global__ __launch_bounds__(1024) void k_sponge_reduce(SpongePar sp, int nv, co
 // vbar[bin][lev][component, stride 4] = 0 + the block sums in order (the
 // host loops of gpu_sum_on_device_sponge and gpu_sum_on_device).
 __global__ void k_sponge_vbar(SpongePar sp, int nv, const double *out, double *vbar) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;  // (component, bin, lev)
-    if (i >= sp.ncomp() * sp.nlat * nv) return;
+    const int j = blockIdx.x * blockDim.x + threadIdx.x, nl = nv - sp.l0;
+    if (j >= sp.ncomp() * sp.nlat * nl) return;
+    const int i = j / nl * nv + sp.l0 + j % nl;  // (component, bin, lev)
     const int comp = i / (sp.nlat * nv), rem = i % (sp.nlat * nv);
     double s = 0.0;
     for (int b = 0; b < sp.nb; b++) s += out[(size_t)i * sp.nb + b];
@@ -4840,17 +4852,18 @@ __global__ __launch_bounds__(256) void k_sponge_apply(Geo g, Fields f, SpongePar
         return vbar[((size_t)intlat * nv + lev) * 4 + c] * intt + vbar[((size_t)(intlat + 1) * nv + lev) * 4 + c] * intl;
     };
     const double rho = LV(f.Rho, lev);
-    const double w = LV(f.W, lev) / rho;
+    const bool damped = lev >= sp.l0;  // else k_sponge_zonal has not formed W
+    const double w = (damped ? LV(f.W, lev) : sponge_w(g, f, p, lev)) / rho;
     const double kuv = rv * sp.Ruv * sp.kf[lev], kw = rv * sp.Rw * sp.kf[lev];
     double unew, vnew, wnew;
-    if (sp.dmu) {
+    if (sp.dmu && damped) {
         unew = (u / dt + kuv * mean_at(0)) / (1.0 / dt + kuv);
         vnew = (v / dt + kuv * mean_at(1)) / (1.0 / dt + kuv);
     } else {
         unew = (u / dt) / (1.0 / dt + kuv);
         vnew = (v / dt) / (1.0 / dt + kuv);
     }
-    if (sp.dmw) wnew = (w / dt + kw * mean_at(2)) / (1.0 / dt + kw);
+    if (sp.dmw && damped) wnew = (w / dt + kw * mean_at(2)) / (1.0 / dt + kw);
     else wnew = (w / dt) / (1.0 / dt + kw);
     const double sl = sp.trig[p], cl = sp.trig[S + p], sa = sp.trig[2 * S + p], ca = sp.trig[3 * S + p];
     const double vx = unew * (-sl) + vnew * (-sa * cl);
@@ -4862,7 +4875,7 @@ __global__ __launch_bounds__(256) void k_sponge_apply(Geo g, Fields f, SpongePar
     LV(f.W, lev) = wnew * rho;
     if (sp.dmt) {  // temperature towards its zonal mean, through the pressure
         const double kT = rv * sp.RT * sp.kf[lev], temperature = LV(f.p, lev) / g.Rd / rho;
-        LV(f.p, lev) = rho * g.Rd * (temperature / dt + kT * mean_at(3)) / (1.0 / dt + kT);
+        LV(f.p, lev) = rho * g.Rd * (damped ? temperature / dt + kT * mean_at(3) : temperature / dt) / (1.0 / dt + kT);
     }
 }
 
@@ -4870,6 +4883,7 @@ __global__ __launch_bounds__(256) void k_sponge_apply(Geo g, Fields f, SpongePar
 // as k_sponge_apply forms it.
 __device__ __forceinline__ double sponge_mean(const Geo &g, const SpongePar &sp, const int *ztab, const double *vbar,
                                               int p, int lev, int c) {
+    if (lev < sp.l0) return 0.0;  // its rate is 0
     const size_t S = g.S;
     const int nv = g.nv, nlat = sp.nlat, intlat = ztab[p];
     const double des_lat = M_PI / nlat, lat = g.lonlat[S + p];
