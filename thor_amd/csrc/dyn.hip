@@ -1290,46 +1290,32 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
     }
     if (e != hipSuccess) return cleanup_fail(fail(THOR_ERR_HIP, std::string("thor_dyn_create: alloc: ") + hipGetErrorString(e)));
     {
-        // per-level constants of the chunked slow modes (both forms)
-        double *slv = nullptr;
-        if (e == hipSuccess) e = dalloc(d, &slv, (size_t)6 * nv);
+        // per-level constants (nv <= 127): of the chunked slow modes, the vertical
+        // solve, k_slow_w and k_column_w, in one allocation
+        const size_t n = (size_t)nv + 1;
+        double *lv = nullptr;
+        if (e == hipSuccess) e = dalloc(d, &lv, (6 + 6 + kSlowConst + kColConst) * n);
         if (e == hipSuccess) {
+            double *slv = lv, *tlv = lv + 6 * n, *scl = tlv + 6 * n, *ccl = scl + kSlowConst * n;
             k_slow_levels<<<(nv + 63) / 64, 64, 0, d.stream>>>(g, slv);
-            e = hipGetLastError();
-            g.slv = slv;
-        }
-        // and of the vertical solve (nv <= 127)
-        double *tlv = nullptr;
-        if (e == hipSuccess) e = dalloc(d, &tlv, (size_t)6 * (nv + 1));
-        if (e == hipSuccess) {
             k_solve_levels<<<1, 128, 0, d.stream>>>(g, tlv);
-            e = hipGetLastError();
-            g.tlv = tlv;
-        }
-        // and of k_slow_w
-        double *scl = nullptr;
-        if (e == hipSuccess) e = dalloc(d, &scl, (size_t)kSlowConst * (nv + 1));
-        if (e == hipSuccess) {
             k_slow_consts<<<1, 128, 0, d.stream>>>(g, scl);
-            e = hipGetLastError();
-            g.scl = scl;
-        }
-        // and of k_column_w
-        double *ccl = nullptr;
-        if (e == hipSuccess) e = dalloc(d, &ccl, (size_t)kColConst * (nv + 1));
-        if (e == hipSuccess) {
             k_column_consts<<<1, 128, 0, d.stream>>>(g, ccl);
             e = hipGetLastError();
+            g.slv = slv;
+            g.tlv = tlv;
+            g.scl = scl;
             g.ccl = ccl;
         }
         if (e != hipSuccess)
             return cleanup_fail(fail(THOR_ERR_HIP, std::string("thor_dyn_create: level table: ") + hipGetErrorString(e)));
     }
     if (d.lw) {
-        double *wlap = nullptr, *wdd = nullptr, *udd = nullptr, *et = nullptr, *wdt = nullptr, *wgt = nullptr;
-        A(&wlap, (size_t)6 * S); A(&wdd, (size_t)63 * S); A(&udd, (size_t)21 * S);
-        A(&et, (size_t)6 * S); A(&wdt, (size_t)42 * S); A(&wgt, (size_t)14 * S);
+        double *w = nullptr;
+        A(&w, (size_t)(6 + 63 + 21 + 6 + 42 + 14) * S);
         if (e == hipSuccess) {
+            double *wlap = w, *wdd = wlap + (size_t)6 * S, *udd = wdd + (size_t)63 * S, *et = udd + (size_t)21 * S,
+                   *wdt = et + (size_t)6 * S, *wgt = wdt + (size_t)42 * S;
             Geo gu = g;
             gu.deep = 0;  // rscale = 1
             k_probe_weights64<<<(P + 255) / 256, 256, 0, d.stream>>>(gu, wlap, wdd, udd, et, wdt, wgt);
@@ -1379,18 +1365,20 @@ extern "C" thor_status thor_dyn_create(const thor_grid_desc *gd, const thor_para
             return cleanup_fail(fail(THOR_ERR_HIP, std::string("thor_dyn_create: mixed-precision set-up: ") + hipGetErrorString(e)));
     }
     {
-        // packed copies of the weights, [ceil(n / W)][S]
+        // packed copies of the weights, [ceil(n / W)][S], 16 bytes each, in one
+        // allocation (values past n are loaded but not used)
+        const size_t planes = 11 + 12 + (d.mixed ? 16 + 6 + 7 : 0) + (d.lw ? 32 + 11 + 21 + 10 : 0);
+        char *next = nullptr;
+        if (e == hipSuccess) e = hipMalloc((void **)&next, planes * S * 16);
+        if (e == hipSuccess) d.allocs.push_back(next);
         auto pack = [&](auto **dst, int n) {
             using V = std::remove_const_t<std::remove_pointer_t<std::remove_pointer_t<decltype(dst)>>>;
-            const int W = sizeof(V) / sizeof(V::x);
-            void *v = nullptr;
-            if (e == hipSuccess) e = hipMalloc(&v, (size_t)((n + W - 1) / W) * S * sizeof(V));
-            if (e == hipSuccess) {
-                d.allocs.push_back(v);
-                e = hipMemsetAsync(v, 0, (size_t)((n + W - 1) / W) * S * sizeof(V), d.stream);
-            }
-            *dst = (V *)v;
-            return (V *)v;
+            constexpr int W = sizeof(V) / sizeof(V::x);
+            static_assert(sizeof(V) == 16);
+            V *v = (V *)next;
+            next += (size_t)((n + W - 1) / W) * S * 16;
+            *dst = v;
+            return v;
         };
         auto put = [&](auto *v, const auto *src, int n, int off) {
             if (e != hipSuccess) return;

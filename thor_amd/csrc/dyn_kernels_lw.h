@@ -637,7 +637,7 @@ __global__ __launch_bounds__(256, 3) void k_diff_lw(Geo g, Fields f, const doubl
 
 // Prepare_Implicit_Vertical (thor_vertical_int.h:566-771) and the horizontal
 // flux divergences of Density_Pressure_Eqs with the stage part of the pressure
-// flux divergence taken from f.hflx_ptk (k_slow_lc2<false, true>) and Sd left to
+// flux divergence taken from f.hflx_ptk (k_slow_w) and Sd left to
 // the vertical solve, as k_prepare_lc<true>: the stage momentum is not read
 // and one plane less is written in every substep (10 doubles per cell instead
 // of 14: 63 -> 45 us at 40 962 x 48, 19.4 -> 14.2 at 10 242 x 40).
