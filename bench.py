@@ -91,15 +91,15 @@ def measured_traffic(kernel: str, workload: str):
 
 # kernel symbol (demangled, rocprofv3) -> launch name of the library's per-kernel timing
 TRAFFIC_NAMES = [
-    (r"k_profx_relax<1>", "profx_held_suarez"),
+    (r"k_profx_relax<1", "profx_held_suarez"),
     (r"k_column_consts", None),  # level tables, once per handle
     (r"k_solve_levels", None),
-    (r"k_slow_consts", None),
+    (r"k_slow_consts|k_pack_weights", None),
     (r"k_column_", "column_prep"),
     (r"k_adv_diff1", "adv_diff1"),
     (r"k_diff2_divm0", "diff2_divm0"),
-    (r"k_diff2_lc", "diff2"),
-    (r"k_divm0_lc<true>", "divm0_stage"),
+    (r"k_diff2_lc|k_diff_lw", "diff2"),
+    (r"k_divm0_l[cw]<true>", "divm0_stage"),
     (r"k_divm0", "divm0"),
     (r"k_divm1", "divm1"),
     (r"k_slow_levels", None),  # the slow modes' level table, once per handle
