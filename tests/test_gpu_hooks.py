@@ -12,7 +12,9 @@ thor_auxiliary.h:376-387, 482-494). Checked here:
     substep ends the step at x0 + S * dt exactly as the RK3 combination
     implies (stage weights 1/3, 1/2 - 1/3 ... sum to one step), for both
     precision modes. Closed form: the stage deviations start at 0, then
-    x_i - x_k, so after stage 3 x_k = x0 + S * (ns * dt / ns) = x0 + S dt.
+    x_i - x_k, so after stage 3 x_k = x0 + S * (ns * dt / ns) = x0 + S dt;
+  * what a hook sets through the library (forcing tendencies, the sponge)
+    counts from the next kernel on that reads it.
 """
 from __future__ import annotations
 
@@ -174,3 +176,98 @@ def test_hook_error_stops_the_step(setup):
     assert e.value.code == capi.THOR_ERR_HOOK
     d.sync()
     d.close()
+
+
+@pytest.mark.parametrize("precision,variant,extra", [
+    (0, "", {}), (1, "", {}), (0, "pm", {}), (0, "", dict(thermo_equation=1)),
+])
+def test_tendencies_set_by_a_hook_count_at_once(setup, precision, variant, extra):
+    """A hook that sets the forcing tendencies with thor_dyn_set_field acts from
+    the next kernel on that reads them, whether the arrays held zeros known to
+    the host (which the step does not read) or written ones: bit for bit the
+    same states. At the first slow-mode hook nothing has read them yet, so that
+    equals setting them before the step, also where Held-Suarez clears the
+    heating in every ProfX; at a fast-mode hook the update of that very substep
+    takes the heating."""
+    capi, g = setup
+    p = earth_params(capi, 4, dt=600.0, ns=6, precision=precision, **extra)
+    st = _state(capi, g, p)
+    rng = np.random.default_rng(17)
+    tend = {"profx_Qheat": 1e-2 * rng.standard_normal((g.P, g.nv)),
+            "profx_dMh": 1e-4 * rng.standard_normal((g.P, g.nv, 3)),
+            "profx_dWh": 1e-5 * rng.standard_normal((g.P, g.nv + 1))}
+
+    def run(when, written, forcing, steps):
+        """when: (hook, its index within the step); written: zeros written to the arrays before."""
+        d = capi.Dyn(g, p, variant=variant)
+        d.set_state(st)
+        if written:
+            for k, v in tend.items():
+                d.set_field(k, np.zeros_like(v))
+        seen = {}
+
+        def hook(kind):
+            def f(stream, nstep, *rest):
+                i = seen[kind, nstep] = seen.get((kind, nstep), -1) + 1
+                if (kind, i) == when:
+                    for k, v in tend.items():
+                        d.set_field(k, v)
+                return 0
+            return f
+
+        d.set_hooks(init=hook("init"), slow_modes=hook("slow"), fast_modes=hook("fast"))
+        d.run(steps, forcing)
+        d.sync()
+        out = d.get_state()
+        d.close()
+        return out
+
+    none, hs = capi.FORCING_NONE, capi.FORCING_HELD_SUAREZ
+    print(f"case: precision {precision} {variant} {extra}: tendencies set by hooks", flush=True)
+    quiet = run(None, False, none, 1)
+    pairs = [("first slow-mode hook = init hook, Held-Suarez", run(("slow", 0), False, hs, 2), run(("init", 0), False, hs, 2))]
+    for when in (("slow", 0), ("slow", 1), ("fast", 0), ("fast", 2)):
+        pairs.append((when, run(when, False, none, 1), run(when, True, none, 1)))
+        assert np.abs(pairs[-1][1]["pressure"] - quiet["pressure"]).max() > 0, when
+    for name, a, b in pairs:
+        for k in a:
+            assert np.isfinite(a[k]).all(), (name, k)
+            assert np.array_equal(a[k], b[k]), (name, k)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_sponge_switched_on_by_a_hook(setup, precision):
+    """The explicit sponge writes the tendencies of the stage. Switched on by the
+    first slow-mode hook of a step it acts in that stage, as when it was
+    switched on before the step: bit for bit the same states."""
+    from common import hj_grid, hj_params
+    capi, _ = setup
+    g, p = hj_grid(capi, 4, 20), hj_params(capi, 4, precision=precision)
+    st = capi.ic_rest(g, p, seed=1104, temperature_noise=1.0, wind_noise=20.0)
+    q = capi.SpongeParams(0.5, 2e-4, 1e-4, 16, 1, 1, 1, 3e-4, 3)
+    out = []
+    for by_hook in (False, True):
+        print(f"case: precision {precision} hot Jupiter g4 L20: explicit sponge, switched on by a hook: {by_hook}", flush=True)
+        d = capi.Dyn(g, p)
+        d.set_state(st)
+        calls = []
+
+        def slow(stream, nstep, times, view):
+            if not calls:
+                d.set_sponge(q)
+            calls.append(nstep)
+            return 0
+
+        if by_hook:
+            d.set_hooks(slow_modes=slow)
+        else:
+            d.set_sponge(q)
+        d.thor()
+        d.sync()
+        out.append(dict(d.get_state(), **{k: d.get_field(k) for k in ("profx_Qheat", "profx_dMh", "profx_dWh")}))
+        d.close()
+    a, b = out
+    assert np.abs(a["profx_dMh"]).max() > 0 and np.abs(a["profx_Qheat"]).max() > 0
+    for k in a:
+        assert np.isfinite(a[k]).all(), k
+        assert np.array_equal(a[k], b[k]), k

@@ -391,8 +391,6 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             k_rk_arrays<<<(unsigned)((rk_count + 255) / 256), blk, 0, st>>>(d.rka, mode);
         });
     };
-    // the explicit sponge writes the tendencies in every stage
-    if (d.sponge_on && d.spg.mode != 0) d.zero_dm = d.zero_q = false;
     if (d.hooks.dyn_core_loop_init) {
         const thor_step_view v = view(stage_fields(d, 0));
         if (d.hooks.dyn_core_loop_init(d.hooks.user, (void *)st, nstep, &v)) return hook_fail("dyn_core_loop_init");
@@ -402,8 +400,13 @@ template <bool MX> static int thor_step_t(Dyn &d) {
         const double times = rk == 0 ? d.prm.timestep / 3.0 : d.prm.timestep / (double)ns_total;
         Fields f = stage_fields(d, rk);
         const Geo g = d.g;
-        if (d.zero_dm) f.dMh = f.dWh = nullptr;
-        if (d.zero_q) f.Qheat = nullptr;
+        // Tendencies that are all zero are not read. A hook may set them (or a
+        // sponge that writes them), so this is asked again after every hook.
+        auto drop_zeros = [&] {
+            f.dMh = d.zero_dm ? nullptr : d.f.dMh;
+            f.dWh = d.zero_dm ? nullptr : d.f.dWh;
+            f.Qheat = d.zero_q ? nullptr : d.f.Qheat;
+        };
         // second stream: the divergence-damping passes of the slow modes need
         // only the stage values, the factorisation only the column preparation
         const bool ovl = overlap_ok;
@@ -537,7 +540,8 @@ template <bool MX> static int thor_step_t(Dyn &d) {
                 return hook_fail("dyn_core_loop_slow_modes");
         }
         if (d.sponge_on && d.spg.mode != 0) {
-            // explicit Rayleigh sponge on the stage values, before the slow modes
+            // explicit Rayleigh sponge on the stage values, before the slow modes: writes the tendencies
+            d.zero_dm = d.zero_q = false;
             Fields fz = f;
             fz.Mh = f.Mhk;
             fz.Rho = f.Rhok;
@@ -563,6 +567,7 @@ template <bool MX> static int thor_step_t(Dyn &d) {
                 k_sponge_dwh<<<dim3((d.P + kTile - 1) / kTile, d.nv + 1), blk, 0, st>>>(g, d.zdw, f.dWh);
             });
         }
+        drop_zeros();
         if (MX && d.slow_lc) {
             // DivM from the second stream, or into the idle hyperdiffusion
             // scratch (its first three planes)
@@ -679,6 +684,7 @@ template <bool MX> static int thor_step_t(Dyn &d) {
                 const thor_step_view v = view(f);
                 if (d.hooks.dyn_core_loop_fast_modes(d.hooks.user, (void *)st, nstep, times, &v))
                     return hook_fail("dyn_core_loop_fast_modes");
+                drop_zeros();
                 launch(d, "density_pressure", W(18, 4), [&] {
                     const dim3 gd((d.P + kTile - 1) / kTile, d.nv);
                     if (solve) k_dp_solve<MX><<<gd, blk, 0, st>>>(g, f, times);
