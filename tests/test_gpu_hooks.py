@@ -271,3 +271,53 @@ def test_sponge_switched_on_by_a_hook(setup, precision):
     for k in a:
         assert np.isfinite(a[k]).all(), k
         assert np.array_equal(a[k], b[k]), k
+
+
+def _with_env(capi, g, p, env):
+    """A handle created under the switches env."""
+    import os
+    old = {k: os.environ.get(k) for k in env}
+    os.environ.update(env)
+    try:
+        return capi.Dyn(g, p)
+    finally:
+        for k, v in old.items():
+            os.environ.pop(k) if v is None else os.environ.update({k: v})
+
+
+def _agree(p, a, b, tol):
+    cs = np.sqrt(p.Cp / (p.Cp - p.Rd) * p.Rd * p.Tmean)
+    for k in a:
+        scale = np.abs(b["Rho"]).max() * cs if k in ("Mh", "Wh", "W") else np.abs(b[k]).max()
+        err = np.abs(a[k] - b[k]).max() / scale
+        print(f"  {k}: {err:.2e}")
+        assert err < tol, k
+
+
+@pytest.mark.parametrize("field,factor", [("hh", 2.0), ("gtilh", 2.0)])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_slow_mode_hook_reaches_the_vertical_solve(setup, precision, field, factor):
+    """hh and gtilh set by a slow-mode hook enter the stage's factorisation, also
+    where the column kernel has formed it before the hook: against the separate
+    kernels (THOR_COLPREP_LEVELS), which form it after. Bound as for the column
+    kernel without a hook: FP64 rounding, 1e-12 of a field's scale, mixed 1e-9."""
+    capi, g = setup
+    p = earth_params(capi, 4, dt=600.0, ns=6, precision=precision)
+    st = _state(capi, g, p)
+    out = []
+    for env, hooked in (({}, True), ({"THOR_COLPREP_LEVELS": "2"}, True), ({}, False)):
+        print(f"case: precision {precision} g4 L20: {field} x {factor} by a slow-mode hook: {hooked}, {env}", flush=True)
+        d = _with_env(capi, g, p, env)
+        d.set_state(st)
+        if hooked:
+            def slow(stream, nstep, times, view):
+                d.set_field(field, factor * d.get_field(field))
+                return 0
+            d.set_hooks(slow_modes=slow)
+        d.thor()
+        d.sync()
+        out.append(d.get_state())
+        d.close()
+    a, b, quiet = out
+    assert np.abs(b["Wh"] - quiet["Wh"]).max() > 1e-4 * np.abs(b["Wh"]).max()  # the hook does something
+    _agree(p, a, b, 1e-9 if precision else 1e-12)

@@ -125,6 +125,7 @@ struct Dyn {
     // zeros they were created with (dMh and dWh) or that ProfX last wrote (Qheat),
     // so the step's kernels need not read them.
     bool zero_dm = true, zero_q = true;
+    bool set_factor = false;  // set_field has written hh or gtilh since the stage began
     bool rows64 = false;   // FP64 path with lw: the mixed form's vertical solve (all rows sweep, one power per
                            // cell) and its split flux divergence, in FP64 storage
     bool fp64_ml = true;   // FP64 path: horizontal stencils over several levels per block (*_ml kernels)
@@ -420,6 +421,7 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             launch(d, "divm1", W(0, 6), [&] { k_divm1_lc<<<grid_lc, blk, 0, s2>>>(g, f, d.dmbuf, lc); }, s2);
             hipEventRecord(d.ev_s[1], s2);  // DivM ready
         }
+        d.set_factor = false;
         // the update of the stage before with this stage's column preparation and
         // factorisation, or the column preparation alone
         if (d.col_w)
@@ -538,6 +540,8 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             const thor_step_view v = view(f);
             if (d.hooks.dyn_core_loop_slow_modes(d.hooks.user, (void *)st, nstep, times, &v))
                 return hook_fail("dyn_core_loop_slow_modes");
+            // k_column_w has formed the factorisation already
+            if (d.col_w && d.set_factor) factor(st);
         }
         if (d.sponge_on && d.spg.mode != 0) {
             // explicit Rayleigh sponge on the stage values, before the slow modes: writes the tendencies
@@ -1766,6 +1770,7 @@ extern "C" thor_status thor_dyn_set_field(thor_dyn *h, const char *name, const d
     int nlev, ncomp;
     if (!field_ptr(*h, name, dev, nlev, ncomp)) return fail(THOR_ERR_BAD_ARG, std::string("set_field: unknown ") + name);
     if (n != (long)h->P * nlev * ncomp) return fail(THOR_ERR_BAD_ARG, "set_field: size mismatch");
+    if (!std::strcmp(name, "hh") || !std::strcmp(name, "gtilh")) h->set_factor = true;
     if (!std::strcmp(name, "profx_Qheat")) h->zero_q = false;
     if (!std::strcmp(name, "profx_dMh") || !std::strcmp(name, "profx_dWh")) h->zero_dm = false;
     HIP_TRY(hipStreamSynchronize(h->stream));
