@@ -321,3 +321,36 @@ def test_slow_mode_hook_reaches_the_vertical_solve(setup, precision, field, fact
     a, b, quiet = out
     assert np.abs(b["Wh"] - quiet["Wh"]).max() > 1e-4 * np.abs(b["Wh"]).max()  # the hook does something
     _agree(p, a, b, 1e-9 if precision else 1e-12)
+
+
+@pytest.mark.parametrize("field", ["pt", "h", "pth"])
+def test_fast_mode_hook_reaches_the_flux_divergences(setup, field):
+    """FP64: what a fast-mode hook sets of pt, h and pth enters the later substeps
+    of the stage whole, also where the stage part of the pressure flux
+    divergence has been formed with the slow tendencies: against the kernels
+    that form it anew in every substep (THOR_THOMAS_SEG64). Bound as for the row
+    solve: FP64 rounding, 1e-12 of a field's scale."""
+    capi, g = setup
+    p = earth_params(capi, 4, dt=600.0, ns=6)
+    st = capi.ic_rest(g, p, seed=1204, temperature_noise=1.0, wind_noise=20.0)
+    out = []
+    for env, hooked in (({}, True), ({"THOR_THOMAS_SEG64": "0"}, True), ({}, False)):
+        print(f"case: FP64 g4 L20: {field} x 1.1 by a fast-mode hook: {hooked}, {env}", flush=True)
+        d = _with_env(capi, g, p, env)
+        d.set_state(st)
+        calls = []
+
+        def fast(stream, nstep, times, view):
+            if len(calls) == 2:  # the second stage's second substep of three
+                d.set_field(field, 1.1 * d.get_field(field))
+            calls.append(times)
+            return 0
+        if hooked:
+            d.set_hooks(fast_modes=fast)
+        d.thor()
+        d.sync()
+        out.append(d.get_state())
+        d.close()
+    a, b, quiet = out
+    assert np.abs(b["pressure"] - quiet["pressure"]).max() > 1e-9 * np.abs(b["pressure"]).max()
+    _agree(p, a, b, 1e-12)

@@ -126,6 +126,7 @@ struct Dyn {
     // so the step's kernels need not read them.
     bool zero_dm = true, zero_q = true;
     bool set_factor = false;  // set_field has written hh or gtilh since the stage began
+    bool set_pt = false;      // set_field has written pt since the slow tendencies
     bool rows64 = false;   // FP64 path with lw: the mixed form's vertical solve (all rows sweep, one power per
                            // cell) and its split flux divergence, in FP64 storage
     bool fp64_ml = true;   // FP64 path: horizontal stencils over several levels per block (*_ml kernels)
@@ -572,6 +573,7 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             });
         }
         drop_zeros();
+        d.set_pt = false;
         if (MX && d.slow_lc) {
             // DivM from the second stream, or into the idle hyperdiffusion
             // scratch (its first three planes)
@@ -634,7 +636,8 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             launch(d, "prepare", MX && d.prep_split ? W(4, 5) : W(7, 3), [&] {
                 if (MX && d.prep_split) k_prepare_lc<true><<<grid_lc, blk, 0, st>>>(g, f, lc);
                 else if (MX) k_prepare_lc<false><<<grid_lc, blk, 0, st>>>(g, f, lc);
-                else if (d.rows64) k_prepare_lw<<<grid_lc, blk, 0, st>>>(g, f, lc);
+                // (the stage part of the pressure flux divergence is k_slow_w's, unless a fast-mode hook has set pt since)
+                else if (d.rows64 && !d.set_pt) k_prepare_lw<<<grid_lc, blk, 0, st>>>(g, f, lc);
                 else if (ml && d.prep64) k_prepare_lc64<<<grid_lc, blk, 0, st>>>(g, f, lc);
                 else if (ml) k_prepare_ml<2><<<grid_ml(2), blk, 0, st>>>(g, f);
                 else k_prepare<MX><<<grid_t2, blk, 0, st>>>(g, f);
@@ -1771,6 +1774,7 @@ extern "C" thor_status thor_dyn_set_field(thor_dyn *h, const char *name, const d
     if (!field_ptr(*h, name, dev, nlev, ncomp)) return fail(THOR_ERR_BAD_ARG, std::string("set_field: unknown ") + name);
     if (n != (long)h->P * nlev * ncomp) return fail(THOR_ERR_BAD_ARG, "set_field: size mismatch");
     if (!std::strcmp(name, "hh") || !std::strcmp(name, "gtilh")) h->set_factor = true;
+    if (!std::strcmp(name, "pt")) h->set_pt = true;
     if (!std::strcmp(name, "profx_Qheat")) h->zero_q = false;
     if (!std::strcmp(name, "profx_dMh") || !std::strcmp(name, "profx_dWh")) h->zero_dm = false;
     HIP_TRY(hipStreamSynchronize(h->stream));
