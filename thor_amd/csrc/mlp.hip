@@ -263,13 +263,17 @@ static void infer(Net &n, long rows) {
     }
 }
 
-static double sum_loss(Net &n, const double *dev, long slots) {
+// Adds the squared errors of the slots to *sum. The wait is the only one of a
+// fused epoch: a failure of any kernel queued before it shows here.
+static hipError_t sum_loss(Net &n, const double *dev, long slots, double *sum) {
     std::vector<double> part((size_t)slots);
-    (void)hipMemcpyAsync(part.data(), dev, slots * sizeof(double), hipMemcpyDeviceToHost, n.stream);
-    (void)hipStreamSynchronize(n.stream);
+    hipError_t e = hipMemcpyAsync(part.data(), dev, slots * sizeof(double), hipMemcpyDeviceToHost, n.stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(n.stream);
+    if (e != hipSuccess) return e;
     double s = 0.0;
     for (double v : part) s += v;
-    return s;
+    *sum += s;
+    return e;
 }
 
 } // namespace mlp
@@ -447,11 +451,11 @@ extern "C" thor_status thor_mlp_train_epoch(thor_mlp *m, int batch, float lr, un
                                                                      bc1, bc2);
         refresh_bf16(n);
         MLP_TRY(hipGetLastError());
-        total += sum_loss(n, n.loss_part, (rows * n.nout + 255) / 256);  // sum of squared errors of the batch
+        MLP_TRY(sum_loss(n, n.loss_part, (rows * n.nout + 255) / 256, &total));  // of the batch
     }
     MLP_TRY(hipGetLastError());
     // fused: every batch left its groups' sums (the last batch has the fewest)
-    if (n.fused) total = sum_loss(n, n.tpart, (nb - 1) * gpb + (n.ndata - (nb - 1) * batch + 31) / 32);
+    if (n.fused) MLP_TRY(sum_loss(n, n.tpart, (nb - 1) * gpb + (n.ndata - (nb - 1) * batch + 31) / 32, &total));
     if (loss) *loss = total / (double)n.ndata / n.nout;
     return THOR_OK;
 }
@@ -504,9 +508,12 @@ extern "C" thor_status thor_mlp_gradients(thor_mlp *m, const float *X, const flo
     if (e == hipSuccess) e = hipStreamSynchronize(net.stream);
     (void)hipFree(dX);
     if (e != hipSuccess) return fail(THOR_ERR_HIP, std::string("thor_mlp_gradients: ") + hipGetErrorString(e));
-    if (loss)
-        *loss = (net.fused ? sum_loss(net, net.tpart, groups) : sum_loss(net, net.loss_part, (n * net.nout + 255) / 256))
-                / (double)(n * net.nout);
+    if (loss) {
+        double sum = 0.0;
+        if (net.fused) MLP_TRY(sum_loss(net, net.tpart, groups, &sum));
+        else MLP_TRY(sum_loss(net, net.loss_part, (n * net.nout + 255) / 256, &sum));
+        *loss = sum / (double)(n * net.nout);
+    }
     return THOR_OK;
 }
 
