@@ -50,26 +50,47 @@ def test_forward_matches_oracle(built):
     m.close()
 
 
-def test_fused_inference_equals_training_forward(built):
-    """thor_mlp_forward runs the fused three-layer inference kernel; the
-    training path (thor_mlp_gradients) runs three separate GEMMs with the same
-    K tiling and epilogues. With zero targets the training loss is mean(Y^2)
-    of the GEMM outputs, so it must equal mean(Y^2) of the fused outputs."""
+def test_fused_forms_equal_the_layer_by_layer_ones(built):
+    """Networks of 256 hidden units, at most 128 inputs and 64 outputs take the
+    fused kernels; the same network with inputs that are zero added beyond 128
+    takes three GEMMs forward and the layer-by-layer backward, with the same K
+    tiling (the added products are exact zeros) and epilogues. The outputs are
+    equal; so is the training loss, the mean of the squared outputs for zero
+    targets, to its FP64 sum's rounding; the gradients' sums over the rows
+    associate differently in FP32, 1000 rows x 2^-24 = 6e-5 of a block's norm,
+    and a delta that falls the other way in BF16 adds 2^-8 of one row in 1000:
+    1e-3."""
     capi = built
-    print("case: fused inference vs three-GEMM forward, 1000 rows (partial last block)", flush=True)
+    rows, pad = 1000, 133
+    print(f"case: fused form vs layer by layer ({pad} inputs), {rows} rows (partial last block)", flush=True)
     m = capi.MLP(*DIMS, seed=6)
     rng = np.random.default_rng(7)
     p = m.params()
     nb = DIMS[0] * DIMS[1]
     p[nb:nb + DIMS[1]] = 0.1 * rng.standard_normal(DIMS[1])
     m.set_params(p)
-    X = rng.standard_normal((1000, DIMS[0])).astype(np.float32)
-    Y = m.forward(X).astype(np.float64)
-    _, loss = m.gradients(X, np.zeros((1000, DIMS[2]), np.float32))
-    want = float((Y ** 2).mean())
-    print(f"mean(Y^2): fused {want:.12e}, GEMM path {loss:.12e}")
-    assert abs(loss / want - 1) < 1e-9
+    dims = (pad, DIMS[1], DIMS[2])
+    wide = capi.MLP(*dims, seed=0)
+    q = np.concatenate([p[:nb], np.zeros((pad - DIMS[0]) * DIMS[1], np.float32), p[nb:]])
+    wide.set_params(q)
+    X = rng.standard_normal((rows, DIMS[0])).astype(np.float32)
+    Xw = np.concatenate([X, np.zeros((rows, pad - DIMS[0]), np.float32)], axis=1)
+    Y, Yw = m.forward(X), wide.forward(Xw)
+    print(f"outputs: {np.count_nonzero(Y != Yw)} of {Y.size} differ, max {np.abs(Y - Yw).max():.2e}")
+    assert np.array_equal(Y, Yw)
+    zero = np.zeros((rows, DIMS[2]), np.float32)
+    (g, loss), (gw, lossw) = m.gradients(X, zero), wide.gradients(Xw, zero)
+    want = float((Y.astype(np.float64) ** 2).mean())
+    print(f"mean(Y^2): {want:.12e}, fused loss {loss:.12e}, layer by layer {lossw:.12e}")
+    assert abs(loss / want - 1) < 1e-9 and abs(lossw / want - 1) < 1e-9
+    ba, bw = _blocks(g, DIMS), _blocks(gw, dims)
+    bw["W1"] = bw["W1"][:nb]
+    for k in ba:
+        e = np.linalg.norm(ba[k] - bw[k]) / np.linalg.norm(bw[k])
+        print(f"  d{k}: relative L2 diff {e:.2e}")
+        assert e < 1e-3, k
     m.close()
+    wide.close()
 
 
 def test_gradients_match_oracle(built):
@@ -262,8 +283,9 @@ def test_fused_training_kernels_match_oracle(built, nin, nout, rows):
     edges of its 32-row groups and 32 x 32 gradient tiles, against the oracle;
     tolerances as test_gradients_match_oracle. Then Adam's first step: the
     parameters move by at most lr, against the gradient's sign where the
-    gradient is not near zero, and the operand copies follow (the next
-    forward uses the new parameters)."""
+    gradient is not near zero, and the forward operands follow (the next
+    forward uses the new parameters; the backward ones:
+    test_training_epoch_matches_oracle)."""
     from oracle import mlp_oracle as mo
     capi = built
     dims = (nin, 256, nout)
@@ -292,3 +314,129 @@ def test_fused_training_kernels_match_oracle(built, nin, nout, rows):
     Yo, _ = mo.forward(m.params(), X, dims, bf=True)
     assert np.abs(Y - Yo).max() / np.abs(Yo).max() < 1e-2
     m.close()
+
+
+class _MT64:
+    """The 64-bit Mersenne Twister (Nishimura 2000), the generator of the epoch's shuffle."""
+
+    def __init__(self, seed):
+        self.x = [seed & (2 ** 64 - 1)]
+        for i in range(1, 312):
+            self.x.append((6364136223846793005 * (self.x[-1] ^ (self.x[-1] >> 62)) + i) & (2 ** 64 - 1))
+        self.i = 312
+
+    def __call__(self):
+        x = self.x
+        if self.i == 312:
+            for i in range(312):
+                y = (x[i] & 0xFFFFFFFF80000000) | (x[(i + 1) % 312] & 0x7FFFFFFF)
+                x[i] = x[(i + 156) % 312] ^ (y >> 1) ^ (0xB5026F5AA96619E9 if y & 1 else 0)
+            self.i = 0
+        y = x[self.i]
+        self.i += 1
+        y ^= (y >> 29) & 0x5555555555555555
+        y ^= (y << 17) & 0x71D67FFFEDA60000
+        y ^= (y << 37) & 0xFFF7EEE000000000
+        return y ^ (y >> 43)
+
+
+def _epoch(p, X, T, dims, batch, lr, seed):
+    """One epoch on the host: the seeded shuffle, mini-batches in order (the last
+    one short), the oracle's gradients, Adam from zero moments in FP64."""
+    from oracle import mlp_oracle as mo
+    n, rng = len(X), _MT64(seed)
+    perm = list(range(n))
+    for i in range(n - 1, 0, -1):
+        j = rng() % (i + 1)
+        perm[i], perm[j] = perm[j], perm[i]
+    p, m, v, total = p.astype(np.float64), 0.0, 0.0, 0.0
+    for t, r0 in enumerate(range(0, n, batch), 1):
+        rows = perm[r0:r0 + batch]
+        loss, g = mo.loss_and_grad(p, X[rows], T[rows], dims, bf=True)
+        total += loss * len(rows)
+        m, v = 0.9 * m + 0.1 * g, 0.999 * v + 0.001 * g * g
+        p = p - lr * (m / (1 - 0.9 ** t)) / (np.sqrt(v / (1 - 0.999 ** t)) + 1e-8)
+    return p, total / n
+
+
+LAYERED = [(133, 256, 66), (33, 64, 16), (7, 33, 3)]
+
+
+@pytest.mark.parametrize("dims,rows", [(LAYERED[0], 201), (LAYERED[1], 77), (LAYERED[2], 1), (LAYERED[2], 4097)])
+def test_layer_by_layer_form_matches_oracle(built, dims, rows):
+    """Shapes outside the fused kernels' (n_hidden 256, n_in <= 128, n_out <= 64):
+    forward, loss and gradients of the layer-by-layer form, at sizes that
+    leave remainders in its 64 x 64 x 32 tiles; tolerances as
+    test_forward_matches_oracle and test_gradients_match_oracle."""
+    from oracle import mlp_oracle as mo
+    capi = built
+    print(f"case: MLP {dims} layer by layer, {rows} rows", flush=True)
+    m = capi.MLP(*dims, seed=21)
+    rng = np.random.default_rng(rows)
+    p = m.params()
+    p += 0.1 * rng.standard_normal(p.size).astype(np.float32)  # non-zero biases
+    m.set_params(p)
+    X = rng.standard_normal((rows, dims[0])).astype(np.float32)
+    T = rng.standard_normal((rows, dims[2])).astype(np.float32)
+    Y = m.forward(X)
+    Yo, _ = mo.forward(p, X, dims, bf=True)
+    err = np.abs(Y - Yo).max() / np.abs(Yo).max()
+    print(f"forward: max rel diff {err:.2e}")
+    assert err < 1e-2
+    g, loss = m.gradients(X, T)
+    lo, go = mo.loss_and_grad(p, X, T, dims, bf=True)
+    assert abs(loss / lo - 1) < 1e-3
+    bg, bo = _blocks(g, dims), _blocks(go, dims)
+    for k in bg:
+        e = np.linalg.norm(bg[k] - bo[k]) / np.linalg.norm(bo[k])
+        print(f"  d{k}: relative L2 diff {e:.2e}")
+        assert e < 3e-2, k
+    m.close()
+
+
+@pytest.mark.parametrize("dims", [(33, 256, 16), (128, 256, 64)] + LAYERED)
+def test_training_epoch_matches_oracle(built, dims):
+    """An epoch of three mini-batches, the last one short (257 rows by 100), in
+    the fused and the layer-by-layer form, against the host's. The losses: 1e-3
+    as test_gradients_match_oracle. The parameters' change: with gradients that
+    differ by delta relative, Adam's normalised step turns round in about
+    delta / pi of the entries, 2 lr each, so sqrt(4 delta / pi) = 0.2 of the
+    change at the gradients' delta of 3e-2. Then, after steps large enough to
+    change every weight (lr 0.05 against weights of about 0.1), the gradients
+    at the new parameters: all copies of the weights have followed, those of
+    the backward products too."""
+    from oracle import mlp_oracle as mo
+    capi = built
+    mt = _MT64(5489)
+    for _ in range(9999):
+        mt()
+    assert mt() == 9981545732273789042  # the C++ standard's check value of this generator
+    rows, batch = 257, 100
+    print(f"case: MLP {dims} epoch of {rows} rows in batches of {batch}", flush=True)
+    rng = np.random.default_rng(dims[0])
+    X = rng.standard_normal((rows, dims[0])).astype(np.float32)
+    T = rng.standard_normal((rows, dims[2])).astype(np.float32)
+    for lr in (1e-3, 0.05):
+        m = capi.MLP(*dims, seed=23)
+        p0 = m.params()
+        m.set_data(X, T)
+        loss = m.train_epoch(batch, lr, 77)
+        p1 = m.params()
+        if lr == 1e-3:
+            ph, lh = _epoch(p0, X, T, dims, batch, lr, 77)
+            e = np.linalg.norm(p1 - ph) / np.linalg.norm(ph - p0)
+            print(f"loss {loss:.6e}, host {lh:.6e}; parameters' change: relative L2 diff {e:.2e}")
+            assert abs(loss / lh - 1) < 1e-3
+            assert e < 0.2
+        else:
+            assert np.linalg.norm(p1 - p0) > 0.2 * np.linalg.norm(p0)
+            g, l1 = m.gradients(X, T)
+            lo, go = mo.loss_and_grad(p1, X, T, dims, bf=True)
+            print(f"loss at the new parameters {l1:.6e}, oracle {lo:.6e}")
+            assert abs(l1 / lo - 1) < 1e-3
+            bg, bo = _blocks(g, dims), _blocks(go, dims)
+            for k in bg:
+                e = np.linalg.norm(bg[k] - bo[k]) / np.linalg.norm(bo[k])
+                print(f"  d{k}: relative L2 diff {e:.2e}")
+                assert e < 3e-2, k
+        m.close()
