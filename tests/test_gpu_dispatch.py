@@ -15,11 +15,11 @@ from common import HIP_D2H, HIP_H2D, STATE, earth_params, grid, hip_runtime
 pytestmark = pytest.mark.gpu
 
 
-def _run(capi, g, p, st, env, steps=2):
+def _run(capi, g, p, st, env, steps=2, variant=""):
     old = {k: os.environ.get(k) for k in env}
     os.environ.update(env)
     try:
-        d = capi.Dyn(g, p)  # the switches are read when the handle is created
+        d = capi.Dyn(g, p, variant=variant)  # the switches are read when the handle is created
     finally:
         for k, v in old.items():
             if v is None:
@@ -38,16 +38,20 @@ def _run(capi, g, p, st, env, steps=2):
 @pytest.mark.parametrize("precision", [0, 1])
 def test_shapes_by_size_equal_the_fixed_ones(built, glevel, nv, precision):
     capi = built
-    print(f"case: g{glevel} L{nv} precision {precision}: shapes by size vs 16-level chunks, 64 columns", flush=True)
+    print(f"case: g{glevel} L{nv} precision {precision}: chunks by size vs 16 levels, columns 16 vs 64", flush=True)
     g = grid(capi, glevel, nv)
     p = earth_params(capi, glevel, dt=600.0, ns=4, precision=precision)
     st = capi.ic_rest(g, p, seed=2040 + nv, temperature_noise=1e-3, wind_noise=1.0)
-    # (columns set in both: the FP64 vertical solve with one lane per column)
-    a = _run(capi, g, p, st, {"THOR_THOMAS_COLUMNS": "16"})
-    b = _run(capi, g, p, st, {"THOR_STENCIL_LEVELS": "16", "THOR_THOMAS_COLUMNS": "64"})
-    for k in STATE:
-        assert np.isfinite(a[k]).all(), k
-        assert np.array_equal(a[k], b[k]), k
+    # the default kernels, chunks by size or of 16 levels, in both builds; then the vertical
+    # solve with one lane per column (the columns are set in both), 16 or 64 of them per block
+    lane = {"THOR_THOMAS_SEG": "0", "THOR_THOMAS_ROWS": "0"} if precision else {}
+    for x, y, build in (({}, {"THOR_STENCIL_LEVELS": "16"}, ""), ({}, {"THOR_STENCIL_LEVELS": "16"}, "pm"),
+                        (dict(lane, THOR_THOMAS_COLUMNS="16"),
+                         dict(lane, THOR_STENCIL_LEVELS="16", THOR_THOMAS_COLUMNS="64"), "")):
+        a, b = _run(capi, g, p, st, x, variant=build), _run(capi, g, p, st, y, variant=build)
+        for k in STATE:
+            assert np.isfinite(a[k]).all(), (x, build, k)
+            assert np.array_equal(a[k], b[k]), (x, build, k)
 
 
 @pytest.mark.parametrize("nv,extra", [
@@ -87,8 +91,9 @@ def test_row_solve_equals_the_one_lane_solve(built, nv, extra, precision):
     scanned over the rows), the level constants from a table and one power per
     cell, and in FP64 the split flux divergence, against the one-lane solve
     (THOR_THOMAS_COLUMNS; mixed THOR_THOMAS_SEG 0), one step, with and without a
-    hook between solve and update; up to 65 levels (four interfaces per row),
-    above them both are the one-lane solve. Bound as above: the recurrences are
+    hook between solve and update; up to 65 levels (four interfaces per row);
+    above them the mixed form's sweeps run on all rows of k_thomas_dp and in FP64
+    both are the one-lane solve. Bound as above: the recurrences are
     the same numbers in another association, each power within the portable
     pow's 2.5 (1 + |y log x|) ulp; the mixed form rounds the momentum deviation
     that follows to FP32, so 1e-9 there."""
@@ -118,6 +123,7 @@ def test_row_solve_equals_the_one_lane_solve(built, nv, extra, precision):
 @pytest.mark.parametrize("precision,nv,extra", [
     (0, 20, {}), (1, 20, {}), (0, 3, {}), (1, 33, dict(DeepModel=0, NonHydro=0, GravHeightVar=1)),
     (0, 33, dict(DeepModel=0, NonHydro=0, GravHeightVar=1)), (1, 23, dict(DivDampP=0)), (0, 23, dict(HyDiff=0)),
+    (0, 21, dict(NonHydro=0)), (1, 21, dict(NonHydro=0, GravHeightVar=1)),
     (0, 21, dict(thermo_equation=1)), (0, 20, dict(VertHyDiff=1, VertHyDiffOrder=6, Diffc_v=2e-3)),
 ])
 def test_slow_modes_equal_the_reference_order(built, precision, nv, extra):

@@ -109,7 +109,8 @@ def test_chunked_slow_modes_equal_per_level_kernel(built, nv, extra):
     g = grid(capi, 4, nv)
     p = earth_params(capi, 4, dt=600.0, ns=6, **extra)
     st = capi.ic_rest(g, p, seed=1070 + nv, temperature_noise=1e-3, wind_noise=1.0)
-    a = _run_env(capi, g, p, st, 2, {"THOR_SLOW_CHUNKED": "1"})
+    # (chunks of 16 levels: by size a grid of this size takes one level per block)
+    a = _run_env(capi, g, p, st, 2, {"THOR_SLOW_CHUNKED": "1", "THOR_STENCIL_LEVELS": "16"})
     b = _run_env(capi, g, p, st, 2, {"THOR_SLOW_CHUNKED": "0"})
     for k in STATE:
         assert np.isfinite(a[k]).all()
@@ -133,7 +134,7 @@ def test_segment_vertical_solve_equals_fp64_kernel(built, nv, extra):
     p = earth_params(capi, 4, dt=600.0, ns=6, **extra)
     st = capi.ic_rest(g, p, seed=1080 + nv, temperature_noise=1e-3, wind_noise=1.0)
     a = _run_env(capi, g, p, st, 2, {"THOR_THOMAS_SEG64": "16"})
-    b = _run_env(capi, g, p, st, 2, {"THOR_THOMAS_SEG64": "0"})
+    b = _run_env(capi, g, p, st, 2, {"THOR_THOMAS_SEG64": "0", "THOR_THOMAS_COLUMNS": "64"})
     for k in STATE:
         assert np.isfinite(a[k]).all()
         assert np.array_equal(a[k], b[k]), k
@@ -158,10 +159,10 @@ def test_segment_vertical_solve_equals_fp64_kernel(built, nv, extra):
 
 
 @pytest.mark.parametrize("nv,extra,env", [
-    (20, dict(DeepModel=1, NonHydro=1), {"THOR_PREPARE_LC64": "1"}),
-    (23, dict(DeepModel=0, NonHydro=0, GravHeightVar=1), {"THOR_PREPARE_LC64": "1"}),
+    (20, dict(DeepModel=1, NonHydro=1), {"THOR_PREPARE_LC64": "1", "THOR_STENCIL_LEVELS": "16"}),
+    (23, dict(DeepModel=0, NonHydro=0, GravHeightVar=1), {"THOR_PREPARE_LC64": "1", "THOR_STENCIL_LEVELS": "16"}),
     (23, dict(DeepModel=1, NonHydro=1, thermo_equation=1), {"THOR_PREPARE_LC64": "1", "THOR_STENCIL_LEVELS": "5"}),
-    (23, dict(DeepModel=1, NonHydro=1), {"THOR_ML_LEVELS": "2"}),
+    (23, dict(DeepModel=1, NonHydro=1), {"THOR_ML_LEVELS": "2", "THOR_STENCIL_LEVELS": "16"}),
 ])
 def test_chunked_prepare_equals_multilevel_kernel(built, nv, extra, env):
     """FP64 implicit-solve sources and flux divergences over level chunks

@@ -238,10 +238,11 @@ def test_chunked_slow_modes_equal_per_level_kernel(built, deep, nonhydro, ghv):
     a = _two_steps(capi, g, p, st, {"THOR_SLOW_CHUNKED": "0"})
     # both chunked kernels: k_slow_lc and k_slow_lc2 (two blocks per CU)
     for v2 in ("0", "1"):
-        b = _two_steps(capi, g, p, st, {"THOR_PREPARE_SPLIT": "0", "THOR_SLOW_V2": v2})
+        # (chunks of 16 levels: by size a grid of this size takes one level per block)
+        b = _two_steps(capi, g, p, st, {"THOR_PREPARE_SPLIT": "0", "THOR_SLOW_V2": v2, "THOR_STENCIL_LEVELS": "16"})
         for k in a:
             assert np.array_equal(a[k], b[k]), (v2, k)
-    # Default: the substep pressure flux divergence adds the stage part
+    # Default (k_slow_w): the substep pressure flux divergence adds the stage part
     # (formed by the slow-mode kernel) to the deviation part, whose h and pt
     # factors are read as FP32 copies (they multiply the FP32 momentum
     # deviation); the same sums grouped differently with one more FP32
@@ -255,8 +256,9 @@ def test_chunked_slow_modes_equal_per_level_kernel(built, deep, nonhydro, ghv):
 
 
 def test_thomas_loop_unroll_is_bitwise_unchanged(built):
-    """The fused vertical-solve kernel with its level loops unrolled by two
-    (the default) gives the same states as without unrolling, in both
+    """The fused vertical-solve kernel of 64 columns per block (by switch on a
+    grid of this size; mixed: without the row solve) with its level loops
+    unrolled by two gives the same states as without unrolling, in both
     precision forms."""
     capi = built
     g = grid(capi, 4, 20)
@@ -264,8 +266,9 @@ def test_thomas_loop_unroll_is_bitwise_unchanged(built):
         p = earth_params(capi, 4, dt=600.0, precision=prec, HyDiff=1, DivDampP=1)
         print(f"case: precision {prec} g4 L20, Thomas level loops unrolled by 2 vs 1", flush=True)
         st = capi.ic_rest(g, p, seed=1012, temperature_noise=1.0, wind_noise=2.0)
-        a = _two_steps(capi, g, p, st, {"THOR_THOMAS_UNROLL": "1"})
-        b = _two_steps(capi, g, p, st, {"THOR_THOMAS_UNROLL": "2"})
+        cols = {"THOR_THOMAS_COLUMNS": "64", "THOR_THOMAS_SEG": "0"}
+        a = _two_steps(capi, g, p, st, {"THOR_THOMAS_UNROLL": "1", **cols})
+        b = _two_steps(capi, g, p, st, {"THOR_THOMAS_UNROLL": "2", **cols})
         for k in a:
             assert np.array_equal(a[k], b[k]), (prec, k)
 
@@ -281,7 +284,7 @@ def test_chunked_last_diffusion_pass_stays_close(built):
     print("case: mixed g4 L20, chunked vs per-level last diffusion pass + divergence-damping pass 0", flush=True)
     st = capi.ic_rest(g, p, seed=1013, temperature_noise=1.0, wind_noise=2.0)
     a = _two_steps(capi, g, p, st, {"THOR_DIFF2_CHUNKED": "0"})
-    b = _two_steps(capi, g, p, st, {})
+    b = _two_steps(capi, g, p, st, {"THOR_STENCIL_LEVELS": "16"})  # by size: one level per block here
     tol = {"Mh": 1e-5, "Wh": 1e-5, "W": 1e-5, "Rho": 1e-7, "pressure": 1e-7}
     for k in a:
         err = float(np.abs(b[k] - a[k]).max() / np.abs(a[k]).max())
@@ -311,8 +314,9 @@ def test_column_prep_level_window_is_bitwise_unchanged(built, deep, nonhydro, gh
 
 def test_row_parallel_vertical_sweeps_stay_close(built):
     """The mixed path's vertical solve with both sweeps on all rows of the
-    block (segment maps chained through LDS) against the one-lane sweeps:
-    two steps agree to FP64 rounding."""
+    block (segment maps chained through LDS, what k_thomas_dp runs above 65
+    levels; here by switch) against the one-lane sweeps: two steps agree to
+    FP64 rounding."""
     capi = built
     for nv in (20, 48):
         g = grid(capi, 4, nv)
@@ -320,7 +324,7 @@ def test_row_parallel_vertical_sweeps_stay_close(built):
         print(f"case: mixed g4 L{nv}, row-parallel vs one-lane vertical sweeps", flush=True)
         st = capi.ic_rest(g, p, seed=1017, temperature_noise=1.0, wind_noise=2.0)
         a = _two_steps(capi, g, p, st, {"THOR_THOMAS_ROWS": "0"})
-        b = _two_steps(capi, g, p, st, {})
+        b = _two_steps(capi, g, p, st, {"THOR_THOMAS_SEG": "0"})
         for k in a:
             err = float(np.abs(b[k] - a[k]).max() / np.abs(a[k]).max())
             print(f"  L{nv} {k}: max rel diff {err:.2e}")
@@ -329,10 +333,10 @@ def test_row_parallel_vertical_sweeps_stay_close(built):
 
 @pytest.mark.parametrize("nv,deep,nonhydro,ghv", [(20, 1, 1, 0), (33, 0, 0, 1), (48, 1, 1, 1), (64, 1, 0, 0)])
 def test_segment_vertical_solve_stays_close(built, nv, deep, nonhydro, ghv):
-    """The segment form of the mixed vertical solve (each row of the block
-    owns a contiguous run of interfaces in all three phases and keeps its
-    cells' values in registers for the density/pressure update), with 16 and
-    32 columns per block, and the segment form of the stage's factorisation
+    """The mixed vertical solve by segments (each row of the block owns a
+    contiguous run of interfaces in all three phases and keeps its cells'
+    values in registers for the density/pressure update), k_solve with 16
+    columns per block and k_thomas_dp_seg with 32, and the segment form of the stage's factorisation
     (Moebius maps of the pivot recurrence chained over the rows), against the
     one-lane sweeps and recurrence: two steps agree to FP64 rounding,
     including ragged last segments and rows without interfaces."""
