@@ -402,7 +402,7 @@ def test_training_epoch_matches_oracle(built, dims):
     differ by delta relative, Adam's normalised step turns round in about
     delta / pi of the entries, 2 lr each, so sqrt(4 delta / pi) = 0.2 of the
     change at the gradients' delta of 3e-2. Then, after steps large enough to
-    change every weight (lr 0.05 against weights of about 0.1), the gradients
+    change every weight (lr 0.05 against weights of 0.1 to 0.4), the gradients
     at the new parameters: all copies of the weights have followed, those of
     the backward products too."""
     from oracle import mlp_oracle as mo
@@ -431,7 +431,8 @@ def test_training_epoch_matches_oracle(built, dims):
         else:
             assert np.linalg.norm(p1 - p0) > 0.2 * np.linalg.norm(p0)
             g, l1 = m.gradients(X, T)
-            lo, go = mo.loss_and_grad(p1, X, T, dims, bf=True)
+            with np.errstate(over="ignore"):  # GELU of large negative inputs: 1 / (1 + inf)
+                lo, go = mo.loss_and_grad(p1, X, T, dims, bf=True)
             print(f"loss at the new parameters {l1:.6e}, oracle {lo:.6e}")
             assert abs(l1 / lo - 1) < 1e-3
             bg, bo = _blocks(g, dims), _blocks(go, dims)
