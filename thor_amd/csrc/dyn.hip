@@ -558,10 +558,10 @@ template <bool MX> static int thor_step_t(Dyn &d) {
             const dim3 gpz((d.P + kTile - 1) / kTile, nl);
             if (nl > 0 && (rk == 0 || sp.mode == 3)) {
                 const int nc = sp.ncomp();
-                launch(d, "sponge_zonal", 6 * B, [&] {
+                launch(d, "sponge_zonal", 6 * 8.0 * d.P * nl, [&] {
                     k_sponge_zonal<<<gpz, blk, 0, st>>>(g, fz, sp, d.ztab, d.ztmp);
                 });
-                launch(d, "sponge_mean", 8.0 * nc * sp.nlat * d.nv * sp.max_count, [&] {
+                launch(d, "sponge_mean", 8.0 * nc * sp.nlat * nl * sp.max_count, [&] {
                     k_sponge_reduce<<<nl * nc * sp.nlat, 1024, 0, st>>>(sp, d.nv, d.ztmp, d.zout);
                     k_sponge_vbar<<<(nc * sp.nlat * nl + 255) / 256, 256, 0, st>>>(sp, d.nv, d.zout, d.vbar);
                 });
@@ -759,12 +759,12 @@ static int profx(Dyn &d, int forcing) {
         const int nl = d.nv - sp.l0;  // levels with a zonal mean
         const dim3 gpz((d.P + kTile - 1) / kTile, nl);
         // Wh 2, Mh 3, rho in; W and the three zonal slots out
-        if (nl > 0) launch(d, "sponge_zonal", 10 * B, [&] {
+        if (nl > 0) launch(d, "sponge_zonal", 10 * 8.0 * d.P * nl, [&] {
             k_sponge_zonal<<<gpz, blk, 0, d.stream>>>(g, f, sp, d.ztab, d.ztmp);
         });
         if (nl > 0 && (sp.dmu || sp.dmw || sp.dmt)) {
             const int nc = sp.ncomp();
-            launch(d, "sponge_mean", 8.0 * nc * sp.nlat * d.nv * sp.max_count, [&] {
+            launch(d, "sponge_mean", 8.0 * nc * sp.nlat * nl * sp.max_count, [&] {
                 k_sponge_reduce<<<nl * nc * sp.nlat, 1024, 0, d.stream>>>(sp, d.nv, d.ztmp, d.zout);
                 k_sponge_vbar<<<(nc * sp.nlat * nl + 255) / 256, 256, 0, d.stream>>>(sp, d.nv, d.zout, d.vbar);
             });
