@@ -18,7 +18,10 @@ Prints ONE JSON line. Extra objects:
   roofline       - dominant kernel of the headline form: algorithmic bytes per
                    launch (per-cell arrays of the reference kernels it fuses,
                    each at its storage width, x P x nv) / average launch time
-                   from HIP events on the library's stream, against 8 TB/s;
+                   from HIP events on the library's stream, against 8 TB/s
+                   (a launch that moves fewer bytes than the kernels it
+                   replaces can book more than the peak: traffic_frac is the
+                   rate on the bytes it moved);
                    "traffic" = HBM bytes per launch from the committed
                    rocprofv3 FETCH_SIZE / WRITE_SIZE runs (profiles/hbm_traffic_*.json);
                    "step" = the whole large step's algorithmic bytes / wall time;

@@ -343,7 +343,11 @@ typedef struct thor_step_view {
  *   dyn_core_loop_end         after the new state is in place (:1465).
  * stream is the handle's hipStream_t (a module enqueues its kernels on it),
  * nstep the 1-based number of the Thor step this handle is taking, times the
- * RK stage's step (dt/3, dt/ns, dt/ns) as in the reference. A non-zero return
+ * RK stage's step (dt/3, dt/ns, dt/ns) as in the reference. What a callback
+ * sets through the library (thor_dyn_set_field: the state, the tendencies, the
+ * stage's temperature .. gtilh; thor_dyn_set_sponge) counts from the next
+ * kernel on that reads it; hh and gtilh enter the vertical solve of a stage up
+ * to its slow-mode callback. A non-zero return
  * stops the step with THOR_ERR_HOOK (the state is then partly updated). Any
  * callback may be NULL; hooks = NULL removes them. */
 typedef struct thor_hooks {

@@ -2409,8 +2409,8 @@ __global__ __launch_bounds__(256, THOR_DIVM0_LC_MINB) void k_divm0_lc(Geo g, Fie
 
 // Divergence-damping pass 1 of the slow part (the DivM term of
 // Compute_Slow_Modes, thor_slowmodes.h:82-105) in FP32 over level chunks, with
-// the operation order of divm_w<true>, written to dm [3][nv] for k_slow_lc and
-// k_slow_lc2.
+// the operation order of divm_w<true>, written to dm [3][nv] for k_slow_w,
+// k_slow_lc and k_slow_lc2.
 __global__ __launch_bounds__(256, 3) void k_divm1_lc(Geo g, Fields f, float *dm, int lc) {
     int r, l0, l1;
     if (!block_tile_lc(g, lc, r, l0, l1)) return;
@@ -3842,8 +3842,9 @@ __global__ __launch_bounds__(256) void k_thomas_dp(Geo g, Fields f, double delta
 // equals k_thomas_dp<.., false> bit for bit.
 // SEG: interfaces per row at most; the host launches it with
 // (nv - 1 + NROW - 1) / NROW <= SEG. DP = false: the vertical solve alone
-// (Whs written; k_dp applies the update after a physics hook). Up to 65 levels
-// both forms of the production build take k_solve instead.
+// (Whs written; k_dp applies the update after a physics hook). Taken by the
+// switches THOR_THOMAS_SEG = 32 (mixed) and THOR_THOMAS_SEG64 = 16 (FP64) only: the
+// default is k_solve up to 65 levels and k_thomas_dp above them.
 template <int CB, int SEG, bool DP = true, bool MX = true>
 __global__ __launch_bounds__(256) void k_thomas_dp_seg(Geo g, Fields f, double deltat) {
     constexpr int NROW = 256 / CB;

@@ -14,7 +14,7 @@
 //
 // Measured at 40 962 x 48 (us per launch, triangle walk -> here; the field
 // traffic at the 4.7 TB/s of a large copy in brackets): advection and first
-// Laplacian 243 -> 78 [60], last Laplacian 224 -> 60 [48], damping pass 0 100 ->
+// Laplacian 243 -> 78 [60], last Laplacian 224 -> 60 [43], damping pass 0 100 ->
 // 38 [24], pass 1 64 -> 30 [20], momentum 107 -> 49 [43]; the FP64 step
 // 7.70 -> 5.00 ms. At 2 562 x 23, one level per block: 27.6 -> 9.3, 22.4 -> 7.1,
 // 17.0 -> 9.5, 13.9 -> 7.2, 20.2 -> 10.2.
@@ -96,7 +96,8 @@ __global__ __launch_bounds__(256) void k_probe_weights64(Geo gu, double *wlap, d
 
 // Divergence-damping pass 0 (DivM_Op, thor_div.h:49-315) on the deviations Mhs /
 // Whs, or with STAGE on the stage values Mhk / Whk. Bound by its field traffic
-// (8 doubles per cell) and the 84 weights per point and chunk, read from L2.
+// (7 doubles per cell: M 3 and W in, 3 out) and the 84 weights per point and chunk,
+// read from L2.
 template <bool STAGE>
 __global__ __launch_bounds__(256, 2) void k_divm0_lw(Geo g, Fields f, int lc) {
 #pragma clang fp contract(fast)
@@ -297,7 +298,7 @@ __global__ __launch_bounds__(256, 2) void k_momentum_lw(Geo g, Fields f, int div
 }
 
 // Divergence-damping pass 1 of the slow part (thor_slowmodes.h:82-105) into dm
-// [3][nv], for k_slow_lc2<false>.
+// [3][nv], for k_slow_w<false>.
 __global__ __launch_bounds__(256, 3) void k_divm1_lw(Geo g, Fields f, double *dm, int lc) {
 #pragma clang fp contract(fast)
     int r, l0, l1;

@@ -103,8 +103,11 @@ __device__ __forceinline__ double dp_pressure(const DpConst &k, double ps, doubl
 // of its own. The form before it (k_thomas_dp_seg: about nine FP64 divisions,
 // 64-bit addresses per value, the update's loads behind the sweeps, a chain
 // over up to 15 rows in LDS) took 24 cycles of a CU per cell, VALU as much as
-// memory: 77 us at 40 962 x 48, 22.9 at 10 242 x 40 and 10.7 at 2 562 x 20 (65, 7.5
-// and 1 for its 156 bytes per cell); here 63.5, 15.8 and 7.8.
+// memory: 77 us at 40 962 x 48, 22.9 at 10 242 x 40 and 10.7 at 2 562 x 20 in the
+// mixed form; here 59, 16.1 and 7.9. Its floor there: 140 bytes per cell (14 FP64
+// planes and diffpr in, 3 out; Qheat, where it is not known to be zero, 8 more;
+// FP64 form 4 more), so 58 us at the 4.73 TB/s of a large copy, and 6.7 and 0.8 at
+// the 8.5 TB/s of one within the 256 MB cache.
 // SEG: interfaces per row, ceil((nv - 1) / 16). DP = false: the solve alone
 // (k_dp_solve then applies the update after a physics hook).
 template <int SEG, bool DP, bool MX>
