@@ -306,3 +306,45 @@ def test_sponge_from_any_level_bitwise(built, ns, mode, temp):
     d.close()
     for k in STATE:
         assert np.array_equal(a[k], b[k]), k
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("hooked", [False, True])
+def test_row_solve_takes_a_cell_without_pressure(built, precision, hooked):
+    """A cell whose pressure is exactly zero: the update of the row solve divides
+    by a power of it, the reference's does not; the new pressure is the
+    reference's all the same, P_Ref (-Rd flux dt / P_Ref)^(Cp/Cv). Against the FP64
+    one-lane solve in the reference's order, one short step; bounds as
+    test_row_solve_equals_the_one_lane_solve, mixed against the FP64 form 1e-4."""
+    capi = built
+    print(f"case: precision {precision} g4 L20: zero pressure in one cell, hook {hooked}", flush=True)
+    g = grid(capi, 4, 20)
+    st = capi.ic_rest(g, earth_params(capi, 4, dt=1.0, ns=6), seed=2740, temperature_noise=1e-3, wind_noise=1.0)
+    st["pressure"][1000, 7] = 0.0
+    p = earth_params(capi, 4, dt=1.0, ns=6, precision=precision)
+    d = capi.Dyn(g, p)
+    if hooked:
+        d.set_hooks(fast_modes=lambda stream, nstep, times, view: 0)
+    d.set_state(st)
+    d.run(1, capi.FORCING_NONE)
+    d.sync()
+    a = d.get_state()
+    d.close()
+    q = earth_params(capi, 4, dt=1.0, ns=6)
+    os.environ["THOR_THOMAS_COLUMNS"] = "16"
+    try:
+        d = capi.Dyn(g, q)
+    finally:
+        del os.environ["THOR_THOMAS_COLUMNS"]
+    d.set_state(st)
+    d.run(1, capi.FORCING_NONE)
+    d.sync()
+    b = d.get_state()
+    d.close()
+    cs = np.sqrt(p.Cp / (p.Cp - p.Rd) * p.Rd * p.Tmean)
+    for k in STATE:
+        assert np.isfinite(b[k]).all(), k
+        scale = np.abs(b["Rho"]).max() * cs if k in ("Mh", "Wh", "W") else np.abs(b[k]).max()
+        err = np.abs(a[k] - b[k]).max() / scale
+        print(f"  {k}: {err:.2e}")
+        assert err < (1e-4 if precision else 1e-12), k

@@ -76,7 +76,7 @@ struct DpConst {
 __device__ __forceinline__ double dp_pressure(const DpConst &k, double ps, double pk, double flux, double dpr, double q) {
     const double pf = ps + pk;
     const double x = -flux * k.RoP * pow_fma(pf * k.iP, -k.kap);
-    double g1;
+    double dp;
     if (fabs(x) < 0.0078125) {
         double c[10];
         c[1] = k.gam;
@@ -85,11 +85,14 @@ __device__ __forceinline__ double dp_pressure(const DpConst &k, double ps, doubl
         double h = c[9];
 #pragma unroll
         for (int i = 8; i >= 1; i--) h = __builtin_fma(h, x, c[i]);
-        g1 = h * x;
+        dp = pf * (h * x);
     } else {
-        g1 = pow_fma(1.0 + x, k.gam) - 1.0;
+        // a cell of no pressure (x is infinite or NaN): pnew = P_Ref (-Rd flux dt / P_Ref)^(Cp/Cv)
+        const bool none = pf == 0.0;
+        const double q1 = pow_fma(none ? -flux * k.RoP : 1.0 + x, k.gam);
+        dp = none ? q1 / k.iP : pf * (q1 - 1.0);
     }
-    return ps + pf * g1 + (dpr * k.dt + k.RoCdt * q);
+    return ps + dp + (dpr * k.dt + k.RoCdt * q);
 }
 
 // The forward elimination x_l = (-C_l - x_{l-1} AA_l) TT_l and the back
